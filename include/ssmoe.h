@@ -26,7 +26,7 @@ extern "C" {
 #define SSMOE_ERR_TOKEN 4     /* draft token outside [0, V) */
 #define SSMOE_ERR_NONFINITE 8 /* non-finite logits reached a p/q decision */
 #define SSMOE_ERR_TIMEOUT 16  /* a persistent launch's bounded wait (2^22 polls) for another workgroup ran out: its
-                               * workgroups were not all resident at once, e.g. because a kernel on another stream
+                               * workgroups were not all resident at once, e.g. because a graph replayed on another stream
                                * held CUs. The launch still finishes; its outputs are not valid. */
 
 /* Text of the last error on this host thread ("" if none). */
@@ -62,7 +62,8 @@ int ssmoe_record_layout(int H, int I, int64_t* off);
  * Writes h_buf fp32 [R, K, I], o_buf fp32 [R, K, H] (o = (Wd h) * w), out fp32 [R, H] (rank-order sum).
  * Constraints: H % 128 == 0, H <= 4096, I % 128 == 0, I <= 1024, 1 <= K <= 16.
  * Takes no workspace (as the reference's): the library's static scratch has one slot per stream for the first 8
- * streams that call it on a device, so calls on different streams may overlap; a ninth stream shares a slot. */
+ * streams that call it on a device; a ninth stream shares a slot. Calls on different streams may be issued at the
+ * same time: the device runs them one after the other (they wait for each other by an event). */
 int ssmoe_moe_decode(const void* x, int x_is_f32, const int32_t* expert_ids, const float* weights, int layer,
                      const int32_t* map, int64_t map_len, const int64_t* slot_ptr, int64_t n_slots, float* h_buf,
                      float* o_buf, float* out, int R, int H, int I, int K, int E, void* stream);

@@ -18,8 +18,8 @@ __device__ int ss_status_storage;
 // Scratch of ssmoe_moe_decode, which (like the reference's moe_decode) takes no workspace argument: h fragments,
 // h partial sums and the persistent kernel's counters for one block of <= 4 rows. Zero at load; every launch leaves
 // its counters zero. One slot per stream for the first kDecodeSlots streams that call it on a device (a host table
-// assigns them), so calls on different streams do not share a slot; calls on one stream run in order. A stream past
-// the first kDecodeSlots shares a slot with an earlier one.
+// assigns them); a stream past the first kDecodeSlots shares a slot with an earlier one. Calls run one after the
+// other on a device (PersistentOrder), so the slots only keep graph replays on different streams apart.
 constexpr size_t kDecodeScratch = 320 * 1024;
 constexpr int kDecodeSlots = 8;
 __device__ __align__(256) unsigned char ss_decode_scratch[kDecodeSlots][kDecodeScratch];
@@ -131,6 +131,58 @@ int noalloc_scratch_ptr(void** out, hipStream_t st) {
   return ok();
 }
 
+// Orders the persistent launches of a device across streams. Their workgroups wait for each other inside the kernel,
+// so every workgroup of a launch has to become resident; two such launches on two streams could each hold CUs that
+// the other's remaining workgroups need, and both would wait until their poll limits ran out. The first launch on
+// another stream than the last one therefore waits (an event, on the device) for what that stream holds; launches on
+// one stream order themselves and pay one compare. Held over the launches of one call, so that two host threads
+// cannot slip between each other's wait and launch. A launch recorded into a graph is not ordered: where and when it
+// runs is decided at the replay.
+class PersistentOrder {
+ public:
+  int begin(hipStream_t st) {
+    int dev = 0;
+    if (int rc = current_device(&dev)) return rc;
+    State& s = state(dev);
+    lock_ = std::unique_lock<std::mutex>(s.mu);
+    if (s.any && s.last == st) return SSMOE_OK;
+    if (capturing(st)) return SSMOE_OK;
+    if (s.any && !capturing(s.last)) {
+      if (!s.ev) {
+        const hipError_t e = hipEventCreateWithFlags(&s.ev, hipEventDisableTiming);
+        if (e != hipSuccess) return hip_check(e, "hipEventCreate(launch order)");
+      }
+      hipError_t e = hipEventRecord(s.ev, s.last);
+      if (e == hipSuccess) e = hipStreamWaitEvent(st, s.ev, 0);
+      if (e != hipSuccess) (void)hipGetLastError();  // the last stream no longer exists
+    }
+    s.any = true;
+    s.last = st;
+    return SSMOE_OK;
+  }
+
+ private:
+  struct State {
+    std::mutex mu;
+    bool any = false;
+    hipStream_t last = nullptr;
+    hipEvent_t ev = nullptr;
+  };
+  static State& state(int dev) {
+    static State states[kMaxDevices];
+    return states[dev];
+  }
+  static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) != hipSuccess) {
+      (void)hipGetLastError();
+      return true;
+    }
+    return c != hipStreamCaptureStatusNone;
+  }
+  std::unique_lock<std::mutex> lock_;
+};
+
 bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
 int check_moe_shape(int R, int H, int I, int K, int E) {
@@ -202,6 +254,8 @@ int ssmoe_moe_decode(const void* x, int x_is_f32, const int32_t* expert_ids, con
   if (int rc = status_ptr(&err)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (int rc = decode_scratch_ptr(st, &scratch)) return rc;
+  PersistentOrder order;
+  if (int rc = order.begin(st)) return rc;
   const size_t xsz = x_is_f32 ? 4 : 2;
   for (int r0 = 0; r0 < R; r0 += kBlock) {
     ss::VerifyArgs a{};
@@ -328,6 +382,8 @@ static int verify_layer_impl(const uint16_t* x, const uint16_t* router_w, const 
   int* err = nullptr;
   if (int rc = status_ptr(&err)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  PersistentOrder order;
+  if (int rc = order.begin(st)) return rc;
   for (int r0 = 0; r0 < T; r0 += kBlock) {
     ss::VerifyArgs a{};
     a.mode = 0;
@@ -517,6 +573,8 @@ int ssmoe_moe_verify_chain(const uint16_t* stream_in, float eps, const ssmoe_cha
   a.E = E;
   a.err = err;
   a.trace = g_trace;
+  PersistentOrder order;
+  if (int rc = order.begin(static_cast<hipStream_t>(stream))) return rc;
   return hip_check(ss::launch_chain(a, static_cast<hipStream_t>(stream)), "verify chain launch");
 }
 
@@ -568,6 +626,8 @@ int ssmoe_accept_greedy(const float* target, const int32_t* drafts, int D, int V
   a.V = V;
   a.out = out;
   a.work = static_cast<float*>(workspace);
+  PersistentOrder order;
+  if (int rc = order.begin(static_cast<hipStream_t>(stream))) return rc;
   return hip_check(ss::launch_accept_greedy(a, static_cast<hipStream_t>(stream)), "accept greedy launch");
 }
 
@@ -593,6 +653,8 @@ int ssmoe_accept_pq(const float* target, const float* draft, const int32_t* draf
   a.work = static_cast<float*>(workspace);
   a.err = err;
   a.trace = g_trace;
+  PersistentOrder order;
+  if (int rc = order.begin(static_cast<hipStream_t>(stream))) return rc;
   return hip_check(ss::launch_accept_pq(a, static_cast<hipStream_t>(stream)), "accept pq launch");
 }
 
@@ -892,6 +954,8 @@ int ssmoe_sample_rows(const float* logits, int R, int V, float temperature, cons
                 (long long)(ss::draw_work_floats(R, V) * 4));
   int* err = nullptr;
   if (int rc = status_ptr(&err)) return rc;
+  PersistentOrder order;
+  if (int rc = order.begin(static_cast<hipStream_t>(stream))) return rc;
   return hip_check(ss::launch_draw_rows(logits, R, V, temperature, uniforms, workspace, tokens, err,
                                         static_cast<hipStream_t>(stream)),
                    "sample rows launch");
@@ -978,6 +1042,8 @@ int ssmoe_lm_head_pq(const void* x, int x_f32, int D, int K, const int32_t* q, c
                 (long long)ss::lm_head_pq_workspace_bytes(D, N));
   int* err = nullptr;
   if (int rc = status_ptr(&err)) return rc;
+  PersistentOrder order;
+  if (int rc = order.begin(static_cast<hipStream_t>(stream))) return rc;
   return hip_check(ss::launch_lm_head_pq(x, x_f32 ? 1 : 0, D, K, q, s, b, N, draft, drafts, uniforms, temperature,
                                          workspace, logits, out, err, static_cast<hipStream_t>(stream)),
                    "lm_head p/q launch");
