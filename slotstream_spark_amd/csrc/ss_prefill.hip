@@ -11,9 +11,8 @@
 //    in fp32, so one rounding of q*s + b, fused or not, gives the same value).
 //  * down: out_rows[r, n] = (sum_k h[r, k] * bf16(q*s + b)[n, k]) * row_weight[r], fp32.
 //  * combine: out[t] = ((o[t,0] + o[t,1]) + ...) + o[t,K-1], sequential fp32.
-// Tiles are constants of the kernel (128 rows x 256 weight rows x 64 K), never functions of R.
+// Every output row is accumulated in one fixed K order, whatever the tile shape and the number of rows.
 #include <type_traits>
-#include <utility>
 
 #include "ss_common.hpp"
 #include "ss_launch.hpp"
@@ -202,42 +201,43 @@ hipError_t launch_moe_align(const AlignArgs& a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------- grouped GEMM
-// Block: 256 threads (4 waves) x 128 sorted rows (one expert) x 256 weight rows, K in steps of 64 (one
-// quantisation group). Each wave owns 64 weight rows (four 16-column MFMA B fragments) for all 128 rows of the
-// block, so every weight of the block is dequantized exactly once, by the wave that multiplies it, straight into
-// MFMA B registers. Gate/up: wave w owns gate rows n0 + 32 w .. + 31 (fragments 0, 1) and the same up rows
-// (fragments 2, 3), so silu(g) * u is formed in registers. Down: wave w owns rows n0 + 64 w .. + 63. Column n of
-// fragment j is the wave's weight row 4 n + j (gate/up: h column 2 n + (j & 1)), so a lane's fragments hold adjacent
-// outputs and the epilogues store 16-byte pieces.
-// K order inside a group: lane quad q (lane >> 4) holds packed words 2q, 2q + 1 of its weight row's group
-// (elements 16 q .. 16 q + 15); MFMA slice s (0, 1) uses word 2q + s, i.e. elements 16 q + 8 s .. + 7, and the A
-// fragment of slice s holds the same elements of each row. A dot product does not depend on which MFMA lanes its
-// K terms go to, only on the accumulation, which the MFMA unit fixes.
+// Block: 256 threads (4 waves) x 128 sorted rows (one expert) x `tpb` tiles of 64 NB weight rows, K in steps of 128 (two
+// quantisation groups). Each wave owns 16 NB weight rows of a tile (NB 16-column MFMA B fragments) for all rows of the
+// block, so every weight is dequantized exactly once, by the wave that multiplies it, straight into MFMA B registers.
+// Gate/up: the first NB / 2 fragments are gate rows, the others the same up rows, so silu(g) * u is formed in
+// registers. Column n of fragment j is the wave's weight row NB n + j (gate/up: h column (NB / 2) n + j % (NB / 2)), so
+// a lane's fragments hold adjacent outputs and the epilogues store whole pieces.
+// K order inside a step: lane quad q (lane >> 4) holds the 16 bytes of packed words 4q .. 4q + 3 of its weight row
+// (elements 32 q .. 32 q + 31, one group); MFMA slice s (0..3) uses word 4q + s, and the A fragment of slice s holds
+// the same elements of each row. The order is the same for every tile shape and every number of live rows, so a
+// row's bits depend on that row and its record only.
 // Memory paths:
-//  * A (activations for gate/up, h for down): global -> registers -> LDS (two LDS stages); each load instruction
-//    covers 8 whole 128-byte rows (8 lanes per row), and only the live rows are loaded. The register-staged path
-//    keeps every wait precise (a direct-to-LDS load in flight makes the compiler wait for it before any LDS read).
-//  * Scales and biases of the block's 256 weight rows for the whole K range: read once, coalesced, into LDS as
-//    (s, b) dword pairs.
-//  * Packed weights: 8 bytes per lane per K step straight into registers.
-//  * The loads of a step are issued PD steps ahead of its MFMAs (register slots; see gemm_loop).
-// 16-byte chunk c of A row m sits at chunk position a_pos(m, c) of the row's 128 bytes, so the 16 rows one MFMA
-// operand read touches (and each group of 8 of them) fall on distinct banks. Rows past the block's valid count
-// get no MFMAs beyond the last 32-row pair of fragments that holds a valid row.
+//  * A (activations for gate/up, h for down): direct global -> LDS loads of 16 bytes per lane (four whole 256-byte row
+//    pieces per instruction), double-buffered; only the live 16-row fragments are loaded. The two stages are separate
+//    LDS objects, so the compiler knows that a pending load into one does not touch reads of the other. 16-byte chunk
+//    c of row m sits at chunk position c ^ a_swz(m), the lane that loads a position reads the chunk that belongs
+//    there, and the 16 lanes one ds_read_b128 phase serves fall on distinct banks (1.6 M conflict cycles per gate/up
+//    launch at 8192 tokens; with c ^ (m & 15) 23 M).
+//  * Packed weights: 16 bytes per lane per step straight into registers, one stage ahead.
+//  * Scales and biases: 8 groups (4 steps) of the wave's own rows at a time, direct to LDS, loaded once the last
+//    step of the previous 8 groups has read its values.
+// A stage holds KS steps: KS rises as the live rows fall (the loads of one stage are in flight while the previous one
+// is computed, and a light stage has little to compute), at the same LDS bytes.
+// What bounds it (MI355X, 8192 tokens x top-10, H 2048 / I 512, gate/up): 372 us, 924 TFLOP/s; without the loads 330,
+// without the dequantisation 315, without either 256, MFMA alone 161: the dequantisation (19 VALU per 8 nibbles) and
+// the MFMAs of the two waves of a SIMD overlap only in part (ordering one slice's dequantisation between the MFMAs of
+// the slice before, with or without wave priorities, changes nothing). The down product writes 671 MB of out_rows: 280
+// us, 195 without the stores. The former kernel (64-wide K steps, activations through registers, a barrier per 64 K,
+// four fragments always) took 424 and 325 us, and the pair 245 us at 2048 tokens and 45 at 19 (now 232 and 39).
 constexpr int kBM = 128;
-constexpr int kBK = 64;
-constexpr int kAStage = kBM * kBK * 2;  // 16 KB
-constexpr int kGateUpTileN = 128;       // gate (and up) rows per block
-constexpr int kDownTileN = 256;         // down rows per block
-constexpr int kBN = 256;                // weight rows per block (both kernels)
-constexpr int kMaxGroups = 64;          // K / 64 <= 64 (H, I <= 4096)
-// Dynamic LDS of one block: the two A stages, then the (s, b) table of kBN rows x (G + 1) dwords (G = K / 64; the
-// extra dword per row staggers the banks). Two blocks per CU fit for G <= 60.
-static size_t gemm_lds_bytes(int G) { return 2 * (size_t)kAStage + (size_t)kBN * (G + 1) * 4; }
-constexpr size_t kGemmLdsMax = 2 * kAStage + (size_t)kBN * (kMaxGroups + 1) * 4;
+constexpr int kStepK = 128;          // K per step: two quantisation groups
+constexpr int kRowB = kStepK * 2;    // bytes of one activation row per step
+constexpr int kAStage = kBM * kRowB; // one LDS stage of activations: 32 KB
+constexpr int kSbG = 8;              // groups per (s, b) table chunk
 
 typedef __bf16 ss_bf16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t ss_u32x2 __attribute__((ext_vector_type(2)));
+typedef float ss_f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void ss_lds_void;
 
 // bf16 pair (lo, hi) rounded to nearest even by the hardware conversion.
 SS_DEV uint32_t cvt_pk_bf16(float lo, float hi) {
@@ -294,12 +294,11 @@ SS_DEV void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Block index -> (M block, N tile). The plan's M blocks are dealt round-robin to the XCDs (workgroup b runs on XCD
-// b % 8), in plan order, so every XCD gets an even share of the heavy and the light experts' blocks (the mix also
-// pairs MFMA-bound full blocks with VALU-bound partial ones on a CU); each XCD takes all N tiles of one M block in a
-// row (they share its activation rows in the XCD's L2). Measured on MI355X at BASELINE config 3, this beats both
-// contiguous per-XCD ranges of the plan (XCDs ending 140-180 us apart) and a full-blocks-first order (full blocks
-// sharing a CU slow each other down).
+// Block index -> (M block, group of N tiles). The plan's M blocks are dealt round-robin to the XCDs (workgroup b runs on
+// XCD b % 8), in plan order, so every XCD gets an even share of the heavy and the light experts' blocks; each XCD takes
+// all N tiles of one M block in a row (they share its activation rows in the XCD's L2). Measured on MI355X, contiguous
+// per-XCD ranges of the plan end 140-180 us apart at 2048 tokens, and groups of 2, 4 or 8 M blocks per XCD (for the
+// weights they share) change nothing.
 SS_DEV bool xcd_tile(int mb, int nt, int& pid_m, int& pid_n) {
   const int b = blockIdx.x, x = b & 7, s = b >> 3;
   const int sm = s / nt;
@@ -308,115 +307,226 @@ SS_DEV bool xcd_tile(int mb, int nt, int& pid_m, int& pid_n) {
   return pid_m < mb;
 }
 
-// 16-byte chunk c of A row m sits at chunk position a_pos(m, c) of the row's 128 bytes.
-SS_DEV int a_pos(int m, int c) { return c ^ (m & 7) ^ ((m >> 3) & 1); }
+// Chunk swizzle of activation row m (see above): ds_read_b128 serves lanes 0-3 and 12-15 of one quad with lanes 4-11 of
+// its neighbour, whose chunk numbers differ in bit 2, so rows 4-11 (mod 16) take the upper half of the positions.
+SS_DEV int a_swz(int m) { return (m & 3) | ((m >> 1) & 4) | (((m << 1) ^ m) & 8); }
 
-// Local index of weight row (fragment j, lane row n) of wave w: 64 w + 16 j + n; the (s, b) table row stride is
-// G + 1 dwords, so 16 consecutive rows at one group fall on distinct banks.
+constexpr int kZeroRow = (int)0x80000000u;  // a row whose activations are zero (it reads row 0; its h is stored as 0)
 
-// f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>), in order.
-template <typename F, int... I>
-SS_DEV void ss_static_for_seq(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-SS_DEV void ss_static_for(F&& f) {
-  ss_static_for_seq(f, std::make_integer_sequence<int, N>{});
-}
+struct GemmSmem {
+  int a_row[kBM];    // activation row of each position, or kZeroRow
+  int out_row[kBM];  // row of h / out_rows, -1 past the valid rows
+  float wt[kBM];
+};
 
-// The K loop for NF live 16-row fragments (fragments NF .. 7 are all padding and get no loads or MFMAs), with the
-// global loads of step k + PD issued at the end of step k into register slot k % PD: the packed weights are PD steps
-// ahead of their use, the A rows PD - 1 steps ahead of their LDS store (two LDS stages). Blocks with fewer live rows
-// hold fewer accumulators, so they afford a deeper register ring (their steps are shorter, so they need it more).
-// Thread t stages A rows t / 8 + 32 c (c < NF / 2), 16-byte chunk t % 8.
-template <int NF, int PD>
-SS_DEV void gemm_loop(uint8_t* lds, const uint32_t* sbt, int nsteps, int aoff0, int aoff1, ss_f32x4 (&acc)[8][4],
-                      const uint16_t* const (&asrc)[4], int arow0, int achunk, const uint8_t* wbase,
-                      const int64_t (&wc)[4], uint32_t lw, int sb_lane, int sb_stride) {
-  static_assert(PD % 2 == 0, "the LDS stage of step k is k & 1 = (k % PD) & 1");
-  constexpr int NA = NF / 2;
-  uint4 areg[PD][NA];
-  ss_u32x2 bw[PD][4];
-  // Loads of step k (the last step again past the end: never used) into register slot S.
-  auto load = [&](int k, auto slot_c) {
-    constexpr int S = decltype(slot_c)::value;
-    const int kk = k < nsteps ? k : nsteps - 1;
+// `ntile` N tiles from tile0 for the block's NF live 16-row fragments, KS K-steps per LDS stage.
+template <bool GU, int NB, int NF, int KS>
+SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8_t* a1, uint8_t* lss, uint8_t* lsb,
+                       const uint8_t* base, int tile0, int ntile) {
+  static_assert(NF * KS <= 8 && (KS == 1 || KS == 2 || KS == 4), "a stage holds kAStage bytes; its chunk is loaded whole");
+  constexpr int TN = 64 * NB, HB = NB / 2;  // weight rows per tile; gate (and up) fragments per wave
+  constexpr int NQ = NF > 4 ? 2 : NF;       // A fragments read ahead of their MFMAs
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, q = lane >> 4;
+  const int kdim = GU ? g.H : g.I;
+  const int nsteps = kdim / kStepK, G = kdim / 64;
+  const int nst = (nsteps + KS - 1) / KS;  // stages per tile
+  const int wrow_b = kdim / 2;             // bytes of a packed weight row
+  const uint32_t arow_b = kdim * 2;
+  // Activations: load instruction c of wave w covers rows 16 c + 4 w + q, position n of each.
+  const int ar = 4 * w + q;
+  const uint8_t* abase = reinterpret_cast<const uint8_t*>(g.a) + 16 * (n ^ a_swz(ar));
+  // Lane offset of fragment 0's 16 bytes from the tile's first row; fragment j adds a uniform offset.
+  const uint32_t lw = (uint32_t)((GU ? 8 * NB * w + HB * n : 16 * NB * w + NB * n) * wrow_b + 16 * q);
+  const int64_t tile_w = (int64_t)(GU ? TN / 2 : TN) * wrow_b, tile_s = (int64_t)(GU ? TN / 2 : TN) * G * 2;
+  // (s, b) table: lane (q, n) of wave w fills slot 64 w + lane with its wave's row of fragment q (lanes past NB repeat
+  // the last fragment's), so a fragment's 16 rows are adjacent slots.
+  const int jq = q < NB ? q : NB - 1;
+  const bool s_up = GU && jq >= HB;
+  const int srow = GU ? 8 * NB * w + HB * n + (jq & (HB - 1)) : 16 * NB * w + NB * n + jq;
+  const uint8_t* sptr = base + (s_up ? g.s2_off : g.s_off) + (int64_t)srow * G * 2;
+  const uint32_t sb_dist = (uint32_t)(g.b_off - g.s_off);  // from a row's scales to its biases
+  // Rows of a multiple of 8 groups are 16-byte aligned: a slot is 16 bytes (8 groups). Otherwise (an odd number of
+  // steps) pairs of groups load as dwords: pair p of a slot at 256 p + 4 slot.
+  const bool wide = G % 8 == 0;
+
+  uint4 bw[2][KS][NB];
+  auto load = [&](int tile, int st, auto p_c) {
+    constexpr int P = decltype(p_c)::value;
+    uint8_t* ad = P ? a1 : a0;
 #pragma unroll
-    for (int c = 0; c < NA; ++c) areg[S][c] = ldg16(asrc[c] + (size_t)kk * kBK);
+    for (int u = 0; u < KS; ++u) {
+      const int k = st * KS + u;
+      if (KS == 1 || k < nsteps) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bw[S][j] = *(const SS_G ss_u32x2*)(wbase + wc[j] + lw + 32 * kk);
-  };
-  auto store_a = [&](auto slot_c, int stage) {
-    constexpr int S = decltype(slot_c)::value;
+        for (int c = 0; c < NF; ++c) {
+          const uint32_t row = (uint32_t)sm.a_row[16 * c + ar] & 0x7FFFFFFFu;
+          __builtin_amdgcn_global_load_lds(abase + k * kRowB + (uint64_t)row * arow_b,
+                                           (ss_lds_void*)(ad + (u * NF * 16 + 16 * c + 4 * w) * kRowB), 16, 0, 0);
+        }
+        uint32_t lv = lw;
+        asm volatile("" : "+v"(lv));  // the addresses are formed here, not kept in registers over the loop
+        const uint8_t* wt = base + tile * tile_w + 64 * k;
 #pragma unroll
-    for (int c = 0; c < NA; ++c) {
-      const int m = arow0 + 32 * c;
-      *reinterpret_cast<uint4*>(lds + stage * kAStage + m * (kBK * 2) + 16 * a_pos(m, achunk)) = areg[S][c];
-    }
-  };
-  ss_static_for<PD>([&](auto p) { load(decltype(p)::value, p); });
-  store_a(std::integral_constant<int, 0>{}, 0);
-  lds_barrier();
-  // One K step from register slot S (= k % PD) and LDS stage S & 1; then A of step k + 1 into the other stage, the
-  // loads of step k + PD into slot S, and the barrier.
-  auto step = [&](int k, auto slot_c) {
-    constexpr int S = decltype(slot_c)::value;
-    const uint8_t* st = lds + (S & 1) * kAStage;
-    float sc[4], bi[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t sb = sbt[sb_lane + j * sb_stride + k];
-      sc[j] = __uint_as_float(sb << 16) * 512.f;  // s * 2^9, exact
-      bi[j] = __uint_as_float(sb & 0xFFFF0000u);
-    }
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      ss_u32x4 bf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bf[j] = dequant8(s ? bw[S][j].y : bw[S][j].x, sc[j], bi[j]);
-      const uint8_t* ap = st + (s ? aoff1 : aoff0);
-      // A fragments in batches of up to four: one LDS wait per batch. The scheduling barriers keep one slice's
-      // operands live at a time (the register budget of two waves per SIMD); the two waves of a SIMD overlap one
-      // wave's dequantization with the other's MFMAs.
-#pragma unroll
-      for (int i0 = 0; i0 < NF; i0 += 4) {
-        constexpr int NB = NF < 4 ? NF : 4;
-        ss_u32x4 av[NB];
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-          if (i0 + i < NF) av[i] = *reinterpret_cast<const ss_u32x4*>(ap + (i0 + i) * 16 * (kBK * 2));
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-          if (i0 + i < NF)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i0 + i][j] = ss_mfma(av[i], bf[j], acc[i0 + i][j]);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < NB; ++j)
+          bw[P][u][j] = ldg16(wt + (GU && j >= HB ? g.w2_off : g.w_off) + (int64_t)(GU ? j & (HB - 1) : j) * wrow_b + lv);
       }
     }
-    store_a(std::integral_constant<int, (S + 1) % PD>{}, (S & 1) ^ 1);
-    load(k + PD, slot_c);
-    lds_barrier();
   };
-  // Whole groups of PD steps with no guard inside, so that every path into the loop head has the same loads in
-  // flight (a guarded step gave the head a second path without the last slot's loads, and the compiler then waited
-  // for every load at the head: the next steps' prefetches included); the nsteps % PD last steps after it.
-  const int nfull = nsteps - nsteps % PD;
+  // groups g0 .. g0 + 7 of the tile's rows into this wave's slots
+  auto load_sb = [&](int tile, int g0) {
+    const uint8_t* p = sptr + tile * tile_s + 2 * g0;
+    if (wide) {
+      __builtin_amdgcn_global_load_lds(p, (ss_lds_void*)(lss + 1024 * w), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(p + sb_dist, (ss_lds_void*)(lsb + 1024 * w), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int d = 0; d < kSbG / 2; ++d)
+        if (g0 + 2 * d < G) {
+          __builtin_amdgcn_global_load_lds(p + 4 * d, (ss_lds_void*)(lss + 1024 * w + 256 * d), 4, 0, 0);
+          __builtin_amdgcn_global_load_lds(p + sb_dist + 4 * d, (ss_lds_void*)(lsb + 1024 * w + 256 * d), 4, 0, 0);
+        }
+    }
+  };
+  const int sb_lane = 1024 * w + (wide ? 16 : 4) * n + 2 * (q >> 1);
+  const int sb_j = wide ? 256 : 64, sb_k = wide ? 4 : 256;
+
+  ss_f32x4 acc[NF][NB];
+  auto zero = [&]() {
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  // Stage st from LDS stage / register set P. When the stage is the last to read the table chunk (`chunk`), its
+  // (s, b) values are all in registers before the next chunk (tile ct, group cg) is requested into the same slots.
+  auto compute = [&](int st, auto p_c, bool chunk, int ct, int cg) {
+    constexpr int P = decltype(p_c)::value;
+    const uint8_t* as = (P ? a1 : a0) + n * kRowB;
+    int apos = 16 * ((4 * q) ^ a_swz(n));
+    asm volatile("" : "+v"(apos));
+    float sc[KS][NB], bi[KS][NB];
+#pragma unroll
+    for (int u = 0; u < KS; ++u)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int at = sb_lane + j * sb_j + ((st * KS + u) & (kSbG / 2 - 1)) * sb_k;
+        sc[u][j] = __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t*>(lss + at) << 16) * 512.f;  // s * 2^9
+        bi[u][j] = __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t*>(lsb + at) << 16);
+      }
+    if (chunk) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      load_sb(ct, cg);
+    }
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      if (u > 0 && st * KS + u >= nsteps) break;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        ss_u32x4 bf[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const uint4 v = bw[P][u][j];
+          bf[j] = dequant8(s == 0 ? v.x : s == 1 ? v.y : s == 2 ? v.z : v.w, sc[u][j], bi[u][j]);
+        }
+        // A fragments a few at a time: the scheduling barriers keep their registers few; the two waves of a SIMD
+        // overlap one wave's dequantisation and LDS reads with the other's MFMAs.
+        const uint8_t* ap = as + u * NF * 16 * kRowB + (apos ^ (16 * s));
+#pragma unroll
+        for (int i0 = 0; i0 < NF; i0 += NQ) {
+          ss_u32x4 av[NQ];
+#pragma unroll
+          for (int i = 0; i < NQ; ++i) av[i] = *reinterpret_cast<const ss_u32x4*>(ap + (i0 + i) * 16 * kRowB);
+#pragma unroll
+          for (int i = 0; i < NQ; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i0 + i][j] = ss_mfma(av[i], bf[j], acc[i0 + i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+  auto epilogue = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = 16 * i + 4 * q + r;
+        const int orow = sm.out_row[m];
+        if (orow < 0) continue;
+        if (GU) {
+          const bool live = sm.a_row[m] >= 0;
+          uint32_t hp = 0;
+#pragma unroll
+          for (int j = 0; j < HB; ++j) {
+            const float gv = acc[i][j][r], uv = acc[i][j + HB][r];
+            // silu with the hardware exp2 and reciprocal (about 1 ulp each): h is rounded to bf16 next, which
+            // hides fp32 differences of a few ulp except at a rounding tie.
+            const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gv * -1.4426950408889634f));
+            const float hv = live ? gv * sig * uv : 0.f;
+            hp |= (uint32_t)ss_f32_to_bf16(hv) << (16 * j);
+          }
+          uint16_t* hd = g.h + (int64_t)orow * g.I + tile * (TN / 2) + 8 * NB * w + HB * n;
+          if constexpr (NB == 4) *(SS_G uint32_t*)hd = hp;
+          else *(SS_G uint16_t*)hd = (uint16_t)hp;
+        } else {
+          const float wt = sm.wt[m];
+          float* od = g.out_rows + (int64_t)orow * g.H + tile * TN + 16 * NB * w + NB * n;
+          if constexpr (NB == 4)
+            stg16(od, make_uint4(__float_as_uint(acc[i][0][r] * wt), __float_as_uint(acc[i][1][r] * wt),
+                                 __float_as_uint(acc[i][2][r] * wt), __float_as_uint(acc[i][3][r] * wt)));
+          else
+            *(SS_G ss_f32x2*)od = ss_f32x2{acc[i][0][r] * wt, acc[i][1][r] * wt};
+        }
+      }
+  };
+
+  zero();
+  int tile = tile0, st = 0;
+  const int nall = ntile * nst;
+  constexpr int SPC = kSbG / 2 / KS;  // stages per table chunk
+  load_sb(tile, 0);
+  load(tile, 0, std::integral_constant<int, 0>{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  lds_barrier();
+  // Stage f of all tiles: the next stage's loads, this stage's MFMAs, the tile's epilogue behind its last stage, then
+  // the wait for the loads (every wave's, by the barrier).
+  auto stage = [&](int f, auto p_c) {
+    constexpr int P = decltype(p_c)::value;
+    int t2 = tile, s2 = st + 1;
+    if (s2 == nst) {
+      s2 = 0;
+      ++t2;
+    }
+    const bool more = f + 1 < nall;
+    if (more) load(t2, s2, std::integral_constant<int, P ^ 1>{});
+    __builtin_amdgcn_sched_barrier(0);
+    compute(st, p_c, more && s2 % SPC == 0, t2, s2 * KS * 2);
+    if (st == nst - 1) {
+      epilogue(tile);
+      zero();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    tile = t2;
+    st = s2;
+  };
 #pragma unroll 1
-  for (int k = 0; k < nfull; k += PD) ss_static_for<PD>([&](auto u) { step(k + decltype(u)::value, u); });
-  if (nfull < nsteps)
-    ss_static_for<PD>([&](auto u) {
-      if (nfull + decltype(u)::value < nsteps) step(nfull + decltype(u)::value, u);
-    });
+  for (int f = 0; f < nall; f += 2) {
+    stage(f, std::integral_constant<int, 0>{});
+    if (f + 1 < nall) stage(f + 1, std::integral_constant<int, 1>{});
+  }
 }
 
-template <bool GATE_UP>
-__global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmArgs g, int nt) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  __shared__ int64_t a_off[kBM];  // element offset of each row's A operand, -1 for a zero row
-  __shared__ int out_row[kBM];
-  __shared__ float wt_s[kBM];
-  uint32_t* sbt = reinterpret_cast<uint32_t*>(lds + 2 * kAStage);  // [kBN][G + 1] (s | b << 16)
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+template <bool GU, int NB>
+__global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmArgs g, int nt, int tpb) {
+  __shared__ __attribute__((aligned(256))) uint8_t a0[kAStage];
+  __shared__ __attribute__((aligned(256))) uint8_t a1[kAStage];
+  __shared__ __attribute__((aligned(256))) uint8_t lss[4096];
+  __shared__ __attribute__((aligned(256))) uint8_t lsb[4096];
+  __shared__ GemmSmem sm;
+  const int tid = threadIdx.x;
   const int mb = g.num_padded[0] / kBM;
   int pid_m, pid_n;
   if (!xcd_tile(mb, nt, pid_m, pid_n)) return;
@@ -424,172 +534,37 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmArgs g, int nt
   if (e < 0) return;
   const uint64_t t_start = g.trace ? __builtin_amdgcn_s_memrealtime() : 0;
   const uint8_t* base = reinterpret_cast<const uint8_t*>(g.group_ptr[e]);
-  const int kdim = GATE_UP ? g.H : g.I;
-  const int G = kdim / 64, sb_stride = G + 1;
   bool valid = false;
   if (tid < kBM) {
     const int r = g.sorted_rows[(int64_t)pid_m * kBM + tid];
     valid = r < g.R;
-    int64_t off = -1;  // -1: a zero row (a token outside [0, T))
+    int row = kZeroRow;
     if (valid) {
-      if (GATE_UP) {
+      if (GU) {
         const int t = g.row_token[r];
-        if (t >= 0 && t < g.T) off = (int64_t)t * g.H;
+        if (t >= 0 && t < g.T) row = t;
       } else {
-        off = (int64_t)r * g.I;
+        row = r;
       }
     }
-    a_off[tid] = off;
-    out_row[tid] = valid ? r : -1;
-    if (!GATE_UP) wt_s[tid] = valid ? g.row_weight[r] : 0.f;
-  }
-  // Column n of B fragment j of wave w is local weight row lr = 64 w + 4 n + j, so a lane's four fragments hold four
-  // adjacent outputs. Global weight row of local row lr and its piece: gate/up local rows map to gate rows (j < 2)
-  // or up rows (j >= 2) n0 + 32 w + 2 n + (j & 1), so g and u of one h column sit in one lane (fragments j and
-  // j + 2) and its two h columns are adjacent; down local rows are rows n0 + lr.
-  auto grow = [&](int lr, bool& up) -> int64_t {
-    if (GATE_UP) {
-      const int ww = lr >> 6, nn = (lr >> 2) & 15, j = lr & 3;
-      up = j >= 2;
-      return (int64_t)pid_n * kGateUpTileN + 32 * ww + 2 * nn + (j & 1);
-    }
-    up = false;
-    return (int64_t)pid_n * kDownTileN + lr;
-  };
-  // (s, b) table: thread t fills local rows t (one row, all G groups; 16-byte loads of 8 groups).
-  {
-    bool up;
-    const int64_t row = grow(tid, up);
-    const uint8_t* srow = base + (up ? g.s2_off : g.s_off) + row * G * 2;
-    const uint8_t* brow = base + (up ? g.b2_off : g.b_off) + row * G * 2;
-    uint32_t* dst = sbt + tid * sb_stride;
-    if (G % 8 == 0) {
-      for (int c = 0; c < G; c += 8) {
-        const uint4 sv = ldg16(srow + 2 * c), bv = ldg16(brow + 2 * c);
-        const uint32_t s4[4] = {sv.x, sv.y, sv.z, sv.w}, b4[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          dst[c + 2 * d] = (s4[d] & 0xFFFFu) | (b4[d] << 16);
-          dst[c + 2 * d + 1] = (s4[d] >> 16) | (b4[d] & 0xFFFF0000u);
-        }
-      }
-    } else {  // G is even (K is a multiple of 128): two groups per dword
-      for (int c = 0; c < G; c += 2) {
-        const uint32_t sv = *(const SS_G uint32_t*)(srow + 2 * c), bv = *(const SS_G uint32_t*)(brow + 2 * c);
-        dst[c] = (sv & 0xFFFFu) | (bv << 16);
-        dst[c + 1] = (sv >> 16) | (bv & 0xFFFF0000u);
-      }
-    }
+    sm.a_row[tid] = row;
+    sm.out_row[tid] = valid ? r : -1;
+    if (!GU) sm.wt[tid] = valid ? g.row_weight[r] : 0.f;
   }
   // Valid rows are a prefix of the block (each expert's rows come first in its padded range).
   const int nvalid = __syncthreads_count(valid);
-
-  // A staging: load instruction c of thread t covers row arow0 + 32 c (arow0 = t / 8), 16-byte chunk t % 8 (each
-  // instruction of a wave covers 8 whole 128-byte rows). A padding row or a zero row reads the first kdim elements
-  // of the expert record (always present): a padding row's MFMA output row is never stored, and a zero row's h is
-  // stored as 0 (silu(0) * 0).
-  const int arow0 = tid >> 3, achunk = tid & 7;
-  const uint16_t* asrc[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int m = arow0 + 32 * c;
-    const int64_t off = a_off[m];
-    asrc[c] = (m < nvalid && off >= 0 ? g.a + off : reinterpret_cast<const uint16_t*>(base)) + 8 * achunk;
-  }
-  // B: lane (n = lane & 15, q = lane >> 4) of fragment j reads words 2q, 2q + 1 of its row's group.
-  const int n = lane & 15, q = lane >> 4;
-  const int64_t wrow_b = kdim / 2;
-  int64_t wc[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    bool up;
-    const int64_t row0 = grow(64 * w + j, up);
-    wc[j] = (up ? g.w2_off : g.w_off) + row0 * wrow_b;
-  }
-  // lane row n is weight row row0 + 2 n (gate/up) or row0 + 4 n (down) of its fragment
-  const uint32_t lw = (uint32_t)((GATE_UP ? 2 : 4) * n * wrow_b + 8 * q);
-  const int sb_lane = (64 * w + 4 * n) * sb_stride;
-
-  ss_f32x4 acc[8][4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // Lane offsets of the A fragments (slice s): row 16 i + n, chunk 2q + s (a_pos depends on n only).
-  const int aoff0 = n * (kBK * 2) + 16 * a_pos(n, 2 * q);
-  const int aoff1 = n * (kBK * 2) + 16 * a_pos(n, 2 * q + 1);
-  const int nsteps = kdim / kBK;  // even: kdim is a multiple of 128
-  const int nf2 = (nvalid + 31) >> 5;  // live fragment pairs (1..4)
-  if (nf2 >= 4)
-    gemm_loop<8, 2>(lds, sbt, nsteps, aoff0, aoff1, acc, asrc, arow0, achunk, base, wc, lw, sb_lane, sb_stride);
-  else if (nf2 == 3)
-    gemm_loop<6, 2>(lds, sbt, nsteps, aoff0, aoff1, acc, asrc, arow0, achunk, base, wc, lw, sb_lane, sb_stride);
-  else if (nf2 == 2)
-    gemm_loop<4, 4>(lds, sbt, nsteps, aoff0, aoff1, acc, asrc, arow0, achunk, base, wc, lw, sb_lane, sb_stride);
-  else
-    gemm_loop<2, 4>(lds, sbt, nsteps, aoff0, aoff1, acc, asrc, arow0, achunk, base, wc, lw, sb_lane, sb_stride);
-
-  if (GATE_UP) {
-    // h = bf16(silu(g) * u) of the live fragments into an LDS tile [128 rows][128 columns] (a lane's two adjacent
-    // columns as one dword), then 16-byte row-contiguous stores of the valid rows.
-    uint32_t* ht = reinterpret_cast<uint32_t*>(lds);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i >= 2 * nf2) break;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 16 * i + 4 * q + r;
-        const bool live = a_off[m] >= 0;
-        uint32_t hp = 0;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const float gv = acc[i][j][r], uv = acc[i][j + 2][r];
-          // silu with the hardware exp2 and reciprocal (about 1 ulp each): h is rounded to bf16 next, which
-          // hides fp32 differences of a few ulp except at a rounding tie.
-          const float sig = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gv * -1.4426950408889634f));
-          const float hv = live ? gv * sig * uv : 0.f;
-          hp |= (uint32_t)ss_f32_to_bf16(hv) << (16 * j);
-        }
-        ht[m * (kGateUpTileN / 2) + 16 * w + n] = hp;
-      }
-    }
-    lds_barrier();
-    const int n0 = pid_n * kGateUpTileN;
-#pragma unroll
-    for (int u = 0; u < (kBM * kGateUpTileN * 2) / (16 * 256); ++u) {
-      const int id = u * 256 + tid;
-      const int m = id >> 4, cc = id & 15;
-      if (m >= nvalid) break;
-      const int r = out_row[m];
-      if (r >= 0) {
-        const uint4 v = *reinterpret_cast<const uint4*>(ht + m * (kGateUpTileN / 2) + 4 * cc);
-        stg16(g.h + (int64_t)r * g.I + n0 + 8 * cc, v);
-      }
-    }
-  } else {
-    // A lane's four fragments are four adjacent outputs: one 16-byte store per row.
-    const int n0 = pid_n * kDownTileN + 64 * w + 4 * n;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (i >= 2 * nf2) break;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = 16 * i + 4 * q + r;
-        const int orow = out_row[m];
-        if (orow >= 0) {
-          const float wt = wt_s[m];
-          const uint4 v = make_uint4(__float_as_uint(acc[i][0][r] * wt), __float_as_uint(acc[i][1][r] * wt),
-                                     __float_as_uint(acc[i][2][r] * wt), __float_as_uint(acc[i][3][r] * wt));
-          stg16(g.out_rows + (int64_t)orow * g.H + n0, v);
-        }
-      }
-    }
-  }
+  const int nf = (nvalid + 15) >> 4;  // live fragments (1..8)
+  const int tile0 = pid_n * tpb;
+  constexpr int KL = NB == 4 ? 2 : 4;  // with four fragments, four steps of weights do not fit the registers
+  if (nf > 6) gemm_tiles<GU, NB, 8, 1>(g, sm, a0, a1, lss, lsb, base, tile0, tpb);
+  else if (nf > 4) gemm_tiles<GU, NB, 6, 1>(g, sm, a0, a1, lss, lsb, base, tile0, tpb);
+  else if (nf > 2) gemm_tiles<GU, NB, 4, 2>(g, sm, a0, a1, lss, lsb, base, tile0, tpb);
+  else if (nf > 1) gemm_tiles<GU, NB, 2, KL>(g, sm, a0, a1, lss, lsb, base, tile0, tpb);
+  else gemm_tiles<GU, NB, 1, KL>(g, sm, a0, a1, lss, lsb, base, tile0, tpb);
   // Diagnostics: gate/up blocks at entries [0, 8192), down blocks at [8192, 16384), four per block.
   if (g.trace && tid == 0) {
-    const size_t at = (GATE_UP ? 0 : 8192) + 4 * (size_t)blockIdx.x;
-    if (at + 4 <= (GATE_UP ? 8192u : 16384u)) {
+    const size_t at = (GU ? 0 : 8192) + 4 * (size_t)blockIdx.x;
+    if (at + 4 <= (GU ? 8192u : 16384u)) {
       const uint32_t hw = __builtin_amdgcn_s_getreg(4 | (31 << 11));   // HW_ID
       const uint32_t xcc = __builtin_amdgcn_s_getreg(20 | (31 << 11)); // XCC_ID
       g.trace[at] = t_start;
@@ -600,11 +575,19 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmArgs g, int nt
   }
 }
 
+template <bool GU>
+static void launch_gemm(const GemmArgs& g, int nb, int tpb, int64_t mb, hipStream_t st) {
+  const int rows = GU ? g.I : g.H, tn = GU ? 32 * nb : 64 * nb;
+  const int nt = rows / tn / tpb;
+  const dim3 grid((unsigned)(8 * nt * ((mb + 7) / 8)));
+  if (nb == 4) hipLaunchKernelGGL((prefill_gemm_kernel<GU, 4>), grid, dim3(256), 0, st, g, nt, tpb);
+  else hipLaunchKernelGGL((prefill_gemm_kernel<GU, 2>), grid, dim3(256), 0, st, g, nt, tpb);
+}
+
 hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
   static_assert(kBM == kPrefillBlockM, "one block size for the plan and the GEMM");
   const SsRecord rec = ss_record_layout(p.H, p.I);
-  const int64_t P = padded_rows(p.R, p.num_local, kBM);
-  if (P == 0 || p.R == 0) return hipSuccess;
+  if (p.R == 0) return hipSuccess;
   GemmArgs g{};
   g.row_token = p.row_token;
   g.row_weight = p.row_weight;
@@ -619,31 +602,33 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
   g.H = p.H;
   g.I = p.I;
   g.trace = p.trace;
-  g.a = p.x;
+  // With no token at all every row is a zero row, whose (unused) activations still come from a readable row.
+  g.a = p.T > 0 ? p.x : reinterpret_cast<const uint16_t*>(p.out_rows);
   g.w_off = rec.gw;
   g.s_off = rec.gs;
   g.b_off = rec.gb;
   g.w2_off = rec.uw;
   g.s2_off = rec.us;
   g.b2_off = rec.ub;
-  // Grids cover the plan's upper bound of M blocks (rounded up to a multiple of 8) times the N tiles; blocks past
-  // the device-side count exit at once.
-  KernelCfg cfg;
-  hipError_t e = kernel_cfg(reinterpret_cast<const void*>(prefill_gemm_kernel<true>), 256, kGemmLdsMax, &cfg);
-  if (e == hipSuccess)
-    e = kernel_cfg(reinterpret_cast<const void*>(prefill_gemm_kernel<false>), 256, kGemmLdsMax, &cfg);
-  if (e != hipSuccess) return e;
-  const int64_t mb = P / kBM;
-  const int nt_gu = p.I / kGateUpTileN, nt_d = p.H / kDownTileN;
-  auto grid_of = [&](int nt) { return (unsigned)(8 * nt * ((mb + 7) / 8)); };
-  hipLaunchKernelGGL(prefill_gemm_kernel<true>, dim3(grid_of(nt_gu)), dim3(256), gemm_lds_bytes(p.H / 64), st, g,
-                     nt_gu);
+  // An expert with rows fills at most its rows / 128 whole M blocks and one partial one, so the grid covers that bound
+  // (rounded up to a multiple of 8) times the N tiles; blocks past the device-side count exit at once.
+  const int64_t P = padded_rows(p.R, p.num_local, kBM);
+  const int64_t bound = (p.R < p.num_local ? p.R : p.num_local) + p.R / kBM;
+  const int64_t mb = bound < P / kBM ? bound : P / kBM;
+  // Tiles: with few rows per expert most M blocks are light and the chip is short of blocks, so a wave takes two
+  // weight fragments instead of four (twice the blocks); with more rows the wider wave reads its activations from LDS
+  // half as often. Measured with 512 experts (us, two / four fragments): gate/up R = 190 24 / 27, 3330 (H 2560 /
+  // I 640) 85 / 90, 6000 67 / 72, 20480 139 / 124; down R = 190 15 / 17, 480 20 / 20, 3330 55 / 54, 6000 48 / 43.
+  // Two down tiles per block (one prologue) pay off once there are blocks to spare: R = 6000 43 / 43, 10000 (H 2560)
+  // 95 against 101 with one, 81920 280 against 300.
+  const int nb_gu = p.R < 16 * (int64_t)p.num_local ? 2 : 4, nb_d = p.R < 2 * (int64_t)p.num_local ? 2 : 4;
+  const int td = p.R >= 8192 && p.H % 512 == 0 ? 2 : 1;
+  launch_gemm<true>(g, nb_gu, 1, mb, st);
   g.a = p.h_buf;
   g.w_off = rec.dw;
   g.s_off = rec.ds;
   g.b_off = rec.db;
-  hipLaunchKernelGGL(prefill_gemm_kernel<false>, dim3(grid_of(nt_d)), dim3(256), gemm_lds_bytes(p.I / 64), st, g,
-                     nt_d);
+  launch_gemm<false>(g, nb_d, td, mb, st);
   return hipGetLastError();
 }
 

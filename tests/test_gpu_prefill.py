@@ -98,6 +98,31 @@ def test_prefill_rows_independent_of_batch():
     assert torch.equal(layer.out_rows[:half * K], full[:half * K])
 
 
+@pytest.mark.parametrize("H,I", [(256, 128), (512, 384), (2560, 640)])
+def test_prefill_rows_same_bits_for_every_tile_shape(H, I):
+    """Gate/up and down take two or four weight fragments per wave and one or two down tiles per block by the number of
+    rows; live fragments and steps per LDS stage follow the rows of a block. A row's bits are the same under all of
+    them (steps of 128 K: 2 to 20, odd at I 384 and 640), and agree with the oracle."""
+    T, K, E = 2100, 4, 8
+    pool, x, ids, w = _prefill_case(T, K, E, H, I, 7 * H + I)
+    lw = LayerWeights(H, E, 64, seed=3)
+    layer = MoEPrefillLayer(pool, 0, lw.router_w, lw.sh_gate, lw.sh_up, lw.sh_down, lw.sh_g, top_k=K, max_tokens=T)
+    layer.routed_experts(x, ids, w)                      # R = 8400: four fragments, two down tiles where H allows
+    torch.cuda.synchronize()
+    h_full, rows_full = layer.h_buf[:T * K].clone(), layer.out_rows[:T * K].clone()
+    for t in (1, 3, 4, 20, 31, 33, 45, 64, 100, 150, 190, 230, 300):  # R 4 .. 1200: up to 150 rows per expert
+        layer.h_buf.fill_(7.0)
+        layer.out_rows.fill_(7.0)
+        layer.routed_experts(x[:t].contiguous(), ids[:t].contiguous(), w[:t].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(layer.h_buf[:t * K], h_full[:t * K]), t
+        assert torch.equal(layer.out_rows[:t * K], rows_full[:t * K]), t
+        assert bool((layer.out_rows[t * K:] == 7.0).all()), t
+    t = 60
+    _, rows_ref = _oracle_rows(pool, x[:t].contiguous(), ids[:t].contiguous(), w[:t].contiguous())
+    assert O.rel_l2(rows_full[:t * K].cpu().numpy(), rows_ref) < 2e-3
+
+
 def test_fused_moe_affine_group_semantics():
     """The reference interface: a group of local experts through expert_map; rows outside it are left alone."""
     T, K, E, H, I = 40, 4, 12, 256, 128
