@@ -145,9 +145,33 @@ int64_t align_scratch_ints(int64_t R, int num_local);
 hipError_t launch_moe_align(const AlignArgs& a, hipStream_t st);
 
 constexpr int kPrefillBlockM = 128;  // the moe_align block the grouped GEMM consumes
+// One M block (kPrefillBlockM positions of sorted_rows, one expert) of a plan in launch order.
+struct alignas(16) MBlock {
+  int64_t record;   // the expert's record base address
+  int32_t expert;
+  int32_t index;    // M block of the plan
+};
+// The plan of R rows over the E experts of one resident layer, straight from the router's ids.
+struct ResidentPlan {
+  const int32_t* ids;  // [R] expert ids
+  const int32_t* map;
+  int64_t map_base, map_len;
+  const int64_t* slot_ptr;
+  int64_t n_slots, R;
+  int E;
+  int32_t* local;         // [R] the expert, or -1 when the id is out of range or not resident (status raised)
+  int32_t* sorted_rows;   // [resident_plan_blocks() * kPrefillBlockM]
+  int32_t* block_expert;  // [resident_plan_blocks()]
+  MBlock* order;          // [resident_plan_blocks()]
+  int32_t* num_padded;    // [1]
+  int32_t* scratch;       // align_scratch_ints(R, E) ints
+  int* err;
+};
+int64_t resident_plan_blocks(int64_t R, int E);
+hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st);
 struct PrefillArgs {
   const uint16_t* x;            // bf16 [T, H]
-  const int32_t* row_token;     // [R]
+  const int32_t* row_token;     // [R], or null: row r belongs to token r / topk
   const float* row_weight;      // [R]
   const int32_t* sorted_rows;   // moe_align plan with block_m = kPrefillBlockM
   const int32_t* block_expert;
@@ -158,17 +182,14 @@ struct PrefillArgs {
   float* out_rows;              // fp32 [R, H]
   int64_t R;
   int T, H, I;                  // T: rows of x (a row_token outside [0, T) reads zeros)
+  const MBlock* order = nullptr;  // the M blocks in launch order, or null (plan order, block_expert and group_ptr)
+  int topk = 1;
   uint64_t* trace = nullptr;    // diagnostics: per-block stamps of the two GEMMs (16384 entries), or null
 };
 hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st);
 // out[t] = sum over k (in order) of rows[t * K + k]; a row whose row_local entry is negative counts as +0.
 hipError_t launch_combine(const float* rows, const int32_t* row_local, int T, int K, int H, float* out,
                           hipStream_t st);
-// Resident-pool tables of a prefill: group_ptr[e] from map/slot_ptr, local[r] = ids[r] (or -1, raising a status
-// bit, when the expert is out of range or not resident), row_token[r] = r / K.
-hipError_t launch_prefill_tables(const int32_t* map, int64_t map_base, int64_t map_len, const int64_t* slot_ptr,
-                                 int64_t n_slots, int E, int64_t* gptr, const int32_t* ids, int64_t R, int K,
-                                 int32_t* local, int32_t* row_token, int* err, hipStream_t st);
 
 // Reference sampler (ss_sampler.hip): Sampler.next over one row with sanitized parameters; u a device float.
 int64_t sample_workspace_bytes(int V);

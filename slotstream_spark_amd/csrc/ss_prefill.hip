@@ -20,7 +20,11 @@
 namespace ss {
 
 // ---------------------------------------------------------------- moe_align
-constexpr int kAlignChunk = 256;
+// Three launches (count, scan, place), or one workgroup for up to kAlignChunk rows and keys: the plan is a chain of
+// small dependent steps, so what it costs is launches and the latency inside each (19 tokens x top-10, 512 experts:
+// seven launches of 1.2-4.2 us each and their gaps before, table look-ups included, one of 10 us now).
+constexpr int kAlignChunk = 1024;         // rows per workgroup of the counting kernel
+constexpr int kAlignWaves = kAlignChunk / 64;
 
 int64_t padded_rows(int64_t R, int num_local, int block_m) {
   const int64_t n = R + (int64_t)num_local * (block_m - 1);
@@ -33,171 +37,325 @@ int64_t align_scratch_ints(int64_t R, int num_local) {
   return R + nch * num_local + 2 * (int64_t)num_local + 1;
 }
 
-SS_DEV int align_key(const int32_t* le, int64_t i, int64_t R, int nl) {
-  if (i >= R) return nl + 1;
-  const int v = le[i];
-  return (v >= 0 && v < nl) ? v : nl;
+namespace {
+
+struct PlanArgs {
+  const int32_t* le;  // [R] local expert of each row, or null: the rows' expert ids through the resident tables
+  const int32_t* ids;
+  const int32_t* map;
+  int64_t map_base, map_len;
+  const int64_t* slot_ptr;
+  int64_t n_slots;
+  int32_t* local;     // [R] local expert written with `ids` (-1: not resident)
+  int* err;
+  int64_t R, P, nb;   // rows; positions of sorted_rows to fill; entries of block_expert
+  int nl, bm, nch;
+  int32_t* rank;
+  int32_t* chunk;
+  int32_t* pad;
+  int32_t* tot;
+  int32_t* sorted_rows;
+  int32_t* block_expert;
+  int32_t* num_padded;
+  MBlock* order;      // null, or the M blocks in launch order
+};
+
+// Key of row i: its local expert, nl for a row that is skipped, nl + 1 past R.
+template <bool IDS>
+SS_DEV int align_key(const PlanArgs& a, int64_t i) {
+  if (i >= a.R) return a.nl + 1;
+  if constexpr (!IDS) {
+    const int v = a.le[i];
+    return (v >= 0 && v < a.nl) ? v : a.nl;
+  } else {
+    const int e = a.ids[i];
+    if (e < 0 || e >= a.nl) {
+      ss_raise(a.err, SS_ERR_EXPERT_ID);
+      return a.nl;
+    }
+    const int64_t mi = a.map_base + e;
+    const int slot = mi < a.map_len ? a.map[mi] : -1;
+    if (slot >= 0 && slot < a.n_slots) return e;
+    ss_raise(a.err, SS_ERR_SLOT);
+    return a.nl;
+  }
 }
 
-// Per chunk: the rank of each row among the earlier rows of the chunk with the same key, and per-key counts.
-// Inside a wave the rank is the number of lower lanes holding the same key (one ballot per distinct key of the
-// wave, taken in lane order); the earlier waves of the chunk add their counts of that key from LDS.
-__global__ __launch_bounds__(kAlignChunk) void align_count_kernel(const int32_t* __restrict__ le, int64_t R, int nl,
-                                                                  int32_t* __restrict__ rank,
-                                                                  int32_t* __restrict__ chunk_cnt) {
-  extern __shared__ uint8_t sm_cnt[];  // [kAlignChunk / 64 waves][nl + 2]: per-wave counts (<= 64) of every key
+// Rank of each thread's row among the earlier rows of the workgroup with the same key, and the workgroup's count of
+// every key (cnt[w * nk + key], summed by the caller). Inside a wave the lanes holding the same key are the AND of the
+// ballots of the key's bits; the earlier waves add their counts of that key from LDS.
+SS_DEV int align_rank(int key, int nk, uint8_t* cnt) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  constexpr int NW = kAlignChunk / 64;
-  const int nk = nl + 2;  // keys 0 .. nl + 1 (nl: outside [0, nl), nl + 1: past R)
-  const int64_t i = (int64_t)blockIdx.x * kAlignChunk + tid;
-  const int key = align_key(le, i, R, nl);
-  for (int e = tid; e < NW * nk; e += kAlignChunk) sm_cnt[e] = 0;
+  for (int e = tid; e < kAlignWaves * nk; e += kAlignChunk) cnt[e] = 0;
   __syncthreads();
-  // rank inside the wave: walk the wave's distinct keys in the order of their lowest lane
-  int r_in = 0;
-  uint64_t todo = ~0ull;
-  while (todo) {
-    const int l0 = (int)__builtin_ctzll(todo);
-    const int k0 = __builtin_amdgcn_readlane(key, l0);
-    const uint64_t same = __ballot(key == k0);
-    if (key == k0) r_in = __popcll(same & ((1ull << lane) - 1ull));
-    if (lane == l0) sm_cnt[w * nk + k0] = (uint8_t)__popcll(same);
-    todo &= ~same;
+  uint64_t same = ~0ull;
+  for (int b = 0; (nk - 1) >> b; ++b) {
+    const uint64_t set = __ballot((key >> b) & 1);
+    same &= (key >> b) & 1 ? set : ~set;
   }
+  int r = __popcll(same & ((1ull << lane) - 1ull));
+  if (r == 0) cnt[w * nk + key] = (uint8_t)__popcll(same);
   __syncthreads();
-  int r = r_in;
-  for (int v = 0; v < w; ++v) r += sm_cnt[v * nk + key];
-  if (i < R) rank[i] = r;
-  for (int e = tid; e < nl; e += kAlignChunk) {
-    int c = 0;
-#pragma unroll
-    for (int v = 0; v < NW; ++v) c += sm_cnt[v * nk + e];
-    chunk_cnt[(int64_t)blockIdx.x * nl + e] = c;
-  }
+  for (int v = 0; v < w; ++v) r += cnt[v * nk + key];
+  return r;
 }
 
-__global__ void align_zero_kernel(int nl, int32_t* __restrict__ tot) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e < nl) tot[e] = 0;
+SS_DEV int align_count_of(const uint8_t* cnt, int nk, int e) {
+  int c = 0;
+#pragma unroll
+  for (int v = 0; v < kAlignWaves; ++v) c += cnt[v * nk + e];
+  return c;
 }
 
-// Per key: exclusive offsets of the key's rows in each chunk (chunk order) and the key's total. One thread per key;
-// its nch loads are independent, so they are all in flight at once.
-__global__ __launch_bounds__(256) void align_keyscan_kernel(int nl, int nch, int32_t* __restrict__ chunk_cnt,
-                                                            int32_t* __restrict__ tot) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= nl) return;
-  int run = 0;
-  for (int c0 = 0; c0 < nch; c0 += 32) {
-    int v[32];
+// Record of expert e (0 when it is not resident; its rows are skipped, so no block names it).
+SS_DEV int64_t record_of(const PlanArgs& a, int e) {
+  const int64_t mi = a.map_base + e;
+  const int slot = mi < a.map_len ? a.map[mi] : -1;
+  return slot >= 0 && slot < a.n_slots ? a.slot_ptr[slot] : 0;
+}
+
+// One workgroup of 1024: the padded start of every key (ps, nl + 1 entries; hv: the heavy blocks before it), the
+// expert of every M block and, with `order`, the blocks in launch order. Thread t holds the totals of keys
+// kpt t .. kpt t + kpt - 1 in loc.
+// Launch order: blocks with more than half their rows first, the others behind them, so the light blocks fill the
+// chip's tail instead of leaving it to a few heavy ones (gate/up at 2048 tokens 136 -> 124 us, at 333 105 -> 92).
+SS_DEV void align_scan(const PlanArgs& a, const int (&loc)[4], int kpt, int* ps, int* hv) {
+  __shared__ int wsum[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int bm = a.bm, nl = a.nl;
+  auto blocks_of = [&](int c) { return (c + bm - 1) / bm; };
+  auto heavy_of = [&](int c) { return c / bm + (c % bm > bm / 2 ? 1 : 0); };
+  int nbk = 0, nh = 0;
 #pragma unroll
-    for (int q = 0; q < 32; ++q) v[q] = c0 + q < nch ? chunk_cnt[(int64_t)(c0 + q) * nl + e] : 0;
+  for (int q = 0; q < 4; ++q)
+    if (q < kpt) {
+      nbk += blocks_of(loc[q]);
+      nh += heavy_of(loc[q]);
+    }
+  int ib = nbk, ih = nh;  // inclusive scans over the wave, then over the waves
 #pragma unroll
-    for (int q = 0; q < 32; ++q) {
-      if (c0 + q < nch) chunk_cnt[(int64_t)(c0 + q) * nl + e] = run;
-      run += v[q];
+  for (int off = 1; off < 64; off <<= 1) {
+    const int vb = __shfl_up(ib, off), vh = __shfl_up(ih, off);
+    if (lane >= off) {
+      ib += vb;
+      ih += vh;
     }
   }
-  tot[e] = run;
-}
-
-// One workgroup: exclusive scan of the padded key sizes -> pad[0 .. nl] (pad[nl] = num_padded), and the expert of
-// every block of bm positions (-1 past num_padded).
-__global__ __launch_bounds__(1024) void align_padscan_kernel(int nl, int bm, int64_t nb, const int32_t* __restrict__ tot,
-                                                             int32_t* __restrict__ pad, int32_t* __restrict__ block_expert,
-                                                             int32_t* __restrict__ num_padded) {
-  extern __shared__ int ps[];  // [nl + 1]
-  __shared__ int part[1024];
-  const int tid = threadIdx.x;
-  // Each thread sums up to 4 consecutive keys, a Hillis-Steele scan over the 1024 thread totals, then the per-thread
-  // prefixes (nl <= 4096).
-  int loc[4], sum = 0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int e = 4 * tid + q;
-    loc[q] = e < nl ? (tot[e] + bm - 1) / bm * bm : 0;
-    sum += loc[q];
-  }
-  part[tid] = sum;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int v = tid >= off ? part[tid - off] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  int run = part[tid] - sum;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int e = 4 * tid + q;
-    if (e < nl) ps[e] = run;
-    run += loc[q];
-  }
-  if (tid == 1023) {
-    ps[nl] = part[1023];
-    *num_padded = part[1023];
+  if (lane == 63) {
+    wsum[0][w] = ib;
+    wsum[1][w] = ih;
   }
   __syncthreads();
-  for (int e = tid; e <= nl; e += 1024) pad[e] = ps[e];
-  for (int64_t q = tid; q < nb; q += 1024) {
+  int run = ib - nbk, runh = ih - nh;
+  for (int v = 0; v < w; ++v) {
+    run += wsum[0][v];
+    runh += wsum[1][v];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int e = kpt * tid + q;
+    if (q < kpt && e < nl) {
+      ps[e] = run * bm;
+      hv[e] = runh;
+      run += blocks_of(loc[q]);
+      runh += heavy_of(loc[q]);
+      if (e == nl - 1) {
+        ps[nl] = run * bm;
+        hv[nl] = runh;
+      }
+    }
+  }
+  __syncthreads();
+  const int total = ps[nl], nheavy = hv[nl];
+  if (tid == 0) *a.num_padded = total;
+  for (int64_t q = tid; q < a.nb; q += 1024) {
     const int64_t pos = q * bm;
-    // the last key e with ps[e] <= pos (binary search), -1 past the end
-    int lo = 0, hi = nl;
+    if (pos >= total) {
+      a.block_expert[q] = -1;
+      continue;
+    }
+    int lo = 0, hi = nl;  // the last key e with ps[e] <= pos
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
       if (ps[mid] <= pos) lo = mid;
       else hi = mid - 1;
     }
-    block_expert[q] = pos < ps[nl] ? lo : -1;
+    a.block_expert[q] = lo;
+    if (a.order) {
+      const int b0 = ps[lo] / bm, j = (int)q - b0, h = hv[lo + 1] - hv[lo];
+      const int at = j < h ? hv[lo] + j : nheavy + (b0 - hv[lo]) + (j - h);
+      a.order[at] = MBlock{record_of(a, lo), lo, (int32_t)q};
+    }
   }
 }
 
-// Sentinel R at every position that holds no row: past a key's rows inside its padded range, and past num_padded.
-__global__ __launch_bounds__(256) void align_fill_kernel(int64_t R, int nl, int bm, int64_t P,
-                                                         const int32_t* __restrict__ pad, const int32_t* __restrict__ tot,
-                                                         const int32_t* __restrict__ block_expert,
-                                                         int32_t* __restrict__ sorted_rows) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= P) return;
-  const int e = block_expert[p / bm];
-  if (e < 0 || p - pad[e] >= tot[e]) sorted_rows[p] = (int32_t)R;
-}
+}  // namespace
 
-__global__ __launch_bounds__(kAlignChunk) void align_scatter_kernel(const int32_t* __restrict__ le, int64_t R, int nl,
-                                                                    const int32_t* __restrict__ rank,
-                                                                    const int32_t* __restrict__ chunk_off,
-                                                                    const int32_t* __restrict__ pad,
-                                                                    int32_t* __restrict__ sorted_rows) {
+// Per chunk of rows: ranks and counts of every key.
+template <bool IDS>
+__global__ __launch_bounds__(kAlignChunk) void align_count_kernel(PlanArgs a) {
+  extern __shared__ uint8_t sm_cnt[];  // [kAlignWaves][nl + 2]: per-wave counts (<= 64) of keys 0 .. nl + 1
   const int64_t i = (int64_t)blockIdx.x * kAlignChunk + threadIdx.x;
-  const int key = align_key(le, i, R, nl);
-  if (key < nl) sorted_rows[pad[key] + chunk_off[(int64_t)blockIdx.x * nl + key] + rank[i]] = (int32_t)i;
+  const int key = align_key<IDS>(a, i), nk = a.nl + 2;
+  const int r = align_rank(key, nk, sm_cnt);
+  if (i < a.R) {
+    a.rank[i] = r;
+    if (IDS) a.local[i] = key < a.nl ? key : -1;
+  }
+  for (int e = threadIdx.x; e < a.nl; e += kAlignChunk)
+    a.chunk[(int64_t)blockIdx.x * a.nl + e] = align_count_of(sm_cnt, nk, e);
 }
 
-hipError_t launch_moe_align(const AlignArgs& a, hipStream_t st) {
-  const int nch = (int)((a.R + kAlignChunk - 1) / kAlignChunk);
-  int32_t* rank = a.scratch;
-  int32_t* chunk = rank + a.R;
-  int32_t* pad = chunk + (int64_t)nch * a.num_local;
-  int32_t* tot = pad + a.num_local + 1;
-  const int64_t P = padded_rows(a.R, a.num_local, a.block_m);
-  if (nch > 0) {
-    hipLaunchKernelGGL(align_count_kernel, dim3(nch), dim3(kAlignChunk), (size_t)(kAlignChunk / 64) * (a.num_local + 2),
-                       st, a.local_expert,
-                       a.R, a.num_local, rank, chunk);
-    hipLaunchKernelGGL(align_keyscan_kernel, dim3((a.num_local + 255) / 256), dim3(256), 0, st, a.num_local, nch,
-                       chunk, tot);
-  } else {
-    hipLaunchKernelGGL(align_zero_kernel, dim3((a.num_local + 255) / 256), dim3(256), 0, st, a.num_local, tot);
+// One workgroup: exclusive offsets of every key over the chunks (in place) and its total, then the padded starts, the
+// blocks' experts and the launch order. A thread's loads over the chunks are independent, 32 in flight at once.
+__global__ __launch_bounds__(1024) void align_scan_kernel(PlanArgs a) {
+  extern __shared__ int sm_scan[];  // [2][nl + 1]
+  int* ps = sm_scan;
+  int* hv = sm_scan + a.nl + 1;
+  const int tid = threadIdx.x, nl = a.nl, kpt = (nl + 1023) / 1024;
+  int loc[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int e = kpt * tid + q;
+    if (q >= kpt || e >= nl) continue;
+    int run = 0;
+    for (int c0 = 0; c0 < a.nch; c0 += 32) {
+      int v[32];
+#pragma unroll
+      for (int c = 0; c < 32; ++c) v[c] = c0 + c < a.nch ? a.chunk[(int64_t)(c0 + c) * nl + e] : 0;
+#pragma unroll
+      for (int c = 0; c < 32; ++c) {
+        if (c0 + c < a.nch) a.chunk[(int64_t)(c0 + c) * nl + e] = run;
+        run += v[c];
+      }
+    }
+    loc[q] = run;
+    a.tot[e] = run;
   }
-  hipLaunchKernelGGL(align_padscan_kernel, dim3(1), dim3(1024), (size_t)(a.num_local + 1) * 4, st, a.num_local,
-                     a.block_m, P / a.block_m, tot, pad, a.block_expert, a.num_padded);
-  if (P > 0)
-    hipLaunchKernelGGL(align_fill_kernel, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, st, a.R, a.num_local,
-                       a.block_m, P, pad, tot, a.block_expert, a.sorted_rows);
-  if (nch > 0)
-    hipLaunchKernelGGL(align_scatter_kernel, dim3(nch), dim3(kAlignChunk), 0, st, a.local_expert, a.R, a.num_local,
-                       rank, chunk, pad, a.sorted_rows);
+  align_scan(a, loc, kpt, ps, hv);
+  for (int e = tid; e <= nl; e += 1024) a.pad[e] = ps[e];
+}
+
+// sorted_rows: the row at every position that holds one, the sentinel R elsewhere (past a key's rows inside its padded
+// range and past num_padded; with `order` positions past num_padded are left alone, no block reads them).
+__global__ __launch_bounds__(256) void align_place_kernel(PlanArgs a) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (p < a.P) {
+    const int e = a.block_expert[p / a.bm];
+    if (e < 0 ? a.order == nullptr : p - a.pad[e] >= a.tot[e]) a.sorted_rows[p] = (int32_t)a.R;
+  }
+  if (p < a.R) {
+    const int v = a.le[p], key = v >= 0 && v < a.nl ? v : a.nl;
+    if (key < a.nl) a.sorted_rows[a.pad[key] + a.chunk[p / kAlignChunk * a.nl + key] + a.rank[p]] = (int32_t)p;
+  }
+}
+
+// The whole plan in one workgroup (R and num_local up to kAlignChunk).
+template <bool IDS>
+__global__ __launch_bounds__(kAlignChunk) void align_small_kernel(PlanArgs a) {
+  extern __shared__ int sm_small[];  // [2][nl + 1] ints, [nl] totals, then the per-wave counts
+  const int tid = threadIdx.x, nl = a.nl, nk = nl + 2;
+  int* ps = sm_small;
+  int* hv = ps + nl + 1;
+  int* tot = hv + nl + 1;
+  uint8_t* cnt = reinterpret_cast<uint8_t*>(tot + nl);
+  const int key = align_key<IDS>(a, tid);
+  const int r = align_rank(key, nk, cnt);
+  if (IDS && tid < a.R) a.local[tid] = key < nl ? key : -1;
+  int loc[4] = {0, 0, 0, 0};
+  if (tid < nl) tot[tid] = loc[0] = align_count_of(cnt, nk, tid);
+  align_scan(a, loc, 1, ps, hv);
+  const int total = ps[nl];
+  const int64_t fill = a.order ? total : a.P;
+  for (int64_t p = tid; p < fill; p += kAlignChunk) {
+    bool none = p >= total;
+    if (!none) {
+      int lo = 0, hi = nl;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (ps[mid] <= p) lo = mid;
+        else hi = mid - 1;
+      }
+      none = p - ps[lo] >= tot[lo];
+    }
+    if (none) a.sorted_rows[p] = (int32_t)a.R;
+  }
+  if (key < nl) a.sorted_rows[ps[key] + r] = tid;
+}
+
+static hipError_t launch_plan(PlanArgs a, int32_t* scratch, hipStream_t st) {
+  a.nch = (int)((a.R + kAlignChunk - 1) / kAlignChunk);
+  a.rank = scratch;
+  a.chunk = a.rank + a.R;
+  a.pad = a.chunk + (int64_t)a.nch * a.nl;
+  a.tot = a.pad + a.nl + 1;
+  const bool ids = a.le == nullptr;
+  const size_t cnt = (size_t)kAlignWaves * (a.nl + 2);
+  if (a.R <= kAlignChunk && a.nl <= kAlignChunk) {
+    const size_t lds = (size_t)(3 * a.nl + 2) * 4 + cnt;
+    if (ids) hipLaunchKernelGGL(align_small_kernel<true>, dim3(1), dim3(kAlignChunk), lds, st, a);
+    else hipLaunchKernelGGL(align_small_kernel<false>, dim3(1), dim3(kAlignChunk), lds, st, a);
+    return hipGetLastError();
+  }
+  if (a.nch > 0) {
+    // up to 64 KB and a little more with 4096 experts
+    KernelCfg cfg;
+    hipError_t e = kernel_cfg(reinterpret_cast<const void*>(align_count_kernel<true>), kAlignChunk, 72 * 1024, &cfg);
+    if (e == hipSuccess)
+      e = kernel_cfg(reinterpret_cast<const void*>(align_count_kernel<false>), kAlignChunk, 72 * 1024, &cfg);
+    if (e != hipSuccess) return e;
+    if (ids) hipLaunchKernelGGL(align_count_kernel<true>, dim3(a.nch), dim3(kAlignChunk), cnt, st, a);
+    else hipLaunchKernelGGL(align_count_kernel<false>, dim3(a.nch), dim3(kAlignChunk), cnt, st, a);
+  }
+  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(1024), (size_t)(2 * a.nl + 2) * 4, st, a);
+  if (ids) a.le = a.local;
+  const int64_t n = a.P > a.R ? a.P : a.R;
+  if (n > 0) hipLaunchKernelGGL(align_place_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
+}
+
+hipError_t launch_moe_align(const AlignArgs& q, hipStream_t st) {
+  PlanArgs a{};
+  a.le = q.local_expert;
+  a.R = q.R;
+  a.nl = q.num_local;
+  a.bm = q.block_m;
+  a.P = padded_rows(q.R, q.num_local, q.block_m);
+  a.nb = a.P / q.block_m;
+  a.sorted_rows = q.sorted_rows;
+  a.block_expert = q.block_expert;
+  a.num_padded = q.num_padded;
+  // no rows: nothing is read through le, which may be null
+  if (q.R == 0) a.le = reinterpret_cast<const int32_t*>(q.scratch);
+  return launch_plan(a, q.scratch, st);
+}
+
+// M blocks a plan of R rows over E experts can have: an expert with rows fills its rows / kBM whole blocks and at most
+// one more.
+static int64_t mblock_bound(int64_t R, int E) { return (R < E ? R : E) + R / kPrefillBlockM; }
+
+int64_t resident_plan_blocks(int64_t R, int E) { return mblock_bound(R, E); }
+
+hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
+  PlanArgs a{};
+  a.ids = q.ids;
+  a.map = q.map;
+  a.map_base = q.map_base;
+  a.map_len = q.map_len;
+  a.slot_ptr = q.slot_ptr;
+  a.n_slots = q.n_slots;
+  a.local = q.local;
+  a.err = q.err;
+  a.R = q.R;
+  a.nl = q.E;
+  a.bm = kPrefillBlockM;
+  a.nb = mblock_bound(q.R, q.E);
+  a.P = a.nb * kPrefillBlockM;
+  a.sorted_rows = q.sorted_rows;
+  a.block_expert = q.block_expert;
+  a.num_padded = q.num_padded;
+  a.order = q.order;
+  return launch_plan(a, q.scratch, st);
 }
 
 // ---------------------------------------------------------------- grouped GEMM
@@ -277,6 +435,8 @@ struct GemmArgs {
   const int32_t* block_expert; // [P / kBM]
   const int32_t* num_padded;   // [1]
   const int64_t* group_ptr;    // [num_local] record base addresses
+  const MBlock* order;         // null, or the M blocks in launch order (then block_expert and group_ptr are unused)
+  int topk;                    // with row_token null: row r belongs to token r / topk
   uint16_t* h;                 // gate/up output bf16 [R, I]
   float* out_rows;             // down output fp32 [R, H]
   int64_t R;
@@ -530,10 +690,19 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmArgs g, int nt
   const int mb = g.num_padded[0] / kBM;
   int pid_m, pid_n;
   if (!xcd_tile(mb, nt, pid_m, pid_n)) return;
-  const int e = g.block_expert[pid_m];
-  if (e < 0) return;
+  int e;
+  const uint8_t* base;
+  if (g.order) {
+    const MBlock b = g.order[pid_m];
+    e = b.expert;
+    pid_m = b.index;
+    base = reinterpret_cast<const uint8_t*>(b.record);
+  } else {
+    e = g.block_expert[pid_m];
+    if (e < 0) return;
+    base = reinterpret_cast<const uint8_t*>(g.group_ptr[e]);
+  }
   const uint64_t t_start = g.trace ? __builtin_amdgcn_s_memrealtime() : 0;
-  const uint8_t* base = reinterpret_cast<const uint8_t*>(g.group_ptr[e]);
   bool valid = false;
   if (tid < kBM) {
     const int r = g.sorted_rows[(int64_t)pid_m * kBM + tid];
@@ -541,7 +710,7 @@ __global__ __launch_bounds__(256, 2) void prefill_gemm_kernel(GemmArgs g, int nt
     int row = kZeroRow;
     if (valid) {
       if (GU) {
-        const int t = g.row_token[r];
+        const int t = g.row_token ? g.row_token[r] : (int)((uint32_t)r / (uint32_t)g.topk);
         if (t >= 0 && t < g.T) row = t;
       } else {
         row = r;
@@ -595,6 +764,8 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
   g.block_expert = p.block_expert;
   g.num_padded = p.num_padded;
   g.group_ptr = p.group_ptr;
+  g.order = p.order;
+  g.topk = p.topk;
   g.h = p.h_buf;
   g.out_rows = p.out_rows;
   g.R = p.R;
@@ -610,10 +781,9 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
   g.w2_off = rec.uw;
   g.s2_off = rec.us;
   g.b2_off = rec.ub;
-  // An expert with rows fills at most its rows / 128 whole M blocks and one partial one, so the grid covers that bound
-  // (rounded up to a multiple of 8) times the N tiles; blocks past the device-side count exit at once.
-  const int64_t P = padded_rows(p.R, p.num_local, kBM);
-  const int64_t bound = (p.R < p.num_local ? p.R : p.num_local) + p.R / kBM;
+  // Grids cover the bound of M blocks (rounded up to a multiple of 8) times the N tiles; blocks past the device-side
+  // count exit at once.
+  const int64_t P = padded_rows(p.R, p.num_local, kBM), bound = mblock_bound(p.R, p.num_local);
   const int64_t mb = bound < P / kBM ? bound : P / kBM;
   // Tiles: with few rows per expert most M blocks are light and the chip is short of blocks, so a wave takes two
   // weight fragments instead of four (twice the blocks); with more rows the wider wave reads its activations from LDS
@@ -662,47 +832,6 @@ hipError_t launch_combine(const float* rows, const int32_t* row_local, int T, in
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(combine_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rows, row_local, T, K, H,
                      out);
-  return hipGetLastError();
-}
-
-// group_ptr[e] = slot_ptr[map[map_base + e]] for the resident-pool entry point (0 when absent: such rows are
-// skipped by setting their local expert to -1 in the caller's routing).
-__global__ void group_ptr_kernel(const int32_t* __restrict__ map, int64_t map_base, int64_t map_len,
-                                 const int64_t* __restrict__ slot_ptr, int64_t n_slots, int E, int64_t* gptr,
-                                 const int32_t* __restrict__ ids, int64_t R, int32_t* __restrict__ local, int* err) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < E) {
-    const int64_t mi = map_base + i;
-    const int slot = mi < map_len ? map[mi] : -1;
-    gptr[i] = (slot >= 0 && slot < n_slots) ? slot_ptr[slot] : 0;
-  }
-  if (i < R) {
-    const int e = ids[i];
-    int le = -1;
-    if (e >= 0 && e < E) {
-      const int64_t mi = map_base + e;
-      const int slot = mi < map_len ? map[mi] : -1;
-      if (slot >= 0 && slot < n_slots) le = e;
-      else ss_raise(err, SS_ERR_SLOT);
-    } else {
-      ss_raise(err, SS_ERR_EXPERT_ID);
-    }
-    local[i] = le;
-  }
-}
-
-__global__ void row_token_kernel(int64_t R, int K, int32_t* row_token) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < R) row_token[i] = (int32_t)(i / K);
-}
-
-hipError_t launch_prefill_tables(const int32_t* map, int64_t map_base, int64_t map_len, const int64_t* slot_ptr,
-                                 int64_t n_slots, int E, int64_t* gptr, const int32_t* ids, int64_t R, int K,
-                                 int32_t* local, int32_t* row_token, int* err, hipStream_t st) {
-  const int64_t n = R > E ? R : E;
-  hipLaunchKernelGGL(group_ptr_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, map, map_base, map_len,
-                     slot_ptr, n_slots, E, gptr, ids, R, local, err);
-  if (R > 0) hipLaunchKernelGGL(row_token_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, R, K, row_token);
   return hipGetLastError();
 }
 

@@ -743,27 +743,25 @@ int ssmoe_combine_rank_order(const float* out_rows, int T, int K, int H, float* 
                    "combine launch");
 }
 
-// Workspace of ssmoe_moe_prefill: local [R], row_token [R], group_ptr [E] (8-byte), sorted_rows [P],
-// block_expert [P / kPrefillBlockM], num_padded, then the moe_align scratch.
+// Workspace of ssmoe_moe_prefill: local [R], sorted_rows [M blocks x 128], block_expert and launch order [M blocks],
+// num_padded, then the plan's scratch.
 struct PrefillWs {
-  int64_t local, row_token, gptr, sorted, bexp, npad, scratch, total;
+  int64_t local, sorted, bexp, order, npad, scratch, total;
 };
 static PrefillWs prefill_ws(int64_t T, int K, int E) {
   const int64_t R = T * K;
-  const int64_t P = ss::padded_rows(R, E, ss::kPrefillBlockM);
+  const int64_t nb = ss::resident_plan_blocks(R, E);
   auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
   PrefillWs w{};
   int64_t o = 0;
   w.local = o;
   o = up(o + R * 4);
-  w.row_token = o;
-  o = up(o + R * 4);
-  w.gptr = o;
-  o = up(o + (int64_t)E * 8);
   w.sorted = o;
-  o = up(o + P * 4);
+  o = up(o + nb * ss::kPrefillBlockM * 4);
   w.bexp = o;
-  o = up(o + P / ss::kPrefillBlockM * 4);
+  o = up(o + nb * 4);
+  w.order = o;
+  o = up(o + nb * (int64_t)sizeof(ss::MBlock));
   w.npad = o;
   o = up(o + 4);
   w.scratch = o;
@@ -800,35 +798,32 @@ int ssmoe_moe_prefill(const uint16_t* x, const int32_t* expert_ids, const float*
   if (int rc = status_ptr(&err)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
-  int32_t* local = reinterpret_cast<int32_t*>(ws + w.local);
-  int32_t* row_token = reinterpret_cast<int32_t*>(ws + w.row_token);
-  int64_t* gptr = reinterpret_cast<int64_t*>(ws + w.gptr);
-  int32_t* sorted = reinterpret_cast<int32_t*>(ws + w.sorted);
-  int32_t* bexp = reinterpret_cast<int32_t*>(ws + w.bexp);
-  int32_t* npad = reinterpret_cast<int32_t*>(ws + w.npad);
   const int64_t R = T * K;
-  if (int rc = hip_check(ss::launch_prefill_tables(map, (int64_t)layer * E, map_len, slot_ptr, n_slots, E, gptr,
-                                                   expert_ids, R, K, local, row_token, err, st),
-                         "prefill tables launch"))
-    return rc;
-  ss::AlignArgs al{};
-  al.local_expert = local;
-  al.R = R;
-  al.num_local = E;
-  al.block_m = ss::kPrefillBlockM;
-  al.sorted_rows = sorted;
-  al.block_expert = bexp;
-  al.num_padded = npad;
-  al.scratch = reinterpret_cast<int32_t*>(ws + w.scratch);
-  if (int rc = hip_check(ss::launch_moe_align(al, st), "moe_align launch")) return rc;
+  ss::ResidentPlan q{};
+  q.ids = expert_ids;
+  q.map = map;
+  q.map_base = (int64_t)layer * E;
+  q.map_len = map_len;
+  q.slot_ptr = slot_ptr;
+  q.n_slots = n_slots;
+  q.R = R;
+  q.E = E;
+  q.local = reinterpret_cast<int32_t*>(ws + w.local);
+  q.sorted_rows = reinterpret_cast<int32_t*>(ws + w.sorted);
+  q.block_expert = reinterpret_cast<int32_t*>(ws + w.bexp);
+  q.order = reinterpret_cast<ss::MBlock*>(ws + w.order);
+  q.num_padded = reinterpret_cast<int32_t*>(ws + w.npad);
+  q.scratch = reinterpret_cast<int32_t*>(ws + w.scratch);
+  q.err = err;
+  if (int rc = hip_check(ss::launch_resident_plan(q, st), "prefill plan launch")) return rc;
   ss::PrefillArgs p{};
   p.x = x;
-  p.row_token = row_token;
   p.row_weight = weights;
-  p.sorted_rows = sorted;
-  p.block_expert = bexp;
-  p.num_padded = npad;
-  p.group_ptr = gptr;
+  p.sorted_rows = q.sorted_rows;
+  p.block_expert = q.block_expert;
+  p.num_padded = q.num_padded;
+  p.order = q.order;
+  p.topk = K;
   p.num_local = E;
   p.h_buf = h_buf;
   p.out_rows = out_rows;
@@ -838,7 +833,7 @@ int ssmoe_moe_prefill(const uint16_t* x, const int32_t* expert_ids, const float*
   p.I = I;
   p.trace = g_trace;
   if (int rc = hip_check(ss::launch_prefill_gemm(p, st), "prefill gemm launch")) return rc;
-  return hip_check(ss::launch_combine(out_rows, local, (int)T, K, H, out, st), "combine launch");
+  return hip_check(ss::launch_combine(out_rows, q.local, (int)T, K, H, out, st), "combine launch");
 }
 
 // ---------------------------------------------------------------- shared expert (prefill)

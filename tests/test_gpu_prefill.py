@@ -33,6 +33,20 @@ def test_moe_align_matches_oracle(R, nl, bm, seed):
     assert np.array_equal(b.cpu().numpy(), rb)
 
 
+@pytest.mark.parametrize("R,nl,bm", [(1024, 1024, 64), (1025, 1024, 64), (1024, 1025, 8), (5000, 4096, 16), (2049, 3, 128)])
+def test_moe_align_one_and_three_launches(R, nl, bm):
+    """Up to 1024 rows and experts the plan is one workgroup, past that three launches over 1024-row chunks."""
+    print(f"[align] R={R} nl={nl} bm={bm}", flush=True)
+    rng = np.random.default_rng(R + nl)
+    le = np.minimum(rng.zipf(1.2, size=R) - 2, nl).astype(np.int32)  # -1 and nl: skipped
+    s, b, n = moe_align(torch.from_numpy(le).cuda(), nl, bm)
+    torch.cuda.synchronize()
+    rs, rb, rn = O.moe_align(le, nl, bm)
+    assert int(n.item()) == rn
+    assert np.array_equal(s.cpu().numpy(), rs)
+    assert np.array_equal(b.cpu().numpy(), rb)
+
+
 def _prefill_case(T, K, E, H, I, seed):
     pool = make_pool(E, H, I, seed=seed)
     x = normal_bf16((T, H), 1.0, seed + 1)
@@ -156,6 +170,27 @@ def test_combine_rank_order_bitwise():
     out = combine_rank_order(rows, T, K)
     torch.cuda.synchronize()
     assert np.array_equal(out.cpu().numpy(), O.combine_rank_order(rows.cpu().numpy(), T, K))
+
+
+@pytest.mark.parametrize("T", [9, 700])
+def test_prefill_skipped_rows_in_both_plans(T):
+    """Ids out of range and experts that are not resident are skipped (+0 in the sum) and flagged, in the one-workgroup
+    plan and in the chunked one."""
+    K, E, H, I = 2, 8, 256, 128
+    pool, x, ids, w = _prefill_case(T, K, E, H, I, 13)
+    pool.map[5] = -1
+    lw = LayerWeights(H, E, 64, seed=2)
+    layer = MoEPrefillLayer(pool, 0, lw.router_w, lw.sh_gate, lw.sh_up, lw.sh_down, lw.sh_g, top_k=K, max_tokens=T)
+    ids = ids.clone()
+    ids[2, 1], ids[T - 1, 0] = -3, E
+    _lib.device_error()
+    routed = layer.routed_experts(x, ids, w)
+    torch.cuda.synchronize()
+    assert _lib.device_error() & 3 == 3
+    flat = ids.cpu().numpy().reshape(-1)
+    ok = (flat >= 0) & (flat < E) & (flat != 5)
+    _, rows_ref = _oracle_rows(pool, x, torch.from_numpy(np.where(ok, flat, -1).reshape(T, K)), w)
+    assert O.rel_l2(routed.cpu().numpy(), O.combine_rank_order(rows_ref, T, K)) < 2e-3
 
 
 def test_prefill_unmapped_expert_flagged():
