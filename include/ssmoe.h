@@ -290,6 +290,23 @@ int ssmoe_moe_prefill(const uint16_t* x, const int32_t* expert_ids, const float*
                       int64_t workspace_bytes, uint16_t* h_buf, float* out_rows, float* out, int64_t T, int H, int I,
                       int K, int E, void* stream);
 
+/* Bytes of the scratch ssmoe_moe_prefill_layer needs (its contents need not survive the call). */
+int64_t ssmoe_moe_prefill_layer_scratch_bytes(int64_t T, int H, int Is, int E);
+
+/* One whole MoE layer over T >= 1 prompt tokens (SweepMoE.layer with the router and the shared expert around it,
+ * model/moe_sweep.py:80-160, model/layers.py:336-348, 398-402): ssmoe_dense_gemm of the router, ssmoe_router_topk,
+ * ssmoe_moe_prefill, the shared expert (ssmoe_dense_gemm, ssmoe_shared_hs, ssmoe_dense_gemm) and
+ * ssmoe_combine_shared, with their bits, in fewer launches. sh_cat bf16 [2 Is + 1 or more, H]: gate rows, up rows, the
+ * shared_expert_gate row; sh_down bf16 [H, Is]; workspace as ssmoe_moe_prefill, scratch 256-byte aligned. Writes ids
+ * int32 [T, K], weights fp32 [T, K], routed fp32 [T, H] and y bf16 [T, H] (and h_buf, out_rows). H and Is multiples of
+ * 256, E a multiple of 8, K <= 16. */
+int ssmoe_moe_prefill_layer(const uint16_t* x, const uint16_t* router_w, const float* router_bias,
+                            const uint16_t* sh_cat, const uint16_t* sh_down, int layer, const int32_t* map,
+                            int64_t map_len, const int64_t* slot_ptr, int64_t n_slots, void* workspace,
+                            int64_t workspace_bytes, void* scratch, int64_t scratch_bytes, uint16_t* h_buf,
+                            float* out_rows, int32_t* ids, float* weights, float* routed, uint16_t* y, int64_t T, int H,
+                            int I, int Is, int K, int E, void* stream);
+
 /* ---------------------------------------------------------------- reference sampler */
 
 /* Bytes of the workspace ssmoe_sample needs for a V-token row (-1 outside 1 <= V <= 1,048,576). */

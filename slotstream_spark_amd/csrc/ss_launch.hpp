@@ -39,6 +39,12 @@ hipError_t launch_dense_rows(const uint16_t* x, int T, int H, const DenseSeg* se
 // Dense bf16 GEMM c = bf16(a b^T) with MFMA fp32 accumulation (ss_gemm.hip): a [M][lda], b [N][ldb], c [M][ldc].
 hipError_t launch_dense_gemm(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, uint16_t* c, int64_t ldc,
                              int M, int N, int K, hipStream_t st);
+// The input projections of a prompt layer in one launch, with the accumulation order of launch_dense_gemm: logits
+// bf16(x router_w^T) [T, E], hs = bf16(bf16(silu(g)) * u) [T, Is] of the shared gate and up rows, and the
+// shared_expert_gate logit sgl [T]. sh_cat [2 Is + 1 or more][H]: gate rows, up rows, the shared_expert_gate row.
+// Is a multiple of 64, E and H as launch_dense_gemm's N and K.
+hipError_t launch_layer_gemm(const uint16_t* x, const uint16_t* router_w, const uint16_t* sh_cat, uint16_t* logits,
+                             uint16_t* hs, uint16_t* sgl, int T, int H, int E, int Is, hipStream_t st);
 
 // Router tail for T tokens: scores = bf16 logits (+ bias), fp32 softmax, top-k (ties -> lower index,
 // sorted by value desc), renormalised weights. probs may be null.
@@ -190,6 +196,9 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st);
 // out[t] = sum over k (in order) of rows[t * K + k]; a row whose row_local entry is negative counts as +0.
 hipError_t launch_combine(const float* rows, const int32_t* row_local, int T, int K, int H, float* out,
                           hipStream_t st);
+// launch_combine and launch_combine_shared in one pass: out and y from the same sums.
+hipError_t launch_combine_layer(const float* rows, const int32_t* row_local, const uint16_t* sh, const uint16_t* sgl,
+                                int T, int K, int H, float* out, uint16_t* y, hipStream_t st);
 
 // Reference sampler (ss_sampler.hip): Sampler.next over one row with sanitized parameters; u a device float.
 int64_t sample_workspace_bytes(int V);

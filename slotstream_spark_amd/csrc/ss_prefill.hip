@@ -803,14 +803,25 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------- combine_rank_order (fused_moe_affine.py:164-172)
+// With LAYER also y = bf16(bf16(out) + bf16(bf16(sigmoid(sgl)) * sh)), the roundings of combine_shared_kernel, so the
+// sums are not read back (at 8192 tokens the two launches took 162 + 21 us). Bound by HBM: T K H 4 bytes in.
+template <bool LAYER>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ rows,
-                                                      const int32_t* __restrict__ row_local, int T, int K, int H,
-                                                      float* __restrict__ out) {
+                                                      const int32_t* __restrict__ row_local,
+                                                      const uint16_t* __restrict__ sh,
+                                                      const uint16_t* __restrict__ sgl, int T, int K, int H,
+                                                      float* __restrict__ out, uint16_t* __restrict__ y) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // one float4 of one token
   const int h4 = H >> 2;
   if (idx >= (int64_t)T * h4) return;
   const int64_t t = idx / h4, c = idx - t * h4;
   const float4* p = reinterpret_cast<const float4*>(rows) + (t * K) * h4 + c;
+  uint2 s2 = make_uint2(0u, 0u);
+  float gl = 0.f;
+  if (LAYER) {
+    s2 = reinterpret_cast<const uint2*>(sh)[idx];
+    gl = ss_bf16_to_f32(sgl[t]);
+  }
   // Every row is loaded (in bounds) and a skipped row's value replaced by +0 afterwards: a select between a local
   // zero and a loaded value is kept on values, never turned into a load through a selected address.
   float4 acc = p[0];
@@ -824,14 +835,33 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
     acc.w = acc.w + (skip ? 0.f : v.w);
   }
   reinterpret_cast<float4*>(out)[idx] = acc;
+  if (LAYER) {
+    const float sg = ss_round_bf16(1.f / (1.f + ss_expf(-gl)));
+    const float rv[4] = {acc.x, acc.y, acc.z, acc.w};
+    const uint32_t sv[4] = {s2.x & 0xFFFFu, s2.x >> 16, s2.y & 0xFFFFu, s2.y >> 16};
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = ss_f32_to_bf16(ss_round_bf16(rv[e]) + ss_round_bf16(sg * ss_bf16_to_f32(sv[e])));
+    reinterpret_cast<uint2*>(y)[idx] = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+  }
 }
 
 hipError_t launch_combine(const float* rows, const int32_t* row_local, int T, int K, int H, float* out,
                           hipStream_t st) {
   const int64_t n = (int64_t)T * (H / 4);
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rows, row_local, T, K, H,
-                     out);
+  hipLaunchKernelGGL(combine_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rows, row_local,
+                     nullptr, nullptr, T, K, H, out, nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_combine_layer(const float* rows, const int32_t* row_local, const uint16_t* sh, const uint16_t* sgl,
+                                int T, int K, int H, float* out, uint16_t* y, hipStream_t st) {
+  const int64_t n = (int64_t)T * (H / 4);
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(combine_kernel<true>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rows, row_local, sh, sgl,
+                     T, K, H, out, y);
   return hipGetLastError();
 }
 

@@ -775,10 +775,11 @@ int64_t ssmoe_moe_prefill_workspace_bytes(int64_t T, int K, int E) {
   return prefill_ws(T, K, E).total;
 }
 
-int ssmoe_moe_prefill(const uint16_t* x, const int32_t* expert_ids, const float* weights, int layer,
-                      const int32_t* map, int64_t map_len, const int64_t* slot_ptr, int64_t n_slots, void* workspace,
-                      int64_t workspace_bytes, uint16_t* h_buf, float* out_rows, float* out, int64_t T, int H, int I,
-                      int K, int E, void* stream) {
+// The routed rows of a prompt chunk into out_rows; *local receives the rows' local experts for the combine.
+static int prefill_rows_impl(const uint16_t* x, const int32_t* expert_ids, const float* weights, int layer,
+                             const int32_t* map, int64_t map_len, const int64_t* slot_ptr, int64_t n_slots,
+                             void* workspace, int64_t workspace_bytes, uint16_t* h_buf, float* out_rows, float* out,
+                             int64_t T, int H, int I, int K, int E, void* stream, const int32_t** local) {
   if (T < 0 || K < 1 || K > 64 || E < 1 || E > 4096) return fail(SSMOE_EINVAL, "need T >= 0, 1 <= K <= 64, 1 <= E <= 4096");
   if (int rc = check_prefill_shape(T * K, H, I)) return rc;
   if (layer < 0) return fail(SSMOE_EINVAL, "layer must be >= 0, got %d", layer);
@@ -832,8 +833,80 @@ int ssmoe_moe_prefill(const uint16_t* x, const int32_t* expert_ids, const float*
   p.H = H;
   p.I = I;
   p.trace = g_trace;
-  if (int rc = hip_check(ss::launch_prefill_gemm(p, st), "prefill gemm launch")) return rc;
-  return hip_check(ss::launch_combine(out_rows, q.local, (int)T, K, H, out, st), "combine launch");
+  *local = q.local;
+  return hip_check(ss::launch_prefill_gemm(p, st), "prefill gemm launch");
+}
+
+int ssmoe_moe_prefill(const uint16_t* x, const int32_t* expert_ids, const float* weights, int layer,
+                      const int32_t* map, int64_t map_len, const int64_t* slot_ptr, int64_t n_slots, void* workspace,
+                      int64_t workspace_bytes, uint16_t* h_buf, float* out_rows, float* out, int64_t T, int H, int I,
+                      int K, int E, void* stream) {
+  const int32_t* local = nullptr;
+  if (int rc = prefill_rows_impl(x, expert_ids, weights, layer, map, map_len, slot_ptr, n_slots, workspace,
+                                 workspace_bytes, h_buf, out_rows, out, T, H, I, K, E, stream, &local))
+    return rc;
+  if (T == 0) return ok();
+  return hip_check(ss::launch_combine(out_rows, local, (int)T, K, H, out, static_cast<hipStream_t>(stream)),
+                   "combine launch");
+}
+
+// Scratch of ssmoe_moe_prefill_layer: logits [T, E], hs [T, Is], sh [T, H], sgl [T], all bf16.
+struct LayerScratch {
+  int64_t hs, sh, sgl, total;
+};
+static LayerScratch layer_scratch(int64_t T, int H, int Is, int E) {
+  auto up = [](int64_t v) { return (v + 255) / 256 * 256; };
+  LayerScratch s{};
+  s.hs = up(T * E * 2);
+  s.sh = s.hs + up(T * Is * 2);
+  s.sgl = s.sh + up(T * H * 2);
+  s.total = s.sgl + up(T * 2);
+  return s;
+}
+
+int64_t ssmoe_moe_prefill_layer_scratch_bytes(int64_t T, int H, int Is, int E) {
+  if (T < 0 || H < 1 || Is < 1 || E < 1) return -1;
+  return layer_scratch(T, H, Is, E).total;
+}
+
+int ssmoe_moe_prefill_layer(const uint16_t* x, const uint16_t* router_w, const float* router_bias,
+                            const uint16_t* sh_cat, const uint16_t* sh_down, int layer, const int32_t* map,
+                            int64_t map_len, const int64_t* slot_ptr, int64_t n_slots, void* workspace,
+                            int64_t workspace_bytes, void* scratch, int64_t scratch_bytes, uint16_t* h_buf,
+                            float* out_rows, int32_t* ids, float* weights, float* routed, uint16_t* y, int64_t T, int H,
+                            int I, int Is, int K, int E, void* stream) {
+  if (T < 1 || T > (1 << 30)) return fail(SSMOE_EINVAL, "T must be in [1, 2^30], got %lld", (long long)T);
+  if (E < 8 || E % 8 || E > 4096 || K < 1 || K > 16 || K > E)
+    return fail(SSMOE_EINVAL, "need E a multiple of 8 in [8, 4096] and 1 <= K <= min(16, E), got E=%d K=%d", E, K);
+  if (H < 256 || H % 256 || Is < 256 || Is % 256)
+    return fail(SSMOE_EINVAL, "need H and Is positive multiples of 256, got H=%d Is=%d", H, Is);
+  if (!x || !router_w || !sh_cat || !sh_down || !scratch || !ids || !weights || !routed || !y)
+    return fail(SSMOE_EINVAL, "every pointer except router_bias must be non-null");
+  if (!aligned(x, 16) || !aligned(router_w, 16) || !aligned(sh_cat, 16) || !aligned(sh_down, 16) || !aligned(y, 16) ||
+      !aligned(scratch, 256))
+    return fail(SSMOE_EINVAL, "x, weights and y must be 16-byte, scratch 256-byte aligned");
+  const LayerScratch s = layer_scratch(T, H, Is, E);
+  if (scratch_bytes < s.total)
+    return fail(SSMOE_EINVAL, "scratch holds %lld bytes, need %lld", (long long)scratch_bytes, (long long)s.total);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  uint8_t* sb = static_cast<uint8_t*>(scratch);
+  uint16_t* logits = reinterpret_cast<uint16_t*>(sb);
+  uint16_t* hs = reinterpret_cast<uint16_t*>(sb + s.hs);
+  uint16_t* sh = reinterpret_cast<uint16_t*>(sb + s.sh);
+  uint16_t* sgl = reinterpret_cast<uint16_t*>(sb + s.sgl);
+  if (int rc = hip_check(ss::launch_layer_gemm(x, router_w, sh_cat, logits, hs, sgl, (int)T, H, E, Is, st),
+                         "prefill projections launch"))
+    return rc;
+  if (int rc = hip_check(ss::launch_router_topk(logits, router_bias, nullptr, ids, weights, (int)T, E, K, st),
+                         "router top-k launch"))
+    return rc;
+  const int32_t* local = nullptr;
+  if (int rc = prefill_rows_impl(x, ids, weights, layer, map, map_len, slot_ptr, n_slots, workspace, workspace_bytes,
+                                 h_buf, out_rows, routed, T, H, I, K, E, stream, &local))
+    return rc;
+  if (int rc = hip_check(ss::launch_dense_gemm(hs, Is, sh_down, Is, sh, H, (int)T, H, Is, st), "shared down launch"))
+    return rc;
+  return hip_check(ss::launch_combine_layer(out_rows, local, sh, sgl, (int)T, K, H, routed, y, st), "combine launch");
 }
 
 // ---------------------------------------------------------------- shared expert (prefill)

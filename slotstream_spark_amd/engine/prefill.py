@@ -8,7 +8,9 @@ The dense projections run on libssmoe's bf16 MFMA GEMM (ssmoe_dense_gemm, lin's 
 the router, one GEMM for the shared expert's gate, up and shared_expert_gate rows together (their weights
 concatenated once at construction), and the shared down projection. The routed experts, the routing, the shared
 expert's elementwise chain (ssmoe_shared_hs) and the final y (ssmoe_combine_shared) run in libssmoe as well, with the
-reference's bf16 rounding of every op; torch only allocates.
+reference's bf16 rounding of every op; torch only allocates. A call of the layer is one C call (ssmoe_moe_prefill_layer:
+the input projections in one launch with the elementwise chain behind them, the combine and y in one pass) with the
+bits of the separate methods.
 """
 from __future__ import annotations
 
@@ -83,11 +85,16 @@ class MoEPrefillLayer:
             raise ValueError(f"x must be a contiguous bf16 [T, {self.hidden}] tensor")
         if x.shape[0] > self.max_tokens:
             raise ValueError(f"at most {self.max_tokens} tokens per call, got {x.shape[0]}")
-        t = x.shape[0]
-        ids, w = self.route(x)
-        routed = self.routed_experts(x, ids, w)
-        sh, sgl = self.shared(x)
-        y = torch.empty((t, self.hidden), dtype=torch.bfloat16, device=x.device)
-        _lib.check(_lib.lib().ssmoe_combine_shared(routed.data_ptr(), sh.data_ptr(), sgl.data_ptr(), y.data_ptr(), t,
-                                                   self.hidden, _lib.stream_of(x)))
+        t, H, Is, dev = x.shape[0], self.hidden, self.shared_inter, x.device
+        L, p = _lib.lib(), self.pool
+        ids, w, routed = self.ids[:t], self.weights[:t], self.routed[:t]
+        y = torch.empty((t, H), dtype=torch.bfloat16, device=dev)
+        scratch = torch.empty(max(int(L.ssmoe_moe_prefill_layer_scratch_bytes(t, H, Is, self.experts)), 1),
+                              dtype=torch.uint8, device=dev)
+        _lib.check(L.ssmoe_moe_prefill_layer(
+            x.data_ptr(), self.router_w.data_ptr(), _lib.ptr(self.router_bias), self.sh_cat.data_ptr(),
+            self.sh_down.data_ptr(), self.layer, p.map.data_ptr(), p.map.numel(), p.slot_ptr.data_ptr(),
+            p.slot_ptr.numel(), self.workspace.data_ptr(), self.workspace.numel(), scratch.data_ptr(), scratch.numel(),
+            self.h_buf.data_ptr(), self.out_rows.data_ptr(), ids.data_ptr(), w.data_ptr(), routed.data_ptr(),
+            y.data_ptr(), t, H, self.inter, Is, self.top_k, self.experts, _lib.stream_of(x)))
         return y, ids, w, routed

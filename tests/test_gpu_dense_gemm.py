@@ -98,3 +98,16 @@ def test_prefill_router_against_reference_cpu_router():
           f"{n_rows} of {T} rows select otherwise, each at a tie within that difference")
     assert diff_logits <= 2e-3 * mine.size
     assert n_rows == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(2100, 1544, 256), (1700, 1800, 512)])
+def test_dense_gemm_same_bits_for_every_tile(M, N, K):
+    """The three tile shapes (by the number of tiles) accumulate in one order: rows computed alone, over few columns or
+    many, are the rows of the large call, bit for bit, ragged edges included."""
+    x, w = normal_bf16((M, K), 1.0, M), normal_bf16((N, K), 0.02, N)
+    full = gemm_bf16(x, w)
+    for m0, m1, n0, n1 in ((0, 33, 0, N), (M - 40, M, 0, 520), (100, 700, 8, N), (M - 1, M, N - 24, N)):
+        part = gemm_bf16(x[m0:m1].contiguous(), w[n0:n1].contiguous())
+        assert torch.equal(part, full[m0:m1, n0:n1])
+    ref = x[:50].float() @ w.float().T
+    assert float((full[:50].float() - ref).norm() / ref.norm()) < 4e-3  # one bf16 rounding (2^-9 at most)

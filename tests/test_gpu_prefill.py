@@ -240,6 +240,29 @@ def test_prefill_layer_end_to_end():
     assert torch.isfinite(y.float()).all()
 
 
+@pytest.mark.parametrize("T,E,H,Is", [(1, 8, 256, 256), (33, 64, 512, 256), (70, 520, 2048, 512), (300, 64, 256, 768),
+                                      (1100, 512, 512, 512)])
+def test_prefill_layer_equals_its_parts(T, E, H, Is):
+    """The layer in one C call (the three dense tile shapes, ragged T and router columns) against the separate calls,
+    bit for bit."""
+    K, I = 4, 128
+    pool = make_pool(E, H, I, seed=T)
+    lw = LayerWeights(H, E, Is, seed=T + 1)
+    layer = MoEPrefillLayer(pool, 0, lw.router_w, lw.sh_gate, lw.sh_up, lw.sh_down, lw.sh_g, top_k=K,
+                            router_bias=zipf_bias(E, 1.1, 3), max_tokens=T)
+    x = normal_bf16((T, H), 1.0, T + 2)
+    ids, w = (t.clone() for t in layer.route(x))
+    routed = layer.routed_experts(x, ids, w).clone()
+    sh, sgl = layer.shared(x)
+    y = torch.empty((T, H), dtype=torch.bfloat16, device="cuda")
+    _lib.check(_lib.lib().ssmoe_combine_shared(routed.data_ptr(), sh.data_ptr(), sgl.data_ptr(), y.data_ptr(), T, H,
+                                               torch.cuda.current_stream().cuda_stream))
+    got = layer(x)
+    torch.cuda.synchronize()
+    for g, ref in zip(got, (y, ids, w, routed)):
+        assert torch.equal(g, ref)
+
+
 @pytest.mark.parametrize("T,Is,ld", [(1, 8, 17), (37, 512, 1032), (300, 640, 1288)])
 def test_shared_hs_bitwise(T, Is, ld):
     g = torch.Generator(device="cuda").manual_seed(T)
