@@ -21,7 +21,8 @@
 // (engine/generate.py:208-229) over D+1 rows: row i is reached only if rows 0..i-1 drew their drafts, so its
 // penalty set is seen + drafts[0..i) and all rows are drawn together; a last one-wave kernel walks the rows in
 // order (a non-finite row ends the round without a draw, :210-212; the round goes on while the token equals the
-// draft). The launch sequence depends only on the parameters, so it can be captured in a graph.
+// draft). The launch sequence depends only on the parameters, so it can be captured in a graph: three launches for
+// rows with a top-k of at most 512 (below), one launch per step otherwise.
 #include "ss_common.hpp"
 #include "ss_launch.hpp"
 
@@ -35,7 +36,7 @@ constexpr int kPerLane = 16;  // chunk arrays of up to 1024 chunks (V <= 2^20)
 constexpr int kRhoBits = 52;  // 32 key bits above 20 index bits
 constexpr int kRounds = kRhoBits / 4;
 constexpr int kFlagNonfinite = 1, kFlagBadDraft = 2, kFlagFallback = 8;
-constexpr int kSlot = 512;  // nonzero exp entries a top-k chunk lists for the compact top-p search
+constexpr int kSlot = 512;  // candidates a chunk of a top-k row lists
 constexpr int kHistShards = 8;  // copies of each top-k histogram; chunk c adds to copy c % 8 (fewer atomics per bin)
 
 SS_DEV bool is_nan(float v) { return v != v; }
@@ -53,7 +54,7 @@ SS_DEV uint64_t amax_key(float v, int j) { return ((uint64_t)nkey(v) << 32) | (0
 
 // Byte offsets of one row's workspace; rows follow each other `bytes` apart.
 struct Layout {
-  size_t L, P, cmax, cnan, ckey, craw, cbad, etot, ftot, tsum, stot, hist, rr, res, cnz, surv, cres, bytes;
+  size_t L, P, cmax, cnan, ckey, craw, cbad, etot, ftot, tsum, stot, hist, rr, res, cnz, cand, gkey, done, bytes;
 };
 
 __host__ __device__ inline Layout layout_of(int V, int nch) {
@@ -78,9 +79,10 @@ __host__ __device__ inline Layout layout_of(int V, int nch) {
   l.hist = take(4 * kHistShards * 256 * 4);  // top-k radix histograms, one per 8-bit pass, kHistShards copies
   l.rr = take((size_t)(kRounds + 1) * 8);   // top-p prefix at the start of each round
   l.res = take(16);                         // token, fallback flag, non-finite row
-  l.cnz = take((size_t)nch * 4);            // nonzero exp entries per chunk (top-k rows)
-  l.surv = take((size_t)nch * kSlot * 8);   // a chunk's nonzero entries (index << 32 | e bits), up to kSlot
-  l.cres = take(16);                        // compact top-p: r* (uint64), then 1 when it was found
+  l.cnz = take((size_t)nch * 4);            // candidates per chunk (top-k rows)
+  l.cand = take((size_t)nch * kSlot * 8);   // a chunk's candidates (index << 32 | logit bits), up to kSlot
+  l.gkey = take((size_t)nch * 16 * 4);      // largest key of each group of the row (top-k rows)
+  l.done = take(4);                         // accept mode: rows drawn (row 0's word)
   l.bytes = o;
   return l;
 }
@@ -95,8 +97,9 @@ struct SW {
   uint64_t* rr;
   int* res;
   int* cnz;
-  uint64_t* surv;
-  uint64_t* cres;  // [0] r*, [1] found (1) or not (0)
+  uint64_t* cand;
+  uint32_t* gkey;
+  int* done;
 };
 
 SS_DEV SW sw_of(void* work, int V, int nch, int row) {
@@ -118,8 +121,9 @@ SS_DEV SW sw_of(void* work, int V, int nch, int row) {
   s.rr = reinterpret_cast<uint64_t*>(b + l.rr);
   s.res = reinterpret_cast<int*>(b + l.res);
   s.cnz = reinterpret_cast<int*>(b + l.cnz);
-  s.surv = reinterpret_cast<uint64_t*>(b + l.surv);
-  s.cres = reinterpret_cast<uint64_t*>(b + l.cres);
+  s.cand = reinterpret_cast<uint64_t*>(b + l.cand);
+  s.gkey = reinterpret_cast<uint32_t*>(b + l.gkey);
+  s.done = reinterpret_cast<int*>(b + l.done);
   return s;
 }
 
@@ -236,11 +240,12 @@ SS_DEV float row_max(const SW& w, int nch) {
 
 // One 8-bit radix step of the top-k select, whole wave: the bin of the need-th largest key among those counted in
 // `hist` (bins descending, counting multiplicity); need becomes its rank inside the bin. Every lane gets the same.
+template <int SH = kHistShards>
 SS_DEV void select_pass(const int* hist, int& need, uint32_t& prefix, int shift) {
   const int lane = threadIdx.x & 63;
-  int hs[kHistShards][4];
+  int hs[SH][4];
 #pragma unroll
-  for (int c = 0; c < kHistShards; ++c)
+  for (int c = 0; c < SH; ++c)
 #pragma unroll
     for (int q = 0; q < 4; ++q) hs[c][q] = hist[256 * c + 255 - 4 * lane - q];
   int h[4], s = 0;
@@ -248,7 +253,7 @@ SS_DEV void select_pass(const int* hist, int& need, uint32_t& prefix, int shift)
   for (int q = 0; q < 4; ++q) {
     h[q] = 0;
 #pragma unroll
-    for (int c = 0; c < kHistShards; ++c) h[q] += hs[c][q];
+    for (int c = 0; c < SH; ++c) h[q] += hs[c][q];
     s += h[q];
   }
   int incl = s;  // inclusive prefix over lanes = count of keys in bins >= 252 - 4 * lane
@@ -431,245 +436,14 @@ __global__ __launch_bounds__(64) void samp_exp_kernel(SampArgs a, int has_k) {
   }
   float sub;
   const float t = chunk_sum(v, sub);
-  if (has_k) {
-    // the chunk's nonzero entries in index order (lane-major: entry lane * 16 + i), up to kSlot of them
-    int nz = 0;
-#pragma unroll
-    for (int i = 0; i < kSub; ++i) nz += v[i] != 0.f;
-    int incl = nz;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int o = __shfl_up(incl, d);
-      incl += lane >= d ? o : 0;
-    }
-    int pos = incl - nz;
-#pragma unroll
-    for (int i = 0; i < kSub; ++i) {
-      if (v[i] != 0.f) {
-        if (pos < kSlot) {
-          const uint32_t j = (uint32_t)(c * kChunk + lane * kSub + i);
-          w.surv[(size_t)c * kSlot + pos] = ((uint64_t)j << 32) | __float_as_uint(v[i]);
-        }
-        ++pos;
-      }
-    }
-    if (lane == 63) w.cnz[c] = incl;
-  }
   if (lane == 0) w.etot[c] = t;
-}
-
-// 4'. Compact top-p (top-k rows, one workgroup per row). Only the top-k survivors carry weight, so cum(r) (the
-// hierarchical mass of p over rho > r) is a step function of the survivors: with S(m) the masked hierarchical sum of
-// the m survivors of largest rho (S grows with m: every partial sum is a monotone function of nonnegative terms),
-// the smallest r with cum(r) < top_p is the rho of the m'-th survivor, m' the smallest m with S(m) >= top_p, or 0
-// when S(all) < top_p: exactly the r* the 13 radix rounds find. S(m) is formed as the rounds form their masses:
-// per chunk, lane b sums sub-chunk b's included entries in index order, the wave butterfly gives the chunk total,
-// the chunk totals are summed in order. Four waves evaluate four values of m at a time. Rows with more than
-// kCompact survivors, or a non-finite z, leave cres[1] = 0 and the rounds run as before.
-constexpr int kCompact = 512;
-constexpr int kCompactChunks = 160;  // active chunks the compact search holds (more: the rounds run)
-
-__global__ __launch_bounds__(256) void samp_topp_compact_kernel(SampArgs a) {
-  __shared__ int s_cnt[kPerLane * 64];   // nonzero count of active chunk q, then its chunk index
-  __shared__ int s_ach[kPerLane * 64];
-  __shared__ int s_aoff[kPerLane * 64 + 1];
-  __shared__ int s_j[kCompact], s_rank[kCompact];
-  __shared__ float s_p[kCompact];
-  __shared__ uint64_t s_rho[kCompact];
-  __shared__ int s_na, s_ok, s_digit;
-  __shared__ __attribute__((aligned(16))) float s_leaf[kCompactChunks * 64];  // leaves; the fallback's masses
-  __shared__ __attribute__((aligned(16))) float s_ct[kCompactChunks];
-  __shared__ float s_S;
-  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  SW sw = sw_of(a.work, a.V, a.nch, row);
-  const int nch = a.nch;
-  // wave 0: the active chunks (nonzero count) in order, their survivor offsets, and whether every count fits
-  if (w == 0) {
-    int run = 0, na = 0, ok = 1;
-    int cv[kPerLane];
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) cv[k] = lane + 64 * k < nch ? sw.cnz[lane + 64 * k] : 0;
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-      const int v = cv[k];
-      ok &= v <= kSlot;
-      const uint64_t act = __ballot(v > 0);
-      const int before = __popcll(act & ((1ull << lane) - 1ull));
-      int incl = v;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(incl, d);
-        incl += lane >= d ? o : 0;
-      }
-      if (v > 0) {
-        s_ach[na + before] = lane + 64 * k;
-        s_aoff[na + before] = run + incl - v;
-        s_cnt[na + before] = v;
-      }
-      run += __shfl(incl, 63);
-      na += __popcll(act);
-    }
-    ok = ss_wave_or((uint32_t)!ok) ? 0 : 1;
-    if (lane == 0) {
-      s_aoff[na] = run;
-      s_na = na;
-      s_ok = ok && run <= kCompact && na <= kCompactChunks;
-    }
-  }
-  __syncthreads();
-  const int na = s_na;
-  const int n = s_aoff[na];
-  const float z = seq_sum(sw.etot, nch);  // the z round 0 would form
-  if (!s_ok || !(z > 0.f) || !(z < __builtin_inff())) {
-    // The 13 radix rounds of samp_topp_kernel inside the workgroup (same masses, digits and order; p = e / z formed
-    // as round 0 forms it, P keeps e): r* = the digits at shifts 48, 44, ..., 0. Four waves take the chunks.
-    float* tsl = s_leaf;  // [16][nch], nch <= 640
-    uint64_t r = 0;
-    for (int round = 0; round < kRounds; ++round) {
-      const int sft = kRhoBits - 4 - 4 * round;
-      const uint64_t r_hi = r >> (sft + 4);
-      for (int c = w; c < nch; c += 4) {
-        float pv[kSub];
-#pragma unroll
-        for (int i = 0; i < kSub; ++i) {
-          const int j = c * kChunk + lane * kSub + i;
-          pv[i] = j < a.V ? sw.P[j] / z : 0.f;
-        }
-        float acc[16];
-#pragma unroll
-        for (int d = 0; d < 16; ++d) acc[d] = 0.f;
-#pragma unroll
-        for (int i = 0; i < kSub; ++i) {
-          const int j = c * kChunk + lane * kSub + i;
-          const float pp = pv[i];
-          if (j < a.V && pp != 0.f) {
-            const uint64_t rho = rho_of(pp, j);
-            const uint64_t hi = rho >> (sft + 4);
-            const int lim = hi > r_hi ? 16 : (hi == r_hi ? (int)((rho >> sft) & 15) : 0);
-#pragma unroll
-            for (int d = 0; d < 16; ++d) acc[d] = acc[d] + (d < lim ? pp : 0.f);
-          }
-        }
-#pragma unroll
-        for (int d = 0; d < 16; ++d) {
-          const float t = ss_wave_sum(acc[d]);
-          if (lane == 0) tsl[d * nch + c] = t;
-        }
-      }
-      __syncthreads();
-      if (w == 0) {
-        float cum = 0.f;
-        for (int c = 0; c < nch; ++c) cum = cum + tsl[(lane & 15) * nch + c];
-        const uint64_t okb = __ballot(lane < 16 && cum < a.top_p);
-        if (lane == 0) s_digit = okb ? (int)__builtin_ctzll(okb) : 15;
-      }
-      __syncthreads();
-      r |= (uint64_t)s_digit << sft;
-    }
-    if (tid == 0) {
-      sw.cres[0] = r;
-      sw.cres[1] = 1;
-    }
-    return;
-  }
-  // gather: survivor q of the row is entry q - aoff[t] of active chunk t (binary search); one batch of loads
-  for (int q = tid; q < n; q += 256) {
-    int lo = 0, hi = na - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (s_aoff[mid] <= q) lo = mid;
-      else hi = mid - 1;
-    }
-    const uint64_t e = sw.surv[(size_t)s_ach[lo] * kSlot + (q - s_aoff[lo])];
-    const int j = (int)(e >> 32);
-    const float pj = __uint_as_float((uint32_t)e) / z;
-    s_j[q] = j;
-    s_p[q] = pj;
-    s_rho[q] = rho_of(pj, j);
-  }
-  __syncthreads();
-  // rank by rho, descending (rho values are distinct: they end in the index)
-  for (int q = tid; q < n; q += 256) {
-    const uint64_t r = s_rho[q];
-    int rk = 0;
-    for (int t = 0; t < n; ++t) rk += s_rho[t] > r;
-    s_rank[q] = rk;
-  }
-  __syncthreads();
-  // S(m) by the workgroup: leaf (active chunk t, sub-chunk b) = its survivors of rank < m summed in index order
-  // (a leaf's survivors are adjacent in the list; its first one sums them), the wave butterfly over each chunk's 64
-  // leaves, then the chunk totals in order. The leaf matrix is kept zero between evaluations.
-  for (int q = tid; q < na * 64; q += 256) s_leaf[q] = 0.f;
-  for (int q = tid; q < n; q += 256) {  // the leaf of survivor q and whether it starts its leaf
-    int lo2 = 0, hi2 = na - 1;
-    while (lo2 < hi2) {
-      const int mid = (lo2 + hi2 + 1) >> 1;
-      if (s_aoff[mid] <= q) lo2 = mid;
-      else hi2 = mid - 1;
-    }
-    const int leaf = lo2 * 64 + ((s_j[q] & (kChunk - 1)) >> 4);
-    const bool first = q == s_aoff[lo2] || ((s_j[q - 1] & (kChunk - 1)) >> 4) != ((s_j[q] & (kChunk - 1)) >> 4);
-    s_cnt[q] = first ? leaf : -1;  // reused: leaf index at a leaf's first survivor, -1 elsewhere
-  }
-  __syncthreads();
-  auto eval = [&](int m) {
-    for (int q = tid; q < n; q += 256) {
-      const int leaf = s_cnt[q];
-      if (leaf >= 0) {
-        float v = 0.f;
-        for (int r = q; r < n && (r == q || s_cnt[r] < 0); ++r) {
-          if (r != q && ((s_j[r] & (kChunk - 1)) >> 4) != ((s_j[q] & (kChunk - 1)) >> 4)) break;
-          const float nx = v + s_p[r];
-          v = s_rank[r] < m ? nx : v;
-        }
-        s_leaf[leaf] = v;
-      }
-    }
-    __syncthreads();
-    for (int t = w; t < na; t += 4) {
-      const float ct = ss_wave_sum(s_leaf[t * 64 + lane]);
-      if (lane == 0) s_ct[t] = ct;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      float S = 0.f;
-      for (int t = 0; t < na; t += 4) {
-        const float4 c4 = *reinterpret_cast<const float4*>(s_ct + t);
-        const float cv[4] = {c4.x, c4.y, c4.z, c4.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float nx = S + cv[e];
-          S = t + e < na ? nx : S;
-        }
-      }
-      s_S = S;
-    }
-    __syncthreads();
-    return s_S;
-  };
-  // smallest m in [0, n] with S(m) >= top_p (n + 1 when none): binary search, S(lo) < top_p <= S(hi)
-  int lo = 0, hi = n + 1;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (eval(mid) >= a.top_p) hi = mid;
-    else lo = mid;
-  }
-  if (tid == 0) {
-    uint64_t rs = 0;
-    if (hi <= n)
-      for (int q = 0; q < n; ++q)
-        if (s_rank[q] == hi - 1) rs = s_rho[q];
-    sw.cres[0] = rs;
-    sw.cres[1] = 1;
-  }
 }
 
 // 4. top-p round k: fold the previous round's digit into the prefix r, then chunk c's hierarchical masses of p over
 // rho > r | d << s | (2^s - 1), d = 0..15. Round 0 also normalizes p = e / z.
-__global__ __launch_bounds__(64) void samp_topp_kernel(SampArgs a, int round, int compact) {
+__global__ __launch_bounds__(64) void samp_topp_kernel(SampArgs a, int round) {
   const int c = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
   SW w = sw_of(a.work, a.V, a.nch, row);
-  if (compact && w.cres[1]) return;  // r* is known
   const int nch = a.nch;
   const int s = kRhoBits - 4 - 4 * round;
   float pv[kSub];
@@ -718,8 +492,7 @@ __global__ __launch_bounds__(64) void samp_topp_kernel(SampArgs a, int round, in
 }
 
 // 5. (has_p) keep rho >= r*; (min_p > 0) chunk maxima of the kept probabilities. `norm`: p = e / z here.
-// With `compact` and r* found by samp_topp_compact_kernel, the rounds did not run: r = r* and P still holds e.
-__global__ __launch_bounds__(64) void samp_keep_kernel(SampArgs a, int has_p, int norm, int compact) {
+__global__ __launch_bounds__(64) void samp_keep_kernel(SampArgs a, int has_p, int norm) {
   const int c = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
   SW w = sw_of(a.work, a.V, a.nch, row);
   const int nch = a.nch;
@@ -730,10 +503,7 @@ __global__ __launch_bounds__(64) void samp_keep_kernel(SampArgs a, int has_p, in
     pv[i] = j < a.V ? w.P[j] : 0.f;
   }
   uint64_t r = 0;
-  if (compact) {
-    r = w.cres[0];
-    norm = 1;
-  } else if (has_p) {
+  if (has_p) {
     r = w.rr[kRounds - 1] | (uint64_t)topp_digit(w.tsum + ((kRounds - 1) & 1) * 16 * nch, nch, a.top_p);
   }
   const float z = norm ? seq_sum(w.etot, nch) : 1.f;
@@ -787,6 +557,79 @@ __global__ __launch_bounds__(64) void samp_total_kernel(SampArgs a, int has_minp
   if (lane == 0) w.ftot[c] = t;
 }
 
+// The inverse-CDF descent over the final weights, whole wave (every lane follows the same scan): chunk totals ct in LDS
+// (zero-padded to a multiple of 16), their sum `total`, sub-chunk totals stot[64 nch], weights P[V] -> the token.
+static SS_DEV int draw_descent(float u, float total, const float* ct, int nch, const float* stot, const float* P, int V) {
+  const int lane = threadIdx.x & 63;
+  const bool ge = u != 0.f;
+  const float target = ge ? u * total : 0.f;
+  auto hit = [&](float x) { return ge ? x >= target : x > target; };
+  // The first chunk whose running total hits the target is the count of leading misses: the zero padding adds +0
+  // and, following a miss with the same total, cannot be the first hit, so no bound check runs per entry.
+  int lead = 0, clast = -1;
+  bool alive = true;
+  float base = 0.f, run = 0.f;
+  const float4* c4 = reinterpret_cast<const float4*>(ct);
+  for (int q0 = 0; q0 < nch; q0 += 16) {  // 16 unconditional reads (the padding is zero), then the in-order scan
+    const float4 a0 = c4[q0 / 4], a1 = c4[q0 / 4 + 1], a2 = c4[q0 / 4 + 2], a3 = c4[q0 / 4 + 3];
+    const float t[16] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w,
+                         a2.x, a2.y, a2.z, a2.w, a3.x, a3.y, a3.z, a3.w};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float nx = run + t[i];
+      alive = alive && !hit(nx);
+      base = alive ? nx : base;
+      lead += alive ? 1 : 0;
+      clast = t[i] > 0.f ? q0 + i : clast;
+      run = nx;
+    }
+  }
+  int cs = lead < nch ? lead : -1;
+  if (cs < 0) {
+    cs = clast < 0 ? 0 : clast;
+    base = lds_seq_sum(ct, cs, 0.f);
+  }
+  const float st = stot[cs * 64 + lane];
+  int slead = 0, blast = -1;
+  float sbase = base;
+  run = base;
+  alive = true;
+#pragma unroll 16
+  for (int b = 0; b < 64; ++b) {
+    const float t = ss_readlane_f(st, b);
+    const float nx = run + t;
+    blast = t > 0.f ? b : blast;
+    alive = alive && !hit(nx);
+    sbase = alive ? nx : sbase;
+    slead += alive ? 1 : 0;
+    run = nx;
+  }
+  int bs = slead < 64 ? slead : -1;
+  if (bs < 0) {
+    bs = blast < 0 ? 0 : blast;
+    sbase = base;
+    for (int b = 0; b < bs; ++b) sbase = sbase + ss_readlane_f(st, b);
+  }
+  const int j0 = cs * kChunk + bs * kSub;
+  const int jl = j0 + (lane & (kSub - 1));
+  const float val = jl < V ? P[jl] : 0.f;
+  int pick = -1, last = -1;
+  run = sbase;
+  for (int i = 0; i < kSub; ++i) {
+    const int j = j0 + i;
+    if (j >= V) break;
+    const float e = ss_readlane_f(val, i);
+    if (e > 0.f) last = j;
+    run = run + e;
+    if (hit(run)) {
+      pick = j;
+      break;
+    }
+  }
+  if (pick < 0) pick = last >= 0 ? last : (j0 < V ? j0 : V - 1);
+  return pick;
+}
+
 // 7. the draw, one wave per row (every lane follows the same scan); greedy rows take the argmax.
 __global__ __launch_bounds__(64) void samp_draw_kernel(SampArgs a) {
   const int row = blockIdx.x, lane = threadIdx.x;
@@ -825,92 +668,179 @@ __global__ __launch_bounds__(64) void samp_draw_kernel(SampArgs a) {
     finish((int)(0xFFFFFFFFu - (uint32_t)k), 1, 0);
     return;
   }
-  const float u = a.u[row];
-  const bool ge = u != 0.f;
-  const float target = ge ? u * total : 0.f;
-  auto hit = [&](float x) { return ge ? x >= target : x > target; };
-  // The first chunk whose running total hits the target is the count of leading misses: the zero padding adds +0
-  // and, following a miss with the same total, cannot be the first hit, so no bound check runs per entry.
-  int lead = 0, clast = -1;
-  bool alive = true;
-  float base = 0.f, run = 0.f;
-  const float4* c4 = reinterpret_cast<const float4*>(ct);
-  for (int q0 = 0; q0 < nch; q0 += 16) {  // 16 unconditional reads (the padding is zero), then the in-order scan
-    const float4 a0 = c4[q0 / 4], a1 = c4[q0 / 4 + 1], a2 = c4[q0 / 4 + 2], a3 = c4[q0 / 4 + 3];
-    const float t[16] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w,
-                         a2.x, a2.y, a2.z, a2.w, a3.x, a3.y, a3.z, a3.w};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float nx = run + t[i];
-      alive = alive && !hit(nx);
-      base = alive ? nx : base;
-      lead += alive ? 1 : 0;
-      clast = t[i] > 0.f ? q0 + i : clast;
-      run = nx;
-    }
-  }
-  int cs = lead < nch ? lead : -1;
-  if (cs < 0) {
-    cs = clast < 0 ? 0 : clast;
-    base = lds_seq_sum(ct, cs, 0.f);
-  }
-  const float st = w.stot[cs * 64 + lane];
-  int slead = 0, blast = -1;
-  float sbase = base;
-  run = base;
-  alive = true;
-#pragma unroll 16
-  for (int b = 0; b < 64; ++b) {
-    const float t = ss_readlane_f(st, b);
-    const float nx = run + t;
-    blast = t > 0.f ? b : blast;
-    alive = alive && !hit(nx);
-    sbase = alive ? nx : sbase;
-    slead += alive ? 1 : 0;
-    run = nx;
-  }
-  int bs = slead < 64 ? slead : -1;
-  if (bs < 0) {
-    bs = blast < 0 ? 0 : blast;
-    sbase = base;
-    for (int b = 0; b < bs; ++b) sbase = sbase + ss_readlane_f(st, b);
-  }
-  const int j0 = cs * kChunk + bs * kSub;
-  const int jl = j0 + (lane & (kSub - 1));
-  const float val = jl < a.V ? w.P[jl] : 0.f;
-  int pick = -1, last = -1;
-  run = sbase;
-  for (int i = 0; i < kSub; ++i) {
-    const int j = j0 + i;
-    if (j >= a.V) break;
-    const float e = ss_readlane_f(val, i);
-    if (e > 0.f) last = j;
-    run = run + e;
-    if (hit(run)) {
-      pick = j;
-      break;
-    }
-  }
-  if (pick < 0) pick = last >= 0 ? last : (j0 < a.V ? j0 : a.V - 1);
-  finish(pick, 0, 0);
+  finish(draw_descent(a.u[row], total, ct, nch, w.stot, w.P, a.V), 0, 0);
 }
 
-// 8. accept mode: the round, walking the rows in order (n_accept, n_emit, n_uniform, flags, tokens).
-__global__ __launch_bounds__(64) void samp_decide_kernel(SampArgs a) {
-  if (threadIdx.x != 0) return;
+// ---------------------------------------------------------------- top-k rows in three launches
+// A row with 0 < top_k <= kTopkMax (and top_k < V) carries weight on its top-k survivors only, so after the k-th largest
+// logit is known everything else is work on a few dozen values, done by one workgroup per row in LDS:
+//   1. samp_scan_kernel, one wave per 1024-entry chunk: raw argmax, non-finite flag, chunk maximum, and the largest key
+//      of each of G groups of the chunk (1, 4 or 16: the smallest that gives 2 k groups in the row);
+//   2. samp_cand_kernel, one wave per chunk: tau, the largest threshold with zero low 16 bits that at least k group
+//      maxima reach, bounds the k-th largest entry from below; the chunk's entries >= tau whose exp is not 0 are listed
+//      in index order (an entry with exp 0 carries no weight, and when fewer than k entries carry weight all of them
+//      survive, whatever the k-th is);
+//   3. samp_topk_draw_kernel, one workgroup per row: the exact k-th by ranks, exp, z, top-p, min-p and the draw.
+// The operations and sums are those of the launches below (or_sample's): sums over zeros change no bit of a
+// non-negative sum, so a chunk total is the butterfly over its nonzero leaves and chunks without survivors drop out.
+// More than kCand candidates or kSurv survivors (ties at the threshold) take the whole sequence inside the workgroup.
+// Latency bound. Three rows over 248,320 tokens at the default parameters (top-k 40, top-p 0.95): 33 us per round (5 +
+// 7 + 21 in the kernels); eleven launches (four radix passes over the row, exp, the compact top-p search, keep, totals,
+// draw, accept walk) took 106.
+constexpr int kTopkMax = 512;
+constexpr int kCand = 2048, kSurv = 1024;
+
+SS_DEV float logit_of(const SampArgs& a, const float* x, int row, int j) {
+  const float xx = x[j];
+  return (penalized(a, row, j) ? xx - a.pp : xx) / a.temperature;
+}
+
+// The chunk's 16 entries of this lane; 16-byte loads where every row is 16-byte aligned (`vec`).
+SS_DEV void load_chunk(const float* x, int j0, int V, bool vec, float (&v)[kSub]) {
+  if (vec && j0 + kSub <= V) {
+#pragma unroll
+    for (int q = 0; q < kSub / 4; ++q) {
+      const uint4 t = ldg16(x + j0 + 4 * q);
+      v[4 * q] = __uint_as_float(t.x);
+      v[4 * q + 1] = __uint_as_float(t.y);
+      v[4 * q + 2] = __uint_as_float(t.z);
+      v[4 * q + 3] = __uint_as_float(t.w);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) v[i] = j0 + i < V ? x[j0 + i] : 0.f;
+  }
+}
+
+SS_DEV float unkey_nan(uint32_t k) { return k == 0xFFFFFFFFu ? __uint_as_float(0x7FC00000u) : ss_unkey(k); }
+
+__global__ __launch_bounds__(64) void samp_scan_kernel(SampArgs a, int groups, int vec) {
+  const int c = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+  SW w = sw_of(a.work, a.V, a.nch, row);
+  const int j0 = c * kChunk + lane * kSub;
+  float xv[kSub];
+  load_chunk(a.x + (size_t)row * a.V, j0, a.V, vec != 0, xv);
+  // the first maximum of the raw logits, and the largest key after the penalty (the temperature is applied to the
+  // maxima: division by it is monotone, so the maximum of the quotients is the quotient of the maximum)
+  uint32_t br = 0, bp = 0, bad = 0;
+  int ir = 0;
+#pragma unroll
+  for (int i = 0; i < kSub; ++i) {
+    const int j = j0 + i;
+    if (j < a.V) {
+      const uint32_t k = nkey(xv[i]);
+      bad |= !is_finite(xv[i]);
+      ir = k > br ? j : ir;
+      br = k > br ? k : br;
+      if (a.pp != 0.f) {
+        const uint32_t k2 = penalized(a, row, j) ? nkey(xv[i] - a.pp) : k;
+        bp = k2 > bp ? k2 : bp;
+      }
+    }
+  }
+  if (a.pp == 0.f) bp = br;
+  const uint64_t kr = ss_wave_max_u64(br ? ((uint64_t)br << 32) | (0xFFFFFFFFu - (uint32_t)ir) : 0ull);
+  bad = ss_wave_or(bad);
+  auto mx = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
+  auto scaled = [&](uint32_t k) { return k ? nkey(unkey_nan(k) / a.temperature) : 0u; };
+  bp = mx(bp, ss_xor_lane<1>(bp));
+  bp = mx(bp, ss_xor_lane<2>(bp));
+  if (groups == 16 && (lane & 3) == 0) w.gkey[c * 16 + lane / 4] = scaled(bp);
+  bp = mx(bp, ss_xor_lane<4>(bp));
+  bp = mx(bp, ss_xor_lane<8>(bp));
+  if (groups == 4 && (lane & 15) == 0) w.gkey[c * 4 + lane / 16] = scaled(bp);
+  uint32_t lo, hi;
+  ss_pair<16>(bp, lo, hi);
+  bp = mx(lo, hi);
+  ss_pair<32>(bp, lo, hi);
+  bp = mx(lo, hi);
+  if (lane == 0) {
+    const uint32_t k = scaled(bp);
+    if (groups == 1) w.gkey[c] = k;
+    w.craw[c] = kr;
+    w.cbad[c] = (int)bad;
+    w.cmax[c] = unkey_nan(k);
+    w.cnan[c] = k == 0xFFFFFFFFu;
+    if (c == 0 && row == 0) *w.done = 0;
+  }
+}
+
+// NV: group keys per lane.
+template <int NV>
+__global__ __launch_bounds__(64) void samp_cand_kernel(SampArgs a, int groups, int vec) {
+  const int c = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+  SW w = sw_of(a.work, a.V, a.nch, row);
+  const float* x = a.x + (size_t)row * a.V;
+  const int ng = groups * a.nch, j0 = c * kChunk + lane * kSub;
+  uint32_t gk[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) gk[i] = lane + 64 * i < ng ? w.gkey[lane + 64 * i] : 0u;
+  float xv[kSub];
+  load_chunk(x, j0, a.V, vec != 0, xv);
+  uint32_t kmax = gk[0];  // the row's largest key: its maximum (NaN: the row takes the fallback, whatever is listed)
+#pragma unroll
+  for (int i = 1; i < NV; ++i) kmax = gk[i] > kmax ? gk[i] : kmax;
+  const float m = unkey_nan(ss_wave_max_u32(kmax));
+  uint32_t tau = 0;
+  if (a.top_k <= ng) {
+#pragma unroll 1
+    for (int b = 31; b >= 16; --b) {
+      const uint32_t t = tau | (1u << b);
+      uint32_t n = 0;
+#pragma unroll
+      for (int i = 0; i < NV; ++i) n += gk[i] >= t;
+      n = ss_butterfly(n, [](uint32_t p, uint32_t q) { return p + q; });
+      tau = (int)n >= a.top_k ? t : tau;
+    }
+  }
+  uint32_t take = 0;
+  float lv[kSub];
+#pragma unroll
+  for (int i = 0; i < kSub; ++i) {
+    const int j = j0 + i;
+    const float l = (j < a.V && penalized(a, row, j) ? xv[i] - a.pp : xv[i]) / a.temperature;
+    lv[i] = l;
+    if (j < a.V && nkey(l) >= tau) take |= 1u << i;
+  }
+  if (__ballot(take != 0)) {
+    // l < m - 103.98 is exactly exp 0 (ss_expf's bound); NaN compares false and is dropped with its row
+#pragma unroll
+    for (int i = 0; i < kSub; ++i)
+      if (!(lv[i] - m >= -103.97208404541015625f)) take &= ~(1u << i);
+  }
+  const int nz = __popc(take);
+  int incl = nz;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(incl, d);
+    incl += lane >= d ? o : 0;
+  }
+  int pos = incl - nz;
+#pragma unroll
+  for (int i = 0; i < kSub; ++i)
+    if ((take >> i) & 1u) {
+      if (pos < kSlot) w.cand[(size_t)c * kSlot + pos] = ((uint64_t)(uint32_t)(j0 + i) << 32) | __float_as_uint(lv[i]);
+      ++pos;
+    }
+  if (lane == 63) w.cnz[c] = incl;
+}
+
+// The accept walk of the sampled round from the rows' results, one thread (see samp_decide_kernel).
+SS_DEV void accept_walk(const SampArgs& a) {
   const int D = a.R - 1;
   int na = 0, ne = 0, nu = 0, fl = 0;
   for (int i = 0; i <= D; ++i) {
     const SW w = sw_of(a.work, a.V, a.nch, i);
-    if (w.res[2]) {
+    const int tok = __hip_atomic_load(w.res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int fb = __hip_atomic_load(w.res + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_load(w.res + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
       fl |= kFlagNonfinite;
       break;
     }
-    const int tok = w.res[0];
     a.out[4 + i] = tok;
     ne = i + 1;
     if (a.temperature > 0.f) nu = i + 1;
-    if (w.res[1]) fl |= kFlagFallback;
+    if (fb) fl |= kFlagFallback;
     if (i == D) break;
     const int d = a.drafts[i];
     if (d < 0 || d >= a.V) fl |= kFlagBadDraft;
@@ -922,6 +852,481 @@ __global__ __launch_bounds__(64) void samp_decide_kernel(SampArgs a) {
   a.out[1] = ne;
   a.out[2] = nu;
   a.out[3] = fl;
+}
+
+constexpr int kDrawThreads = 1024, kDrawWaves = kDrawThreads / 64;
+
+struct DrawSmem {
+  int off[kDrawThreads];       // inclusive candidate counts over the chunks
+  int j[kCand];                // candidates, then (j2, p) the survivors, in index order
+  float l[kCand];
+  __attribute__((aligned(16))) uint32_t key[kCand];  // zero-padded to a multiple of 8
+  int j2[kSurv], rank[kSurv];
+  float p[kSurv];              // exp, probabilities, final weights
+  __attribute__((aligned(16))) uint64_t rho[kSurv];  // zero-padded to a multiple of 4
+  float by_rank[kSurv];        // probabilities by rank
+  int start[kSurv + 1];        // first survivor of each active chunk
+  int multi[kSurv];            // the active chunk has survivors in more than one sub-chunk
+  __attribute__((aligned(16))) float ct[kDrawThreads];  // chunk totals (the draw; the in-workgroup sequence)
+  int wsum[kDrawWaves];
+  uint32_t wmax[kDrawWaves];
+  int hist[256];
+  uint32_t kth;
+  int pick, digit, prefix, need;
+  float z;
+};
+
+// Inclusive sum over the workgroup of v (threads in order); `total` the sum over all.
+SS_DEV int block_scan(int v, int* wsum, int& total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int incl = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(incl, d);
+    incl += lane >= d ? o : 0;
+  }
+  __syncthreads();
+  if (lane == 63) wsum[w] = incl;
+  __syncthreads();
+  int t = 0;
+#pragma unroll
+  for (int q = 0; q < kDrawWaves; ++q) {
+    incl += q < w ? wsum[q] : 0;
+    t += wsum[q];
+  }
+  total = t;
+  return incl;
+}
+
+// Hierarchical sum of the survivors of rank < m (whole wave): lane t holds active chunk t's total; a chunk whose
+// survivors share one sub-chunk is their sum in index order (the butterfly adds zeros), another takes the butterfly
+// over its leaves. Chunk totals are added in order. `ct` (if not null) receives them.
+SS_DEV float masked_sum(const DrawSmem& s, int na, int m, float* ct) {
+  const int lane = threadIdx.x & 63;
+  float S = 0.f;
+  for (int t0 = 0; t0 < na; t0 += 64) {
+    const int t = t0 + lane;
+    float v = 0.f;
+    const bool multi = t < na && s.multi[t];
+    if (t < na && !multi) {
+      const int q0 = s.start[t], q1 = s.start[t + 1];
+      const float p0 = s.p[q0];
+      v = s.rank[q0] < m ? p0 : 0.f;
+      for (int q = q0 + 1; q < q1; ++q) {
+        const float nx = v + s.p[q];
+        v = s.rank[q] < m ? nx : v;
+      }
+    }
+    for (uint64_t todo = __ballot(multi); todo; todo &= todo - 1) {
+      const int src = (int)__builtin_ctzll(todo);
+      float leaf = 0.f;
+      for (int q = s.start[t0 + src]; q < s.start[t0 + src + 1]; ++q) {
+        const float nx = leaf + s.p[q];
+        leaf = s.rank[q] < m && ((s.j2[q] & (kChunk - 1)) >> 4) == lane ? nx : leaf;
+      }
+      leaf = ss_wave_sum(leaf);
+      v = lane == src ? leaf : v;
+    }
+    if (ct && t < na) ct[t] = v;
+    // lanes past the last chunk hold 0, and adding it changes nothing
+    const int nt = na - t0 < 64 ? na - t0 : 64;
+    for (int q = 0; q < nt; q += 16)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S = S + ss_readlane_f(v, q + i);
+  }
+  return S;
+}
+
+// The whole sequence of a top-k row inside the workgroup (the launches below, chunk by chunk): more candidates or
+// survivors than the lists hold. Returns the token, or -1 when the total is not finite and > 0.
+SS_DEV int draw_in_workgroup(const SampArgs& a, const SW& w, DrawSmem& s, int row, float m, float* masses) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nch = a.nch;
+  const float* x = a.x + (size_t)row * a.V;
+  for (int j = tid; j < a.V; j += kDrawThreads) w.L[j] = logit_of(a, x, row, j);
+  uint32_t prefix = 0;
+  int need = a.top_k;
+  for (int pass = 0; pass < 4; ++pass) {
+    const int shift = 24 - 8 * pass;
+    __syncthreads();
+    if (tid < 256) s.hist[tid] = 0;
+    __syncthreads();
+    for (int j = tid; j < a.V; j += kDrawThreads) {
+      const uint32_t k = nkey(w.L[j]);
+      if (pass == 0 || (k >> (shift + 8)) == (prefix >> (shift + 8))) atomicAdd(&s.hist[(k >> shift) & 255], 1);
+    }
+    __syncthreads();
+    if (wv == 0) {
+      select_pass<1>(s.hist, need, prefix, shift);
+      if (lane == 0) {
+        s.prefix = (int)prefix;
+        s.need = need;
+      }
+    }
+    __syncthreads();
+    prefix = (uint32_t)s.prefix;
+    need = s.need;
+  }
+  const float kth = unkey_nan(prefix);
+  for (int c = wv; c < nch; c += kDrawWaves) {
+    float v[kSub], sub;
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) {
+      const int j = c * kChunk + lane * kSub + i;
+      const float l = j < a.V ? w.L[j] : 0.f;
+      v[i] = j < a.V ? (l < kth ? 0.f : ss_expf(l - m)) : 0.f;
+      if (j < a.V) w.P[j] = v[i];
+    }
+    const float t = chunk_sum(v, sub);
+    if (lane == 0) s.ct[c] = t;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    float z = 0.f;
+    for (int c = 0; c < nch; ++c) z = z + s.ct[c];
+    s.z = z;
+  }
+  __syncthreads();
+  const float z = s.z;
+  uint64_t r = 0;
+  if (a.top_p < 1.f) {
+    for (int round = 0; round < kRounds; ++round) {
+      const int sft = kRhoBits - 4 - 4 * round;
+      const uint64_t r_hi = r >> (sft + 4);
+      for (int c = wv; c < nch; c += kDrawWaves) {
+        float acc[16];
+#pragma unroll
+        for (int d = 0; d < 16; ++d) acc[d] = 0.f;
+#pragma unroll
+        for (int i = 0; i < kSub; ++i) {
+          const int j = c * kChunk + lane * kSub + i;
+          const float p = j < a.V ? w.P[j] / z : 0.f;
+          if (j < a.V && p != 0.f) {
+            const uint64_t rho = rho_of(p, j);
+            const uint64_t hi = rho >> (sft + 4);
+            const int lim = hi > r_hi ? 16 : (hi == r_hi ? (int)((rho >> sft) & 15) : 0);
+#pragma unroll
+            for (int d = 0; d < 16; ++d) acc[d] = acc[d] + (d < lim ? p : 0.f);
+          }
+        }
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+          const float t = ss_wave_sum(acc[d]);
+          if (lane == 0) masses[d * nch + c] = t;
+        }
+      }
+      __syncthreads();
+      if (wv == 0) {
+        float cum = 0.f;
+        for (int c = 0; c < nch; ++c) cum = cum + masses[(lane & 15) * nch + c];
+        const uint64_t ok = __ballot(lane < 16 && cum < a.top_p);
+        if (lane == 0) s.digit = ok ? (int)__builtin_ctzll(ok) : 15;
+      }
+      __syncthreads();
+      r |= (uint64_t)s.digit << sft;
+    }
+  }
+  // keep rho >= r; the largest kept probability for min-p
+  float pm = -__builtin_inff();
+  for (int j = tid; j < a.V; j += kDrawThreads) {
+    float p = w.P[j] / z;
+    if (a.top_p < 1.f && !(rho_of(p, j) >= r)) p = 0.f;
+    w.P[j] = p;
+    pm = fmaxf(pm, p);
+  }
+  pm = ss_wave_max(pm);
+  __syncthreads();
+  if (lane == 0) masses[wv] = pm;
+  __syncthreads();
+  for (int q = 0; q < kDrawWaves; ++q) pm = fmaxf(pm, masses[q]);
+  const float cutoff = pm * a.min_p;
+  if (tid < kDrawThreads) s.ct[tid] = 0.f;
+  __syncthreads();
+  for (int c = wv; c < nch; c += kDrawWaves) {
+    float v[kSub], sub;
+#pragma unroll
+    for (int i = 0; i < kSub; ++i) {
+      const int j = c * kChunk + lane * kSub + i;
+      float p = j < a.V ? w.P[j] : 0.f;
+      if (a.min_p > 0.f && p < cutoff) {
+        p = 0.f;
+        if (j < a.V) w.P[j] = 0.f;
+      }
+      v[i] = p;
+    }
+    const float t = chunk_sum(v, sub);
+    w.stot[c * 64 + lane] = sub;
+    if (lane == 0) s.ct[c] = t;
+  }
+  __syncthreads();
+  int pick = -1;
+  if (wv == 0) {
+    const float total = lds_seq_sum(s.ct, nch, 0.f);
+    if (is_finite(total) && total > 0.f) pick = draw_descent(a.u[row], total, s.ct, nch, w.stot, w.P, a.V);
+    if (lane == 0) s.pick = pick;
+  }
+  __syncthreads();
+  return s.pick;
+}
+
+__global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float masses[];  // [16][nch]: the in-workgroup sequence
+  __shared__ __attribute__((aligned(16))) DrawSmem s;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nch = a.nch;
+  SW w = sw_of(a.work, a.V, nch, row);
+  auto finish = [&](int tok, int fb, int nonfinite) {  // whole workgroup
+    if (tid != 0) return;
+    if (!a.accept) {
+      a.out[0] = tok;
+      a.out[1] = fb;
+      return;
+    }
+    __hip_atomic_store(w.res, tok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(w.res + 1, fb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(w.res + 2, nonfinite, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);  // the results are performed before the arrival below is counted
+    int* done = sw_of(a.work, a.V, nch, 0).done;
+    if (__hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.R - 1) accept_walk(a);
+  };
+  const int cnt = tid < nch ? w.cnz[tid] : 0;
+  const bool bad = tid < nch && w.cbad[tid] != 0, over = cnt > kSlot;
+  const uint32_t cm = tid < nch ? nkey(w.cmax[tid]) : 0u;
+  const uint32_t wm = ss_wave_max_u32(cm);
+  if (lane == 0) s.wmax[wv] = wm;
+  if (__syncthreads_or(a.accept && bad)) return finish(-1, 0, 1);
+  uint32_t km = s.wmax[0];
+#pragma unroll
+  for (int q = 1; q < kDrawWaves; ++q) km = s.wmax[q] > km ? s.wmax[q] : km;
+  const float m = unkey_nan(km);
+  if (!is_finite(m)) {
+    // exp(l - m) is NaN somewhere (or everywhere): the total is NaN, and the draw takes the raw argmax
+    const uint64_t k = max_u64_of(w.craw, nch);
+    return finish((int)(0xFFFFFFFFu - (uint32_t)k), 1, 0);
+  }
+  int n;
+  s.off[tid] = block_scan(cnt, s.wsum, n);
+  int ns = 0, na = 0;
+  bool slow = __syncthreads_or(over) || n > kCand;
+  if (!slow) {
+    // gather the candidates in index order
+    for (int q = tid; q < n; q += kDrawThreads) {
+      int lo = 0, hi = nch - 1;  // the first chunk whose inclusive count exceeds q
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (s.off[mid] > q) hi = mid;
+        else lo = mid + 1;
+      }
+      const uint64_t e = w.cand[(size_t)lo * kSlot + (q - (lo ? s.off[lo - 1] : 0))];
+      s.j[q] = (int)(e >> 32);
+      s.l[q] = __uint_as_float((uint32_t)e);
+      s.key[q] = nkey(s.l[q]);
+    }
+    if (tid < 8 && n + tid < kCand) s.key[n + tid] = 0u;
+    if (tid == 0) s.kth = 0u;
+    __syncthreads();
+    // the k-th largest key, counting multiplicity
+    if (n > a.top_k) {
+      for (int q = tid; q < n; q += kDrawThreads) {
+        const uint32_t k = s.key[q];  // above 0, the padding's key
+        int gt = 0, ge = 0;
+        for (int t = 0; t < n; t += 8) {
+          const uint4 o0 = *reinterpret_cast<const uint4*>(s.key + t), o1 = *reinterpret_cast<const uint4*>(s.key + t + 4);
+          gt += (o0.x > k) + (o0.y > k) + (o0.z > k) + (o0.w > k) + (o1.x > k) + (o1.y > k) + (o1.z > k) + (o1.w > k);
+          ge += (o0.x >= k) + (o0.y >= k) + (o0.z >= k) + (o0.w >= k) + (o1.x >= k) + (o1.y >= k) + (o1.z >= k) +
+                (o1.w >= k);
+        }
+        if (gt < a.top_k && a.top_k <= ge) s.kth = k;  // the same value from every thread that holds it
+      }
+      __syncthreads();
+    }
+    const uint32_t kth = s.kth;
+    // survivors, in index order
+    const int q0 = 2 * tid, q1 = q0 + 1;
+    const bool k0 = q0 < n && s.key[q0] >= kth, k1 = q1 < n && s.key[q1] >= kth;
+    int pos = block_scan((int)k0 + (int)k1, s.wsum, ns) - (int)k0 - (int)k1;
+    slow = ns > kSurv;
+    if (!slow) {
+      if (k0) {
+        s.j2[pos] = s.j[q0];
+        s.p[pos] = ss_expf(s.l[q0] - m);
+        ++pos;
+      }
+      if (k1) {
+        s.j2[pos] = s.j[q1];
+        s.p[pos] = ss_expf(s.l[q1] - m);
+      }
+      __syncthreads();
+      // active chunks: first survivor of each, and whether its survivors span several sub-chunks
+      const bool head = tid < ns && (tid == 0 || (s.j2[tid] >> 10) != (s.j2[tid - 1] >> 10));
+      const int t = block_scan(head ? 1 : 0, s.wsum, na) - 1;
+      if (tid < kSurv) s.multi[tid] = 0;
+      if (head) s.start[t] = tid;
+      if (tid == 0) s.start[na] = ns;
+      __syncthreads();
+      if (tid < ns && !head && (s.j2[tid] >> 4) != (s.j2[tid - 1] >> 4)) s.multi[t] = 1;
+      if (tid < ns) s.rank[tid] = 0;
+      __syncthreads();
+      if (wv == 0) {
+        const float z = masked_sum(s, na, 1, nullptr);
+        if (lane == 0) s.z = z;
+      }
+      __syncthreads();
+    }
+  }
+  if (slow) {
+    const int pick = draw_in_workgroup(a, w, s, row, m, masses);
+    if (pick >= 0) return finish(pick, 0, 0);
+    const uint64_t k = max_u64_of(w.craw, nch);
+    return finish((int)(0xFFFFFFFFu - (uint32_t)k), 1, 0);
+  }
+  // probabilities and their ranks by rho (descending; distinct, they end in the index)
+  const float z = s.z;
+  if (tid < ns) {
+    s.p[tid] = s.p[tid] / z;
+    s.rho[tid] = rho_of(s.p[tid], s.j2[tid]);
+  } else if (tid < ns + 4 && tid < kSurv) {
+    s.rho[tid] = 0ull;
+  }
+  __syncthreads();
+  if (tid < ns) {
+    const uint64_t r = s.rho[tid];
+    int rk = 0;
+    for (int t = 0; t < ns; t += 4) {
+      const ulonglong2 a0 = *reinterpret_cast<const ulonglong2*>(s.rho + t);
+      const ulonglong2 a1 = *reinterpret_cast<const ulonglong2*>(s.rho + t + 2);
+      rk += (a0.x > r) + (a0.y > r) + (a1.x > r) + (a1.y > r);
+    }
+    s.rank[tid] = rk;
+    s.by_rank[rk] = s.p[tid];
+  }
+  __syncthreads();
+  if (wv != 0) return;  // one wave from here (its LDS accesses are in order)
+  // top-p: cum(r) is a step function of the survivors, so the smallest r with cum(r) < top_p is the rho of the m'-th
+  // survivor, m' the smallest m with S(m) >= top_p (S grows with m: every partial sum is a monotone function of
+  // non-negative terms): the survivors of rank < m' stay. None: all stay.
+  int keep = ns;
+  if (a.top_p < 1.f) {
+    // The first probe is the count at which the plain prefix sum by rank reaches top_p, then its neighbours: the
+    // masses differ from it by rounding only, so two probes usually close the bracket.
+    int g = 0;
+    for (float run = 0.f; g < ns;) {
+      const float v = g + lane < ns ? s.by_rank[g + lane] : 0.f;
+      float incl = v;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const float o = __shfl_up(incl, d);
+        incl += lane >= d ? o : 0.f;
+      }
+      const uint64_t at = __ballot(run + incl >= a.top_p);
+      if (at) {
+        g += (int)__builtin_ctzll(at) + 1;
+        break;
+      }
+      run += __shfl(incl, 63);
+      g += 64;
+    }
+    int lo = 0, hi = ns + 1, step = 1;
+    g = g < 1 ? 1 : (g > ns ? ns : g);
+    while (hi - lo > 1) {
+      int mid = g;
+      if (mid <= lo || mid >= hi) mid = (lo + hi) >> 1;
+      const bool up = masked_sum(s, na, mid, nullptr) >= a.top_p;
+      if (up) hi = mid;
+      else lo = mid;
+      g = up ? mid - step : mid + step;
+      step *= 2;
+    }
+    keep = hi < ns ? hi : ns;
+  }
+  // min-p on what stays: its largest probability is rank 0's
+  float pm = 0.f;
+  for (int q = lane; q < ns; q += 64) pm = s.rank[q] == 0 ? s.p[q] : pm;
+  pm = ss_wave_max(pm);
+  const float cutoff = pm * a.min_p;
+  for (int q = lane; q < ns; q += 64)
+    if (s.rank[q] >= keep || (a.min_p > 0.f && s.p[q] < cutoff)) s.p[q] = 0.f;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float total = masked_sum(s, na, ns, s.ct);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (!is_finite(total) || !(total > 0.f)) {
+    const uint64_t k = max_u64_of(w.craw, nch);
+    return finish((int)(0xFFFFFFFFu - (uint32_t)k), 1, 0);
+  }
+  // the descent of draw_descent over the survivors: chunks, leaves and entries without weight leave its running sums
+  // and its choices unchanged
+  const float u = a.u[row];
+  const bool ge = u != 0.f;
+  const float target = ge ? u * total : 0.f;
+  auto hit = [&](float v) { return ge ? v >= target : v > target; };
+  int cs = -1, clast = -1;
+  float base = 0.f, run = 0.f;
+  for (int t0 = 0; t0 < na && cs < 0; t0 += 64) {
+    const float v = t0 + lane < na ? s.ct[t0 + lane] : 0.f;
+    const uint64_t pos = __ballot(v > 0.f);
+    if (pos) clast = t0 + 63 - (int)__builtin_clzll(pos);
+    const int nt = na - t0 < 64 ? na - t0 : 64;
+    for (int q = 0; q < nt; ++q) {
+      const float nx = run + ss_readlane_f(v, q);
+      if (hit(nx)) {
+        cs = t0 + q;
+        base = run;
+        break;
+      }
+      run = nx;
+    }
+  }
+  if (cs < 0) {
+    cs = clast;
+    base = 0.f;
+    for (int t = 0; t < cs; ++t) base = base + s.ct[t];
+  }
+  const int a0 = s.start[cs], a1 = s.start[cs + 1];
+  float sub = 0.f;  // lane b: the total of sub-chunk b
+  for (int q = a0; q < a1; ++q) {
+    const float nx = sub + s.p[q];
+    sub = ((s.j2[q] & (kChunk - 1)) >> 4) == lane ? nx : sub;
+  }
+  int bs = -1, blast = 0;
+  float sbase = base;
+  run = base;
+  for (uint64_t todo = __ballot(sub > 0.f); todo; todo &= todo - 1) {
+    const int b = (int)__builtin_ctzll(todo);
+    const float nx = run + ss_readlane_f(sub, b);
+    blast = b;
+    if (hit(nx)) {
+      bs = b;
+      sbase = run;
+      break;
+    }
+    run = nx;
+  }
+  if (bs < 0) {
+    bs = blast;
+    sbase = base;
+    for (int b = 0; b < bs; ++b) sbase = sbase + ss_readlane_f(sub, b);
+  }
+  int pick = -1, last = -1;
+  run = sbase;
+  for (int q = a0; q < a1; ++q) {
+    const int j = s.j2[q];
+    if (((j & (kChunk - 1)) >> 4) != bs) continue;
+    const float v = s.p[q];
+    last = v > 0.f ? j : last;
+    run = run + v;
+    if (hit(run)) {
+      pick = j;
+      break;
+    }
+  }
+  finish(pick >= 0 ? pick : last, 0, 0);
+}
+
+// 8. accept mode: the round, walking the rows in order (n_accept, n_emit, n_uniform, flags, tokens).
+__global__ __launch_bounds__(64) void samp_decide_kernel(SampArgs a) {
+  if (threadIdx.x == 0) accept_walk(a);
 }
 
 namespace {
@@ -945,7 +1350,29 @@ SampArgs args_of(int V, int R, const int32_t* gen, int n_gen, float temperature,
 
 size_t topp_lds_bytes(int nch) { return (size_t)16 * ((nch + 15) & ~15) * sizeof(float); }
 
-// The rows' launch sequence; which kernels run depends only on the parameters.
+// A top-k row's three launches (they draw, and in accept mode walk the round).
+bool topk_rows(const SampArgs& a) {
+  return a.temperature > 0.f && a.top_k > 0 && a.top_k < a.V && a.top_k <= kTopkMax && a.nch <= kDrawThreads;
+}
+
+hipError_t launch_topk_rows(const SampArgs& a, hipStream_t st) {
+  const dim3 g(a.nch, a.R), b(64);
+  // the smallest number of groups per chunk that gives 2 k groups, at most 32 group keys per lane
+  int groups = 1;
+  while (groups < 16 && groups * a.nch < 2 * a.top_k && 4 * groups * a.nch <= 2048) groups *= 4;
+  const int ng = groups * a.nch, vec = a.V % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0;
+  KernelCfg cfg;
+  const hipError_t e = kernel_cfg(reinterpret_cast<const void*>(samp_topk_draw_kernel), kDrawThreads, 64 * 1024, &cfg);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(samp_scan_kernel, g, b, 0, st, a, groups, vec);
+  if (ng <= 256) hipLaunchKernelGGL(samp_cand_kernel<4>, g, b, 0, st, a, groups, vec);
+  else if (ng <= 1024) hipLaunchKernelGGL(samp_cand_kernel<16>, g, b, 0, st, a, groups, vec);
+  else hipLaunchKernelGGL(samp_cand_kernel<32>, g, b, 0, st, a, groups, vec);
+  hipLaunchKernelGGL(samp_topk_draw_kernel, dim3(a.R), dim3(kDrawThreads), (size_t)16 * a.nch * sizeof(float), st, a);
+  return hipGetLastError();
+}
+
+// The rows' launch sequence of every other row; which kernels run depends only on the parameters.
 void launch_rows(const SampArgs& a, hipStream_t st) {
   const dim3 g(a.nch, a.R), b(64);
   if (!(a.temperature > 0.f)) {
@@ -961,16 +1388,11 @@ void launch_rows(const SampArgs& a, hipStream_t st) {
   if (has_k)
     for (int pass = 1; pass < 4; ++pass) hipLaunchKernelGGL(samp_hist_kernel, g, b, 0, st, a, pass);
   hipLaunchKernelGGL(samp_exp_kernel, g, b, 0, st, a, has_k);
-  // top-k rows (k <= kCompact): one workgroup per row finds r* (from the survivors, or by the radix rounds in the
-  // workgroup when a row has more); otherwise the 13 rounds run as launches
-  const int compact = has_k && has_p && a.top_k <= kCompact && a.nch <= kCompactChunks * 4;
-  if (compact) hipLaunchKernelGGL(samp_topp_compact_kernel, dim3(a.R), dim3(256), 0, st, a);
-  else if (has_p)
+  if (has_p)
     for (int round = 0; round < kRounds; ++round)
-      hipLaunchKernelGGL(samp_topp_kernel, g, b, topp_lds_bytes(a.nch), st, a, round, 0);
+      hipLaunchKernelGGL(samp_topp_kernel, g, b, topp_lds_bytes(a.nch), st, a, round);
   if (has_p || has_minp)
-    hipLaunchKernelGGL(samp_keep_kernel, g, b, has_p ? topp_lds_bytes(a.nch) : 0, st, a, has_p, has_p ? 0 : 1,
-                       compact);
+    hipLaunchKernelGGL(samp_keep_kernel, g, b, has_p ? topp_lds_bytes(a.nch) : 0, st, a, has_p, has_p ? 0 : 1);
   hipLaunchKernelGGL(samp_total_kernel, g, b, 0, st, a, has_minp, (has_p || has_minp) ? 0 : 1);
   hipLaunchKernelGGL(samp_draw_kernel, dim3(a.R), b, 0, st, a);
 }
@@ -988,6 +1410,7 @@ hipError_t launch_sample(const float* x, int V, const int32_t* gen, int n_gen, f
   a.x = x;
   a.u = u;
   a.out = out;
+  if (topk_rows(a)) return launch_topk_rows(a, st);
   launch_rows(a, st);
   return hipGetLastError();
 }
@@ -1001,6 +1424,7 @@ hipError_t launch_accept_sampled(const float* target, const int32_t* drafts, int
   a.drafts = drafts;
   a.out = out;
   a.accept = 1;
+  if (topk_rows(a)) return launch_topk_rows(a, st);
   launch_rows(a, st);
   hipLaunchKernelGGL(samp_decide_kernel, dim3(1), dim3(64), 0, st, a);
   return hipGetLastError();

@@ -196,3 +196,53 @@ def test_compact_top_p_and_its_fallback_bitwise(v):
             for u in (np.float32(0.0), np.float32(rng.random()), np.float32(0.9999)):
                 gen = set(rng.integers(0, v, 8).tolist())
                 assert dev.draw(xd, gen, t, tp, tk, mp, pp, u) == O.sample(x, gen, t, tp, tk, mp, pp, u), (ri, tk, u)
+
+
+@pytest.mark.parametrize("v", [40, 1030, 32000, 65537, 248320])
+def test_topk_rows_bitwise_at_the_edges_of_their_lists(v):
+    """Rows with a top-k of at most 512 draw from a list of candidates (entries over a bound from group maxima); group
+    sizes follow v and k, lists that overflow run the whole sequence in the workgroup. Masked vocabularies (-inf, the
+    type's lowest value), one spike, ties at and around the k-th value, a flat row, weights below exp's range, and
+    penalties that move the order, each against or_sample."""
+    print(f"[sampler] top-k lists v={v}", flush=True)
+    rng = np.random.default_rng(v + 3)
+    dev = Dev(v)
+    base = (rng.standard_normal(v) * 3).astype(np.float32)
+    few = np.full(v, -np.inf, np.float32)
+    few[rng.permutation(v)[: min(10, v)]] = base[: min(10, v)]
+    low = np.where(np.isinf(few), np.finfo(np.float32).min, few).astype(np.float32)
+    spike = base.copy()
+    spike[v // 3] = 400.0
+    run = base.copy()
+    run[: min(v, 900)] += np.float32(40.0)          # every survivor in one chunk
+    tied = np.round(base * 2).astype(np.float32) / 2  # ties everywhere
+    tie41 = base.copy()
+    tie41[np.argsort(-base, kind="stable")[30:60 if v >= 60 else v]] = np.sort(base)[::-1][30]
+    rows = dict(base=base, few=few, low=low, spike=spike, run=run, tied=tied, tie41=tie41,
+                flat=np.full(v, -2.5, np.float32), zeros=np.where(np.arange(v) % 2, 0.0, -0.0).astype(np.float32))
+    for name, x in rows.items():
+        xd = torch.from_numpy(x).cuda()
+        gen = set(rng.integers(0, v, 8).tolist()) | {int(np.argmax(x))}
+        for (t, tp, tk, mp, pp) in [(0.8, 0.95, 40, 0.0, 0.0), (0.8, 1.0, 39, 0.0, 0.7), (1.0, 0.9, min(512, v - 1), 0.02, 0.0),
+                                    (0.05, 0.7, 100 if v > 100 else 3, 0.3, -1.5), (1.5, 0.999, 1, 0.0, 0.0)]:
+            for u in (np.float32(0.0), np.float32(rng.random()), np.float32(1.0)):
+                assert dev.draw(xd, gen, t, tp, tk, mp, pp, u) == O.sample(x, gen, t, tp, tk, mp, pp, u), (name, tk, u)
+
+
+def test_topk_round_unaligned_rows_and_two_rounds_on_one_workspace():
+    """Rows of an odd vocabulary (no 16-byte loads), the round walked by its last row, twice on one workspace."""
+    from slotstream_spark_amd.engine.accept import Acceptor
+    v, D = 50001, 3
+    rng = np.random.default_rng(11)
+    acc = Acceptor(D, v)
+    params = (0.8, 0.95, 40, 0.0, 0.4)
+    sp = SampleParams(temperature=0.8, top_p=0.95, top_k=40, presence_penalty=0.4)
+    for _ in range(3):
+        t = (rng.standard_normal((D + 1, v)) * 3).astype(np.float32)
+        u = rng.random(D + 1).astype(np.float32)
+        drafts = _self_drafts(t, {5, 6}, params, u)
+        drafts[2] = (drafts[2] + 1) % v
+        want = O.accept_sampled(t, drafts, {5, 6}, *params, u)
+        got = acc.sampled_async(torch.from_numpy(t).cuda(), torch.from_numpy(drafts).cuda(), sp, {5, 6},
+                                torch.from_numpy(u).cuda()).cpu().numpy()
+        assert got.tolist() == want.tolist()
