@@ -143,18 +143,150 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const uint16_t* __restr
   }
 }
 
-// The same router tail with the scores in registers: one wave per token (four per block), lane l holding entries
-// l + 64 i (E <= 64 NV). The operations and their order are those of router_topk_kernel: max, exp(s - m) summed per
-// lane in i order then by the butterfly, one division per entry; each top-k round takes the largest
-// (key + 1) over the untaken entries and, among lanes holding it, the lowest index; the weights divide by the
-// rank-order sum of the selected probabilities.
+// The same router tail with one entry per thread: one workgroup of NW waves per token, wave i lane l holding entry
+// l + 64 i (E <= 64 NW). The operations and their order are those of router_topk_kernel: max, exp(s - m) summed per
+// lane in i order then by the butterfly, one division per entry, the top K by (key, lowest index), the weights divided
+// by the rank-order sum of the selected probabilities.
+// The selection takes no K dependent rounds: tau, the largest threshold with zero low 16 bits that at least K lane
+// maxima (over the waves) reach, bounds the top K from below; the entries >= tau (a few more than K) go to LDS in index
+// order and each one's rank is the number of larger (key + 1, lower index) words. More than 64 of them, or no tau (NaN
+// rows, mass ties), take the rounds, one wave over LDS.
+// Bound by instruction fetch and by the chain, not by data: inside a prefill layer the code is fetched anew by every
+// launch, and one wave per token with its eight entries unrolled took 11.1 us for 19 tokens (E 512) with K dependent
+// rounds and 10.0 with the list. One entry per thread is a fraction of the code and of the chain: 4.6 us.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void router_topk_block_kernel(const uint16_t* __restrict__ logits,
+                                                                    const float* __restrict__ bias,
+                                                                    float* __restrict__ probs, int32_t* __restrict__ ids,
+                                                                    float* __restrict__ weights, int E, int K) {
+  __shared__ float val[NW][64];
+  __shared__ uint32_t key[NW][64];
+  __shared__ __attribute__((aligned(16))) uint64_t cand[64];
+  __shared__ float wred[NW], sel[64];
+  __shared__ int wcnt[NW], s_id[64];
+  __shared__ float s_z;
+  __shared__ uint32_t s_tau;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int t = blockIdx.x;
+  const bool in = tid < E;
+  float v = -__builtin_inff();
+  if (in) {
+    v = ss_bf16_to_f32(logits[(size_t)t * E + tid]);
+    if (bias) v = v + bias[tid];
+  }
+  // fmaxf skips a NaN on either side, so the order of the maxima does not matter
+  const float wm = ss_wave_max(v);
+  if (lane == 0) wred[w] = wm;
+  __syncthreads();
+  float m = wred[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) m = fmaxf(m, wred[i]);
+  v = in ? ss_expf(v - m) : 0.f;  // an absent entry adds +0 to a non-negative sum
+  val[w][lane] = v;
+  __syncthreads();
+  if (w == 0) {
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) acc = acc + val[i][lane];
+    acc = ss_wave_sum(acc);
+    if (lane == 0) s_z = acc;
+  }
+  __syncthreads();
+  v = v / s_z;
+  const uint32_t kp = in ? ss_key(v) + 1u : 0u;  // NaN probabilities have kp 1
+  if (probs && in) probs[(size_t)t * E + tid] = v;
+  val[w][lane] = v;
+  key[w][lane] = kp;
+  __syncthreads();
+  if (w == 0) {
+    uint32_t lmax = kp;
+#pragma unroll
+    for (int i = 1; i < NW; ++i) lmax = key[i][lane] > lmax ? key[i][lane] : lmax;
+    uint32_t tau = 0;
+#pragma unroll 1
+    for (int b = 31; b >= 16; --b) {
+      const uint32_t c = tau | (1u << b);
+      tau = __popcll(__ballot(lmax >= c)) >= K ? c : tau;
+    }
+    if (lane == 0) s_tau = tau;
+  }
+  __syncthreads();
+  const uint32_t tau = s_tau;
+  const uint64_t bal = __ballot(kp >= tau);
+  if (lane == 0) wcnt[w] = __popcll(bal);
+  if (tid < 64) cand[tid] = 0ull;
+  __syncthreads();
+  int off = 0, nc = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    off += i < w ? wcnt[i] : 0;
+    nc += wcnt[i];
+  }
+  const bool listed = tau != 0 && nc <= 64;
+  if (listed && kp >= tau)
+    cand[off + __popcll(bal & ((1ull << lane) - 1ull))] = ((uint64_t)kp << 32) | (uint64_t)(0xFFFFu - (uint32_t)tid);
+  __syncthreads();
+  if (w != 0) return;
+  if (listed) {
+    const uint64_t my = cand[lane];  // zero past the list: ranks below every key
+    int rank = 0;
+#pragma unroll 1
+    for (int j = 0; j < nc; j += 4) {
+      const ulonglong2* q = reinterpret_cast<const ulonglong2*>(cand + j);
+      const ulonglong2 q0 = q[0], q1 = q[1];
+      rank += (q0.x > my) + (q0.y > my) + (q1.x > my) + (q1.y > my);
+    }
+    if (lane < nc && rank < K) {
+      s_id[rank] = (int)(0xFFFFu - (uint32_t)my);
+      sel[rank] = ss_unkey((uint32_t)(my >> 32) - 1u);  // the probability itself
+    }
+  } else {
+    uint32_t lk[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) lk[i] = key[i][lane];
+#pragma unroll 1
+    for (int r = 0; r < K; ++r) {
+      uint32_t lm = lk[0];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) lm = lk[i] > lm ? lk[i] : lm;
+      const uint32_t mx = ss_wave_max_u32(lm);
+      int li = NW;
+#pragma unroll
+      for (int i = NW - 1; i >= 0; --i) li = lk[i] == mx ? i : li;
+      const int bi = (int)ss_wave_min_u32((uint32_t)(li * 64 + lane));  // the lowest index holding mx
+#pragma unroll
+      for (int i = 0; i < NW; ++i) lk[i] = bi == i * 64 + lane ? 0u : lk[i];
+      if (lane == 0) {
+        s_id[r] = bi;
+        sel[r] = val[bi >> 6][bi & 63];
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float pv = lane < K ? sel[lane] : 0.f;
+  float sum = 0.f;
+#pragma unroll 1
+  for (int r = 0; r < K; ++r) sum = sum + ss_readlane_f(pv, r);  // rank-order sum of the top-k probabilities
+  if (lane < K) {
+    ids[(size_t)t * K + lane] = s_id[lane];
+    weights[(size_t)t * K + lane] = pv / sum;
+  }
+}
+
+// The router tail for many tokens: one wave per token (four per block), lane l holding entries l + 64 i (E <= 64 NV),
+// the same operations and the same selection without barriers. Its time is the waves' instructions: 8192 tokens 24 us
+// with K dependent rounds, 15.9 us with the list (E 512, inside a layer).
 template <int NV>
-__global__ __launch_bounds__(256) void router_topk_reg_kernel(const uint16_t* __restrict__ logits,
+__global__ __launch_bounds__(256) void router_topk_wave_kernel(const uint16_t* __restrict__ logits,
                                                               const float* __restrict__ bias, float* __restrict__ probs,
                                                               int32_t* __restrict__ ids, float* __restrict__ weights,
                                                               int T, int E, int K) {
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  __shared__ __attribute__((aligned(16))) uint64_t cand[4][64];
+  __shared__ float sel[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = blockIdx.x * 4 + w;
   if (t >= T) return;
   const uint16_t* lg = logits + (size_t)t * E;
   float v[NV];
@@ -183,6 +315,59 @@ __global__ __launch_bounds__(256) void router_topk_reg_kernel(const uint16_t* __
     v[i] = v[i] / z;
     kp[i] = e < E ? ss_key(v[i]) + 1u : 0u;
     if (probs && e < E) probs[(size_t)t * E + e] = v[i];
+  }
+  uint32_t lmax = kp[0];
+#pragma unroll
+  for (int i = 1; i < NV; ++i) lmax = kp[i] > lmax ? kp[i] : lmax;
+  uint32_t tau = 0;
+#pragma unroll
+  for (int b = 31; b >= 16; --b) {
+    const uint32_t c = tau | (1u << b);
+    tau = __popcll(__ballot(lmax >= c)) >= K ? c : tau;
+  }
+  uint64_t bal[NV];
+  int nc = 0;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    bal[i] = __ballot(kp[i] >= tau);
+    nc += __popcll(bal[i]);
+  }
+  if (tau != 0 && nc <= 64) {
+    uint64_t* cs = cand[w];
+    int off = 0;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const uint64_t b = bal[i];
+      const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
+      if ((b >> lane) & 1ull) cs[off + below] = ((uint64_t)kp[i] << 32) | (uint64_t)(0xFFFFu - (uint32_t)(lane + 64 * i));
+      off += __popcll(b);
+    }
+    const int ncp = (nc + 7) & ~7;  // zero words pad the list to whole groups of 8; they rank below every key
+    if (lane >= nc && lane < ncp) cs[lane] = 0ull;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint64_t my = lane < nc ? cs[lane] : 0ull;
+    int rank = 0;
+#pragma unroll 1
+    for (int j = 0; j < ncp; j += 8) {
+      const ulonglong2* q = reinterpret_cast<const ulonglong2*>(cs + j);
+      const ulonglong2 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+      rank += (q0.x > my) + (q0.y > my) + (q1.x > my) + (q1.y > my) + (q2.x > my) + (q2.y > my) + (q3.x > my) +
+              (q3.y > my);
+    }
+    const bool in = lane < nc && rank < K;
+    if (in) sel[w][rank] = ss_unkey((uint32_t)(my >> 32) - 1u);  // the probability itself
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float pv = lane < K ? sel[w][lane] : 0.f;
+    float sum = 0.f;
+#pragma unroll 1
+    for (int r = 0; r < K; ++r) sum = sum + ss_readlane_f(pv, r);  // rank-order sum of the top-k probabilities
+    if (in) ids[(size_t)t * K + rank] = (int)(0xFFFFu - (uint32_t)my);
+    if (lane < K) weights[(size_t)t * K + lane] = pv / sum;
+    return;
   }
   float mine = 0.f, sum = 0.f;
   int my_id = 0;
@@ -220,16 +405,29 @@ __global__ __launch_bounds__(256) void router_topk_reg_kernel(const uint16_t* __
   }
 }
 
+constexpr int kRouterBlockRows = 1024;
+
 hipError_t launch_router_topk(const uint16_t* logits, const float* bias, float* probs, int32_t* ids, float* weights,
                               int T, int E, int K, hipStream_t st) {
   if (E <= 512 && K <= 64) {
-    const dim3 grid((unsigned)((T + 3) / 4));
-    if (E <= 128)
-      hipLaunchKernelGGL(router_topk_reg_kernel<2>, grid, dim3(256), 0, st, logits, bias, probs, ids, weights, T, E, K);
-    else if (E <= 256)
-      hipLaunchKernelGGL(router_topk_reg_kernel<4>, grid, dim3(256), 0, st, logits, bias, probs, ids, weights, T, E, K);
-    else
-      hipLaunchKernelGGL(router_topk_reg_kernel<8>, grid, dim3(256), 0, st, logits, bias, probs, ids, weights, T, E, K);
+    // A block per token has the shorter chain, a wave per token the fewer instructions. Launched back to back, block and
+    // wave: E 512 4.3 and 5.1 us at 19 tokens, 5.2 and 5.4 at 1024, 7.0 and 5.9 at 1536, 25.6 and 11.1 at 8192; E 256
+    // and E 128 are level (4.2-4.6 us) to 1024 tokens and the wave is ahead from 2048 and 3072 on.
+    const bool block = T <= kRouterBlockRows;
+    const dim3 grid((unsigned)(block ? T : (T + 3) / 4));
+#define SS_ROUTER(N)                                                                                              \
+  if (block)                                                                                                      \
+    hipLaunchKernelGGL(router_topk_block_kernel<N>, grid, dim3(64 * N), 0, st, logits, bias, probs, ids, weights, E, K); \
+  else                                                                                                            \
+    hipLaunchKernelGGL(router_topk_wave_kernel<N>, grid, dim3(256), 0, st, logits, bias, probs, ids, weights, T, E, K)
+    if (E <= 128) {
+      SS_ROUTER(2);
+    } else if (E <= 256) {
+      SS_ROUTER(4);
+    } else {
+      SS_ROUTER(8);
+    }
+#undef SS_ROUTER
     return hipGetLastError();
   }
   const size_t lds = (size_t)E * 4 + (size_t)E;

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
+from slotstream_spark_amd import _lib
 from slotstream_spark_amd.kernels.router import lin_bf16, route
 from slotstream_spark_amd.kernels.topk_stable import topk_stable
 from slotstream_spark_amd.memory.synth import normal_bf16, zipf_bias
@@ -37,6 +38,32 @@ def test_router_bitexact(t, e, k, use_bias):
     assert np.array_equal(probs.cpu().numpy().view(np.uint32), rp.view(np.uint32))
     assert np.array_equal(ids.cpu().numpy(), ri)
     assert np.array_equal(wts.cpu().numpy().view(np.uint32), rw.view(np.uint32))
+
+
+@pytest.mark.parametrize("t", [1, 7, 1024, 1025])  # a block per token up to 1024 tokens, a wave per token beyond
+@pytest.mark.parametrize("e,k", [(5, 5), (64, 16), (65, 8), (129, 10), (257, 16), (512, 1), (512, 16)])
+def test_router_topk_rows_in_both_kernels(t, e, k):
+    rng = np.random.default_rng(e * 31 + k)
+    x = rng.standard_normal((t, e)).astype(np.float32)
+    x[t // 2] = 0.25                      # all equal: more than 64 entries at the threshold when e > 64
+    x[t - 1] = np.round(x[t - 1])         # many exact ties
+    if t > 4:
+        x[1, ::3] = -100.0                # quotients far below 2^-64
+        x[2, :] = np.where(np.arange(e) < k, 1.0, -np.inf)
+        x[4, e // 2] = np.nan             # a NaN row: ids only (lowest indices), its weights are NaN
+    lg = torch.from_numpy(x).to(torch.bfloat16)
+    lib = _lib.lib()
+    lc = lg.cuda()
+    probs = torch.empty((t, e), dtype=torch.float32, device="cuda")
+    ids = torch.empty((t, k), dtype=torch.int32, device="cuda")
+    wts = torch.empty((t, k), dtype=torch.float32, device="cuda")
+    _lib.check(lib.ssmoe_router_topk(lc.data_ptr(), None, probs.data_ptr(), ids.data_ptr(), wts.data_ptr(), t, e, k,
+                                     _lib.stream_of(lc)))
+    torch.cuda.synchronize()
+    rp, ri, rw = O.router_topk(bits(lg), k)
+    assert np.array_equal(ids.cpu().numpy(), ri)
+    assert np.array_equal(probs.cpu().numpy(), rp, equal_nan=True)
+    assert np.array_equal(wts.cpu().numpy(), rw, equal_nan=True)
 
 
 def test_router_ties_take_lower_index():
