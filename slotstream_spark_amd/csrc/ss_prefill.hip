@@ -427,6 +427,13 @@ SS_DEV ss_u32x4 dequant8(uint32_t w, float s9, float bi) {
   return r;
 }
 
+// out_rows larger than the memory-side cache (256 MB) leave by non-temporal stores: the combine finds them in memory
+// either way, and they no longer push the packed weights and h out of the caches. Smaller ones stay plain, so that the
+// combine reads them from that cache. Measured (layer, us, plain / non-temporal, H 2048): 3300 tokens (270 MB) 474 / 468,
+// 4096 555 / 547, 5500 710 / 691, 8192 974 / 960; 2600 at H 2560 (266 MB) 574 / 572; below the line 2048 (168 MB)
+// 310 / 316, 333 at H 2560 189 / 191.
+constexpr int64_t kStreamBytes = 256ll << 20;
+
 struct GemmArgs {
   const uint16_t* a;           // gate/up: x bf16 [T, H]; down: h bf16 [R, I]
   const int32_t* row_token;    // [R] (gate/up)
@@ -441,17 +448,18 @@ struct GemmArgs {
   float* out_rows;             // down output fp32 [R, H]
   int64_t R;
   int T, H, I;
+  bool stream_out;                 // down: out_rows by non-temporal stores
   int64_t w_off, s_off, b_off;     // gate (or down) pieces
   int64_t w2_off, s2_off, b2_off;  // up pieces (gate/up)
   uint64_t* trace;                 // per-block stamps (start, end, expert << 32 | valid rows, XCC << 32 | HW_ID) or null
 };
 
-// LDS barrier for data exchanged through LDS only: waits for this wave's LDS operations, not for its global loads
-// in flight (which a workgroup-scope fence would also wait for).
+// LDS barrier for data exchanged through LDS: waits for this wave's LDS operations only. (Fences would also wait for its
+// stores to memory: the compiler cannot tell them from pending loads into LDS.)
 SS_DEV void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  asm volatile("" ::: "memory");
 }
 
 // Block index -> (M block, group of N tiles). The plan's M blocks are dealt round-robin to the XCDs (workgroup b runs on
@@ -465,6 +473,15 @@ SS_DEV bool xcd_tile(int mb, int nt, int& pid_m, int& pid_n) {
   pid_m = sm * 8 + x;
   pid_n = s - sm * nt;
   return pid_m < mb;
+}
+
+// Every load of this wave issued so far has landed (vmcnt 0; the other counters are left alone). The builtin and not an
+// asm statement: the compiler counts it, so it adds no wait of its own where the loaded registers are read, behind
+// stores that were issued in between.
+SS_DEV void wait_loads() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  asm volatile("" ::: "memory");
 }
 
 // Chunk swizzle of activation row m (see above): ds_read_b128 serves lanes 0-3 and 12-15 of one quad with lanes 4-11 of
@@ -606,7 +623,8 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
       }
     }
   };
-  auto epilogue = [&](int tile) {
+  auto epilogue_as = [&](int tile, auto stream_c) {
+    constexpr bool STREAM = decltype(stream_c)::value;
 #pragma unroll
     for (int i = 0; i < NF; ++i)
 #pragma unroll
@@ -632,13 +650,20 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
         } else {
           const float wt = sm.wt[m];
           float* od = g.out_rows + (int64_t)orow * g.H + tile * TN + 16 * NB * w + NB * n;
-          if constexpr (NB == 4)
-            stg16(od, make_uint4(__float_as_uint(acc[i][0][r] * wt), __float_as_uint(acc[i][1][r] * wt),
-                                 __float_as_uint(acc[i][2][r] * wt), __float_as_uint(acc[i][3][r] * wt)));
-          else
+          if constexpr (NB == 4) {
+            const ss_f32x4 v = {acc[i][0][r] * wt, acc[i][1][r] * wt, acc[i][2][r] * wt, acc[i][3][r] * wt};
+            if constexpr (STREAM) __builtin_nontemporal_store(v, (SS_G ss_f32x4*)od);
+            else *(SS_G ss_f32x4*)od = v;
+          } else {
             *(SS_G ss_f32x2*)od = ss_f32x2{acc[i][0][r] * wt, acc[i][1][r] * wt};
+          }
         }
       }
+  };
+  auto epilogue = [&](int tile) {
+    if constexpr (!GU && NB == 4)
+      if (g.stream_out) return epilogue_as(tile, std::true_type{});
+    epilogue_as(tile, std::false_type{});
   };
 
   zero();
@@ -647,10 +672,12 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
   constexpr int SPC = kSbG / 2 / KS;  // stages per table chunk
   load_sb(tile, 0);
   load(tile, 0, std::integral_constant<int, 0>{});
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  wait_loads();
   lds_barrier();
-  // Stage f of all tiles: the next stage's loads, this stage's MFMAs, the tile's epilogue behind its last stage, then
-  // the wait for the loads (every wave's, by the barrier).
+  // Stage f of all tiles: the next stage's loads, this stage's MFMAs, the wait for those loads, the tile's epilogue
+  // behind its last stage (its stores drain under the next stage: without this the non-temporal ones cost time,
+  // 979 -> 986 us at 8192 tokens), then the barrier, so that every wave's loads have
+  // landed.
   auto stage = [&](int f, auto p_c) {
     constexpr int P = decltype(p_c)::value;
     int t2 = tile, s2 = st + 1;
@@ -662,13 +689,14 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
     if (more) load(t2, s2, std::integral_constant<int, P ^ 1>{});
     __builtin_amdgcn_sched_barrier(0);
     compute(st, p_c, more && s2 % SPC == 0, t2, s2 * KS * 2);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_loads();
     if (st == nst - 1) {
       epilogue(tile);
       zero();
     }
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    lds_barrier();
+    if (more) lds_barrier();
     tile = t2;
     st = s2;
   };
@@ -793,6 +821,7 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
   // 95 against 101 with one, 81920 280 against 300.
   const int nb_gu = p.R < 16 * (int64_t)p.num_local ? 2 : 4, nb_d = p.R < 2 * (int64_t)p.num_local ? 2 : 4;
   const int td = p.R >= 8192 && p.H % 512 == 0 ? 2 : 1;
+  g.stream_out = p.R * p.H * 4 > kStreamBytes;
   launch_gemm<true>(g, nb_gu, 1, mb, st);
   g.a = p.h_buf;
   g.w_off = rec.dw;
@@ -804,7 +833,8 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
 
 // ---------------------------------------------------------------- combine_rank_order (fused_moe_affine.py:164-172)
 // With LAYER also y = bf16(bf16(out) + bf16(bf16(sigmoid(sgl)) * sh)), the roundings of combine_shared_kernel, so the
-// sums are not read back (at 8192 tokens the two launches took 162 + 21 us). Bound by HBM: T K H 4 bytes in.
+// sums are not read back (at 8192 tokens the two launches took 162 + 21 us). Bound by HBM: T K H 4 bytes in, read
+// once and non-temporally (layer, us, plain / non-temporal loads: 333 tokens at H 2560 189 / 187, 2048 315 / 313).
 template <bool LAYER>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ rows,
                                                       const int32_t* __restrict__ row_local,
@@ -824,10 +854,14 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
   }
   // Every row is loaded (in bounds) and a skipped row's value replaced by +0 afterwards: a select between a local
   // zero and a loaded value is kept on values, never turned into a load through a selected address.
-  float4 acc = p[0];
+  auto row = [&](int k) {
+    const ss_f32x4 v = __builtin_nontemporal_load((const SS_G ss_f32x4*)(p + (int64_t)k * h4));
+    return make_float4(v[0], v[1], v[2], v[3]);
+  };
+  float4 acc = row(0);
   if (row_local && row_local[t * K] < 0) acc = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int k = 1; k < K; ++k) {
-    const float4 v = p[(int64_t)k * h4];
+    const float4 v = row(k);
     const bool skip = row_local && row_local[t * K + k] < 0;
     acc.x = acc.x + (skip ? 0.f : v.x);
     acc.y = acc.y + (skip ? 0.f : v.y);

@@ -331,3 +331,24 @@ def test_moe_prefill_config3_full_size():
     err = O.rel_l2(routed.cpu().numpy(), O.combine_rank_order(rows64, T, K))
     print(f"routed vs exact-dequant fp64 rel_l2 {err:.2e}")
     assert err < 2e-2
+
+
+@pytest.mark.parametrize("T,H", [(6900, 2560), (8193, 2048)])
+def test_prefill_streamed_rows_equal_plain_rows(T, H):
+    """Past 256 MB of out_rows the down product stores them non-temporally. Rows and sums are bit for bit those of the
+    same tokens in chunks below that (T K H 4 = 283 MB and 268 MB + 32 KB, chunks of 40 MB and less)."""
+    K, E, I = 4, 8, 128
+    print(f"[streamed rows] T={T} H={H}", flush=True)
+    pool, x, ids, w = _prefill_case(T, K, E, H, I, 11 * H + T)
+    lw = LayerWeights(H, E, 64, seed=3)
+    layer = MoEPrefillLayer(pool, 0, lw.router_w, lw.sh_gate, lw.sh_up, lw.sh_down, lw.sh_g, top_k=K, max_tokens=T)
+    assert T * K * H * 4 > 256 << 20
+    full = layer.routed_experts(x, ids, w).clone()
+    rows = layer.out_rows[:T * K].clone()
+    for t0 in range(0, T, 1000):
+        t1 = min(T, t0 + 1000)
+        layer.out_rows.fill_(7.0)
+        part = layer.routed_experts(x[t0:t1].contiguous(), ids[t0:t1].contiguous(), w[t0:t1].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(layer.out_rows[:(t1 - t0) * K], rows[t0 * K:t1 * K]), t0
+        assert torch.equal(part, full[t0:t1]), t0
