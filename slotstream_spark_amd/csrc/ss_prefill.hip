@@ -365,10 +365,13 @@ hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
 // Gate/up: the first NB / 2 fragments are gate rows, the others the same up rows, so silu(g) * u is formed in
 // registers. Column n of fragment j is the wave's weight row NB n + j (gate/up: h column (NB / 2) n + j % (NB / 2)), so
 // a lane's fragments hold adjacent outputs and the epilogues store whole pieces.
-// K order inside a step: lane quad q (lane >> 4) holds the 16 bytes of packed words 4q .. 4q + 3 of its weight row
-// (elements 32 q .. 32 q + 31, one group); MFMA slice s (0..3) uses word 4q + s, and the A fragment of slice s holds
-// the same elements of each row. The order is the same for every tile shape and every number of live rows, so a
-// row's bits depend on that row and its record only.
+// K order inside a step: its two groups one after the other, each in MFMA slices 0, 1; lane quad q (lane >> 4) of slice s
+// holds elements 16 q + 8 s .. + 7 of the group (packed word 2q + s), of the weight row and of the activation rows alike.
+// That is the dense GEMM's order, the same for every tile shape and every number of live rows, so a row's bits depend on
+// that row and its record only. A quad loads 16 bytes (four words of one group: quads 0, 1, 2, 3 words 0-3 of the first,
+// 0-3 of the second, 4-7 of the first, 4-7 of the second) and neighbouring quads exchange two words by v_permlane16_swap.
+// (Whole 16-byte pieces in K order, without the exchange, save 1-2 % of a layer but sum in another order; two 8-byte loads
+// instead of the exchange cost 5-9 % of a layer more: 2048 tokens 302 -> 324 us, 19 tokens 69 -> 75.)
 // Memory paths:
 //  * A (activations for gate/up, h for down): direct global -> LDS loads of 16 bytes per lane (four whole 256-byte row
 //    pieces per instruction), double-buffered; only the live 16-row fragments are loaded. The two stages are separate
@@ -485,7 +488,8 @@ SS_DEV void wait_loads() {
 }
 
 // Chunk swizzle of activation row m (see above): ds_read_b128 serves lanes 0-3 and 12-15 of one quad with lanes 4-11 of
-// its neighbour, whose chunk numbers differ in bit 2, so rows 4-11 (mod 16) take the upper half of the positions.
+// its neighbour; both quads' chunk numbers of a slice lie in the same half, so rows 4-11 (mod 16) take the other half of
+// the positions.
 SS_DEV int a_swz(int m) { return (m & 3) | ((m >> 1) & 4) | (((m << 1) ^ m) & 8); }
 
 constexpr int kZeroRow = (int)0x80000000u;  // a row whose activations are zero (it reads row 0; its h is stored as 0)
@@ -514,7 +518,9 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
   const int ar = 4 * w + q;
   const uint8_t* abase = reinterpret_cast<const uint8_t*>(g.a) + 16 * (n ^ a_swz(ar));
   // Lane offset of fragment 0's 16 bytes from the tile's first row; fragment j adds a uniform offset.
-  const uint32_t lw = (uint32_t)((GU ? 8 * NB * w + HB * n : 16 * NB * w + NB * n) * wrow_b + 16 * q);
+  // Quads 0 and 2 take the pieces of the step's first group, quads 1 and 3 those of its second.
+  const uint32_t lw =
+      (uint32_t)((GU ? 8 * NB * w + HB * n : 16 * NB * w + NB * n) * wrow_b + 16 * ((q >> 1) | (q & 1) << 1));
   const int64_t tile_w = (int64_t)(GU ? TN / 2 : TN) * wrow_b, tile_s = (int64_t)(GU ? TN / 2 : TN) * G * 2;
   // (s, b) table: lane (q, n) of wave w fills slot 64 w + lane with its wave's row of fragment q (lanes past NB repeat
   // the last fragment's), so a fragment's 16 rows are adjacent slots.
@@ -565,7 +571,7 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
         }
     }
   };
-  const int sb_lane = 1024 * w + (wide ? 16 : 4) * n + 2 * (q >> 1);
+  const int sb_lane = 1024 * w + (wide ? 16 : 4) * n;
   const int sb_j = wide ? 256 : 64, sb_k = wide ? 4 : 256;
 
   ss_f32x4 acc[NF][NB];
@@ -580,16 +586,16 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
   auto compute = [&](int st, auto p_c, bool chunk, int ct, int cg) {
     constexpr int P = decltype(p_c)::value;
     const uint8_t* as = (P ? a1 : a0) + n * kRowB;
-    int apos = 16 * ((4 * q) ^ a_swz(n));
+    int apos = 16 * ((2 * q) ^ a_swz(n));
     asm volatile("" : "+v"(apos));
-    float sc[KS][NB], bi[KS][NB];
+    uint32_t sp[KS][NB], bp[KS][NB];  // the step's two groups, the first in the low half
 #pragma unroll
     for (int u = 0; u < KS; ++u)
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         const int at = sb_lane + j * sb_j + ((st * KS + u) & (kSbG / 2 - 1)) * sb_k;
-        sc[u][j] = __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t*>(lss + at) << 16) * 512.f;  // s * 2^9
-        bi[u][j] = __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t*>(lsb + at) << 16);
+        sp[u][j] = *reinterpret_cast<const uint32_t*>(lss + at);
+        bp[u][j] = *reinterpret_cast<const uint32_t*>(lsb + at);
       }
     if (chunk) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -598,17 +604,34 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
       if (u > 0 && st * KS + u >= nsteps) break;
+      // Neighbouring quads exchange two words: each then holds words 2 q, 2 q + 1 of the first group, then of the second.
+      uint32_t wd[4][NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const uint4 v = bw[P][u][j];
+        const auto e0 = __builtin_amdgcn_permlane16_swap(v.x, v.z, false, false);
+        const auto e1 = __builtin_amdgcn_permlane16_swap(v.y, v.w, false, false);
+        wd[0][j] = e0[0];
+        wd[1][j] = e1[0];
+        wd[2][j] = e0[1];
+        wd[3][j] = e1[1];
+      }
+      float sc[NB], bi[NB];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
+        if (s % 2 == 0) {
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            sc[j] = __uint_as_float(s ? sp[u][j] & 0xFFFF0000u : sp[u][j] << 16) * 512.f;  // s * 2^9
+            bi[j] = __uint_as_float(s ? bp[u][j] & 0xFFFF0000u : bp[u][j] << 16);
+          }
+        }
         ss_u32x4 bf[NB];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          const uint4 v = bw[P][u][j];
-          bf[j] = dequant8(s == 0 ? v.x : s == 1 ? v.y : s == 2 ? v.z : v.w, sc[u][j], bi[u][j]);
-        }
+        for (int j = 0; j < NB; ++j) bf[j] = dequant8(wd[s][j], sc[j], bi[j]);
         // A fragments a few at a time: the scheduling barriers keep their registers few; the two waves of a SIMD
         // overlap one wave's dequantisation and LDS reads with the other's MFMAs.
-        const uint8_t* ap = as + u * NF * 16 * kRowB + (apos ^ (16 * s));
+        const uint8_t* ap = as + u * NF * 16 * kRowB + (apos ^ (16 * ((s & 1) | (s & 2) << 2)));
 #pragma unroll
         for (int i0 = 0; i0 < NF; i0 += NQ) {
           ss_u32x4 av[NQ];

@@ -137,6 +137,31 @@ def test_prefill_rows_same_bits_for_every_tile_shape(H, I):
     assert O.rel_l2(rows_full[:t * K].cpu().numpy(), rows_ref) < 2e-3
 
 
+@pytest.mark.parametrize("I", [512, 768])
+def test_down_rows_accumulate_in_the_dense_gemms_order(I):
+    """The grouped GEMM adds up a row in the order of the dense GEMM (MFMA slices of 16 q + 8 s .. + 7 inside 64 K):
+    with unit row weights its fp32 rows, rounded to bf16, are the dense product of the same h and the dequantized
+    weights, bit for bit. Another order of the fp32 sums would flip some of the rounded values. Experts of 3 to 300 rows
+    take every number of live fragments; I 768 has an odd number of 8-group chunks."""
+    H, counts = 1024, [3, 20, 40, 60, 90, 128, 300]
+    E, R = len(counts), sum(counts)
+    print(f"[K order] I={I}", flush=True)
+    pool = make_pool(E, H, I, seed=I)
+    x = normal_bf16((R, H), 1.0, I + 1)
+    row_expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32).cuda()
+    gptr = pool.slot_ptr[pool.map[:E].long()].contiguous()
+    h = torch.empty((R, I), dtype=torch.bfloat16, device="cuda")
+    out_rows = torch.empty((R, H), device="cuda")
+    fused_moe_affine(x, torch.arange(R, dtype=torch.int32, device="cuda"), torch.ones(R, device="cuda"),
+                     torch.arange(E, dtype=torch.int32, device="cuda"), gptr, out_rows, row_expert=row_expert, h_buf=h)
+    cache, r0 = DenseCache(pool), 0
+    for e, n in enumerate(counts):
+        down = torch.from_numpy(O.expert_bf16(cache.record(e), H, I)[2]).to(torch.bfloat16).cuda()
+        ref = gemm_bf16(h[r0:r0 + n].contiguous(), down)
+        assert torch.equal(out_rows[r0:r0 + n].to(torch.bfloat16), ref), (e, n)
+        r0 += n
+
+
 def test_fused_moe_affine_group_semantics():
     """The reference interface: a group of local experts through expert_map; rows outside it are left alone."""
     T, K, E, H, I = 40, 4, 12, 256, 128
