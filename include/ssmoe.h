@@ -63,7 +63,9 @@ int ssmoe_record_layout(int H, int I, int64_t* off);
  * Constraints: H % 128 == 0, H <= 4096, I % 128 == 0, I <= 1024, 1 <= K <= 16.
  * Takes no workspace (as the reference's): the library's static scratch has one slot per stream for the first 8
  * streams that call it on a device; a ninth stream shares a slot. Calls on different streams may be issued at the
- * same time: the device runs them one after the other (they wait for each other by an event). */
+ * same time: the device runs them one after the other (each waits there for the launch before it). A replay of
+ * a graph that holds such calls is not ordered; graphs captured on streams that share a slot must not run at the same
+ * time. */
 int ssmoe_moe_decode(const void* x, int x_is_f32, const int32_t* expert_ids, const float* weights, int layer,
                      const int32_t* map, int64_t map_len, const int64_t* slot_ptr, int64_t n_slots, float* h_buf,
                      float* o_buf, float* out, int R, int H, int I, int K, int E, void* stream);

@@ -646,6 +646,7 @@ __global__ __launch_bounds__(256) void greedy_round_kernel(AcceptArgs a, int uni
     a.out[OUT_NEMIT] = emit;
     a.out[OUT_NUNI] = 0;
     a.out[OUT_FLAGS] = flags;
+    ss_mark(a.done);
   }
 }
 
@@ -745,6 +746,8 @@ __global__ __launch_bounds__(256) void pq_round_kernel(AcceptArgs a, int units) 
     }
     // every workgroup has published, so every one has read the epoch: the next launch's tag may follow
     if (blockIdx.x == 0 && tid == 0) st_ag(k.ctr + kEpochInt, (int)(epoch + 1u));
+    // and every one has started (marked by the last workgroup: it holds row D, which has no second hand-off)
+    if (gw == ((units + 3) & ~3) - 1 && lane == 0) ss_mark(a.done);
     PQ_TRACE(2, tid == 0);
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -1077,20 +1080,22 @@ struct DrawArgs {
   int32_t* tokens;
   float* work;
   int* err;
+  uint32_t* done;  // null, or the count of ordered launches (OrderedStream)
   int R, V;
   float temperature;
 };
+static_assert(sizeof(DrawArgs) <= 64, "one line of kernel arguments (a second one costs 0.5 us of 8.6)");
 
 constexpr int kDrawStage = 2048;  // R x nchp chunk parts staged per workgroup (R nch <= 1024, R <= 64)
 
 template <int KM>
-__global__ __launch_bounds__(256) void draw_rows_kernel(DrawArgs a, int units) {
+__global__ __launch_bounds__(256) void draw_rows_kernel(DrawArgs a) {
   __shared__ __attribute__((aligned(16))) float sv[kDrawStage], sm[kDrawStage], sb[kDrawStage], sc[kDrawStage];
   __shared__ float mrow[64], zrow[64];
   __shared__ int brow[64];
   __shared__ uint32_t s_epoch;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int R = a.R, V = a.V, nch = nchunks_of(V), nchp = (nch + 15) & ~15;
+  const int R = a.R, V = a.V, nch = nchunks_of(V), nchp = (nch + 15) & ~15, units = R * nch;
   const int kc = KM < kMaxPerLane ? KM : (nch + 63) >> 6;
   const float invT = 1.0f / a.temperature;
   Work k = work_of(a.work, R, nch);
@@ -1152,6 +1157,7 @@ __global__ __launch_bounds__(256) void draw_rows_kernel(DrawArgs a, int units) {
     rows_stats<2, KM>(sv, sm, sb, rr, r0 + 4 < R ? 2 : 1, nch, nchp, mrow, zrow, brow);
   }
   __syncthreads();
+  if (gw == ((units + 3) & ~3) - 1 && lane == 0) ss_mark(a.done);  // every workgroup has started; no barrier follows
   if (!has) return;
   // the row's chunk: masses r_c = s_c a_c in the chunk layout
   float rv[KM];
@@ -1171,7 +1177,7 @@ __global__ __launch_bounds__(256) void draw_rows_kernel(DrawArgs a, int units) {
 }
 
 hipError_t launch_draw_rows(const float* x, int R, int V, float temperature, const float* u, void* work,
-                            int32_t* tokens, int* err, hipStream_t st) {
+                            int32_t* tokens, int* err, const OrderedStream& st) {
   const int nch = (V + kChunk - 1) / kChunk;
   const int kc = (nch + 63) >> 6;
   auto kern = kc == 1 ? draw_rows_kernel<1> : kc == 2 ? draw_rows_kernel<2> : kc == 3 ? draw_rows_kernel<3>
@@ -1192,31 +1198,29 @@ hipError_t launch_draw_rows(const float* x, int R, int V, float temperature, con
     d.tokens = tokens + r0;
     d.work = static_cast<float*>(work);
     d.err = err;
+    d.done = st.done;
     d.temperature = temperature;
     const int units = d.R * nch;
-    hipLaunchKernelGGL(kern, dim3((units + 3) / 4), dim3(256), 0, st, d, units);
-    e = hipGetLastError();
+    e = launch_ordered(kern, dim3((units + 3) / 4), dim3(256), 0, st, d);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
 }
 
-hipError_t launch_accept_greedy(const AcceptArgs& a, hipStream_t st) {
+hipError_t launch_accept_greedy(const AcceptArgs& a, const OrderedStream& st) {
   const int nch = (a.V + kChunk - 1) / kChunk;
   const int units = (a.D + 1) * nch;
   KernelCfg cfg;
   hipError_t e = kernel_cfg(reinterpret_cast<const void*>(greedy_round_kernel), 256, 0, &cfg);
   if (e != hipSuccess) return e;
   const int grid = (units + 3) / 4;
-  if (units <= kFastUnits && cfg.per_cu >= 1 && grid <= cfg.cus) {
-    hipLaunchKernelGGL(greedy_round_kernel, dim3(grid), dim3(256), 0, st, a, units);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(greedy_kernel, dim3(nch, a.D + 1), dim3(64), 0, st, a);
+  if (units <= kFastUnits && cfg.per_cu >= 1 && grid <= cfg.cus)
+    return launch_ordered(greedy_round_kernel, dim3(grid), dim3(256), 0, st, a, units);
+  hipLaunchKernelGGL(greedy_kernel, dim3(nch, a.D + 1), dim3(64), 0, st.st, a);
   return hipGetLastError();
 }
 
-hipError_t launch_accept_pq(const AcceptArgs& a, hipStream_t st) {
+hipError_t launch_accept_pq(const AcceptArgs& a, const OrderedStream& st) {
   const int nch = (a.V + kChunk - 1) / kChunk;
   const int rows = 2 * a.D + 1;
   const int units = (a.D + 1) * nch;
@@ -1228,12 +1232,10 @@ hipError_t launch_accept_pq(const AcceptArgs& a, hipStream_t st) {
   hipError_t e = kernel_cfg(reinterpret_cast<const void*>(kern), 256, 0, &cfg);
   if (e != hipSuccess) return e;
   const int grid = (units + 3) / 4;
-  if (units <= kFastUnits && cfg.per_cu >= 1 && grid <= cfg.cus) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, st, a, units);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(pq_sum_kernel, dim3(nch, rows), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(pq_residual_kernel, dim3(nch), dim3(256), 0, st, a);
+  if (units <= kFastUnits && cfg.per_cu >= 1 && grid <= cfg.cus)
+    return launch_ordered(kern, dim3(grid), dim3(256), 0, st, a, units);
+  hipLaunchKernelGGL(pq_sum_kernel, dim3(nch, rows), dim3(256), 0, st.st, a);
+  hipLaunchKernelGGL(pq_residual_kernel, dim3(nch), dim3(256), 0, st.st, a);
   return hipGetLastError();
 }
 

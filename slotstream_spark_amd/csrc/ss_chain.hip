@@ -1064,13 +1064,14 @@ __global__ __launch_bounds__(256) void chain_kernel(ChainArgs a, SsRecord rec) {
             for (int q = 0; q < kCShards; ++q)
               __hip_atomic_store(cshard(ctr, c, q), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_add(cshard(ctr, CTR_EPOCH, 0), NL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ss_mark(a.done);
       }
     }
   }
 }
 
 template <int NJG, int NJD, bool SHQ4>
-static hipError_t launch_chain_nj(const ChainArgs& a, hipStream_t st) {
+static hipError_t launch_chain_nj(const ChainArgs& a, const OrderedStream& st) {
   const SsRecord rec = ss_record_layout(a.H, a.I);
   auto kern = chain_kernel<NJG, NJD, SHQ4>;
   const CDLayout dly = cdlayout(a.T, a.H, a.I, a.Is, a.K, a.E);
@@ -1083,8 +1084,7 @@ static hipError_t launch_chain_nj(const ChainArgs& a, hipStream_t st) {
   if (dly.P < 1 || dly.total > kLdsBudget || cfg.lds_static + dly.total > 160 * 1024) return hipErrorInvalidConfiguration;
   const int grid = cfg.cus;
   if (grid <= a.H / 16 || a.E + a.Is < 4 * grid) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), dly.total, st, a, rec);
-  return hipGetLastError();
+  return launch_ordered(kern, dim3(grid), dim3(256), dly.total, st, a, rec);
 }
 
 bool chain_shape_supported(int H, int I) { return (H == 2048 && I == 512) || (H == 2560 && I == 640); }
@@ -1093,7 +1093,7 @@ const char* chain_shapes_text() {
   return "the chain kernel is built for H 2048 with I 512 (BASELINE) and H 2560 with I 640 (the reference model)";
 }
 
-hipError_t launch_chain(const ChainArgs& a, hipStream_t st) {
+hipError_t launch_chain(const ChainArgs& a, const OrderedStream& st) {
   // One instantiated shape: H 2048 x I 512, the BASELINE layer (the layer loop is sized to the register file for it);
   // other shapes run one ssmoe_moe_verify_layer_chain launch per layer.
   const int njg = a.H / 128, njd = a.I / 128;

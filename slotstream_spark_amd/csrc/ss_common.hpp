@@ -253,6 +253,11 @@ SS_DEV void ss_raise(int* err, int bit) {
   if (err) __hip_atomic_fetch_or(err, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// One more ordered launch whose workgroups have all started (one thread per launch; null: a launch that is not ordered).
+SS_DEV void ss_mark(uint32_t* done) {
+  if (done) __hip_atomic_fetch_add(done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ---------------------------------------------------------------- affine-4bit record layout
 // One expert record, pieces in the reference order (docs/model-and-repack.md:39-53,
 // kernels/moe_gemv_affine.py:22-25): gate.w gate.s gate.b up.w up.s up.b down.w down.s down.b.

@@ -440,7 +440,7 @@ int64_t lm_head_pq_workspace_bytes(int D, int N) { return (accept_work_floats(D,
 
 hipError_t launch_lm_head_pq(const void* x, int x_f32, int D, int K, const int32_t* q, const uint16_t* s,
                              const uint16_t* b, int N, const float* draft, const int32_t* drafts, const float* uniforms,
-                             float temperature, void* work, float* logits, int32_t* out, int* err, hipStream_t st) {
+                             float temperature, void* work, float* logits, int32_t* out, int* err, const OrderedStream& st) {
   GemvArgs a{};
   a.K = K;
   a.N = N;
@@ -455,7 +455,7 @@ hipError_t launch_lm_head_pq(const void* x, int x_f32, int D, int K, const int32
     a.x = static_cast<const uint8_t*>(x) + (size_t)r0 * xrow;
     a.R = R - r0 < kGR ? R - r0 : kGR;
     a.y = logits + (size_t)r0 * N;
-    hipError_t e = launch_chunk(a, x_f32, st);
+    hipError_t e = launch_chunk(a, x_f32, st.st);
     if (e != hipSuccess) return e;
   }
   AcceptArgs p{};
@@ -469,6 +469,7 @@ hipError_t launch_lm_head_pq(const void* x, int x_f32, int D, int K, const int32
   p.out = out;
   p.work = static_cast<float*>(work);
   p.err = err;
+  p.done = st.done;
   return launch_accept_pq(p, st);
 }
 

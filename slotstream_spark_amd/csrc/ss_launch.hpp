@@ -24,6 +24,24 @@ struct KernelCfg {
 };
 hipError_t kernel_cfg(const void* kern, int threads, size_t max_dyn, KernelCfg* out);
 
+// Where a kernel whose workgroups wait on each other is launched: the stream, the device's count of such launches whose
+// workgroups have all started (the kernel raises it through its `done` argument; null while the stream is being captured)
+// and the host's count of those issued.
+struct OrderedStream {
+  hipStream_t st;
+  uint32_t* done;
+  uint32_t* issued;
+};
+template <typename K, typename... A>
+hipError_t launch_ordered(K kern, dim3 grid, dim3 block, size_t lds, const OrderedStream& o, A... args) {
+  hipLaunchKernelGGL(kern, grid, block, lds, o.st, args...);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess && o.done) ++*o.issued;
+  return e;
+}
+// Holds the stream until *done has reached `issued` (ss_verify.hip).
+hipError_t launch_order_gate(const uint32_t* done, uint32_t issued, int* err, hipStream_t st);
+
 // One dense bf16 row segment for launch_dense_rows: rows [0, n) of w (bf16 [n, H], row-major) against
 // every token; the fp32 dot is rounded once to bf16 and stored at out[t * out_ld + row].
 struct DenseSeg {
@@ -96,6 +114,7 @@ struct VerifyArgs {
   void* scratch;            // verify_scratch_bytes(), counters zero on entry (the kernel leaves them zero)
   int T, H, I, Is, K, E;
   int* err;
+  uint32_t* done;           // null, or the count of ordered launches (OrderedStream)
   uint64_t* trace;          // null, or [grid][16] phase timestamps (s_memrealtime, 100 MHz)
   // Chained layers (verify mode, bf16 x): with norm_in, x is the residual stream and the layer runs on
   // bf16((x * r) * norm_w), r = 1 / sqrt(sum(x^2) / H + norm_eps) (the order of ssmoe_residual_rmsnorm; norm_w null =
@@ -106,9 +125,9 @@ struct VerifyArgs {
   uint16_t* x_plus_y;
 };
 size_t verify_scratch_bytes(int T, int H, int I, int Is, int K, int E);
-hipError_t launch_verify(const VerifyArgs& a, hipStream_t st);
+hipError_t launch_verify(const VerifyArgs& a, const OrderedStream& st);
 // The affine 4-bit shared-expert instantiations (ss_verify_q4.hip); launch_verify calls it when sh_gs is set.
-hipError_t launch_verify_q4(const VerifyArgs& a, hipStream_t st);
+hipError_t launch_verify_q4(const VerifyArgs& a, const OrderedStream& st);
 // Zeroes `bytes` (a multiple of 16) at the 16-byte aligned `p` with vector stores (a kernel, so that it can sit in a
 // captured graph where a memset node could not).
 hipError_t launch_zero16(void* p, size_t bytes, hipStream_t st);
@@ -129,12 +148,13 @@ struct ChainArgs {
   void* scratch;                 // chain_scratch_bytes(), counters zero on entry (the kernel leaves them zero)
   int T, H, I, Is, K, E;
   int* err;
+  uint32_t* done;                // null, or the count of ordered launches (OrderedStream)
   uint64_t* trace;               // null, or [grid][16] phase timestamps of the last layer
 };
 size_t chain_scratch_bytes(int T, int H, int I, int Is, int K, int E);
 bool chain_shape_supported(int H, int I);
 const char* chain_shapes_text();  // the supported shapes, for error messages
-hipError_t launch_chain(const ChainArgs& a, hipStream_t st);
+hipError_t launch_chain(const ChainArgs& a, const OrderedStream& st);
 
 // Prefill (ss_prefill.hip).
 struct AlignArgs {
@@ -209,7 +229,7 @@ hipError_t launch_sample(const float* x, int V, const int32_t* gen, int n_gen, f
 // before its first use.
 int64_t draw_work_floats(int R, int V);
 hipError_t launch_draw_rows(const float* x, int R, int V, float temperature, const float* u, void* work,
-                            int32_t* tokens, int* err, hipStream_t st);
+                            int32_t* tokens, int* err, const OrderedStream& st);
 hipError_t launch_accept_sampled(const float* target, const int32_t* drafts, int D, int V, const int32_t* seen,
                                  int n_seen, float temperature, float top_p, int top_k, float min_p, float pp,
                                  const float* uniforms, void* work, int32_t* out, hipStream_t st);
@@ -253,7 +273,7 @@ hipError_t launch_lm_head_greedy(const void* x, int x_f32, int D, int K, const i
 int64_t lm_head_pq_workspace_bytes(int D, int N);
 hipError_t launch_lm_head_pq(const void* x, int x_f32, int D, int K, const int32_t* q, const uint16_t* s,
                              const uint16_t* b, int N, const float* draft, const int32_t* drafts, const float* uniforms,
-                             float temperature, void* work, float* logits, int32_t* out, int* err, hipStream_t st);
+                             float temperature, void* work, float* logits, int32_t* out, int* err, const OrderedStream& st);
 // Argmax ids of R rows (R <= 64; workspace lm_head_greedy_workspace_bytes(R - 1, N)).
 hipError_t launch_lm_head_argmax(const void* x, int x_f32, int R, int K, const int32_t* q, const uint16_t* s,
                                  const uint16_t* b, int N, int round_bf16, void* work, float* logits, int32_t* ids,
@@ -314,10 +334,11 @@ struct AcceptArgs {
   int32_t* out;          // [D + 5]: n_accept, n_emit, n_uniform, flags, tokens[D+1]
   float* work;           // workspace floats
   int* err;
+  uint32_t* done;        // null, or the count of ordered launches (OrderedStream)
   uint64_t* trace;       // diagnostics: per-workgroup phase stamps of the one-launch p/q round, or null
 };
 int64_t accept_work_floats(int D, int V);
-hipError_t launch_accept_greedy(const AcceptArgs& a, hipStream_t st);
-hipError_t launch_accept_pq(const AcceptArgs& a, hipStream_t st);
+hipError_t launch_accept_greedy(const AcceptArgs& a, const OrderedStream& st);
+hipError_t launch_accept_pq(const AcceptArgs& a, const OrderedStream& st);
 
 }  // namespace ss

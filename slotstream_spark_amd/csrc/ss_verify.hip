@@ -23,12 +23,33 @@ hipError_t launch_zero16(void* p, size_t bytes, hipStream_t st) {
   return hipGetLastError();
 }
 
+// One wave that ends once every workgroup of the ordered launches issued so far has started (the count wraps, so the
+// difference is compared). Short polls for the first milliseconds, then sparse ones, bounded at about 20 s (a launch may sit
+// behind other work of its stream): then SS_ERR_TIMEOUT, and the stream goes on.
+__global__ __launch_bounds__(64) void order_gate_kernel(const uint32_t* done, uint32_t issued, int* err) {
+  for (int it = 0;; ++it) {
+    const uint32_t v = __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((int32_t)(v - issued) >= 0) return;
+    if (it >= kSpinMax) {
+      if (threadIdx.x == 0) ss_raise(err, SS_ERR_TIMEOUT);
+      return;
+    }
+    if (it < 4096) __builtin_amdgcn_s_sleep(8);
+    else __builtin_amdgcn_s_sleep(127);
+  }
+}
+
+hipError_t launch_order_gate(const uint32_t* done, uint32_t issued, int* err, hipStream_t st) {
+  hipLaunchKernelGGL(order_gate_kernel, dim3(1), dim3(64), 0, st, done, issued, err);
+  return hipGetLastError();
+}
+
 template <int NJG, int NJD>
-static hipError_t launch_x(const VerifyArgs& a, hipStream_t st) {
+static hipError_t launch_x(const VerifyArgs& a, const OrderedStream& st) {
   return a.x_f32 ? launch_nj<NJG, NJD, true, false>(a, st) : launch_nj<NJG, NJD, false, false>(a, st);
 }
 
-hipError_t launch_verify(const VerifyArgs& a, hipStream_t st) {
+hipError_t launch_verify(const VerifyArgs& a, const OrderedStream& st) {
   // Shapes with instantiated kernels: H in {1024, 2048, 2560, 4096} x I in {128, 256, 512, 640, 1024}.
   if (a.mode == 0 && a.sh_gs) return launch_verify_q4(a, st);
   const int njg = a.H / 128, njd = a.I / 128;

@@ -573,13 +573,14 @@ __global__ __launch_bounds__(256) void verify_kernel(VerifyArgs a, SsRecord rec)
             for (int q = 0; q < kShards; ++q)
               __hip_atomic_store(shard(ctr, c, q), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_add(shard(ctr, CTR_EPOCH, 0), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ss_mark(a.done);
       }
     }
   }
 }
 
 template <int NJG, int NJD, bool XF32, bool SHQ4>
-static hipError_t launch_nj(const VerifyArgs& a, hipStream_t st) {
+static hipError_t launch_nj(const VerifyArgs& a, const OrderedStream& st) {
   const SsRecord rec = ss_record_layout(a.H, a.I);
   auto kern = verify_kernel<NJG, NJD, XF32, SHQ4>;
   const DLayout dly = dlayout(a.T, a.H, a.I, a.K, a.E, XF32 ? 1 : 0, a.mode == 0 ? 1 : 0);
@@ -595,8 +596,7 @@ static hipError_t launch_nj(const VerifyArgs& a, hipStream_t st) {
   if (a.mode == 0 && (size_t)a.T * a.Is * 4 > dly.total - dly.pref) return hipErrorInvalidConfiguration;
   const int grid = cfg.cus;
   if (grid < a.H / 16) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), dly.total, st, a, rec);
-  return hipGetLastError();
+  return launch_ordered(kern, dim3(grid), dim3(256), dly.total, st, a, rec);
 }
 
 }  // namespace ss

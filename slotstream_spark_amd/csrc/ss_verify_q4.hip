@@ -6,11 +6,11 @@
 namespace ss {
 
 template <int NJG, int NJD>
-static hipError_t launch_x_q4(const VerifyArgs& a, hipStream_t st) {
+static hipError_t launch_x_q4(const VerifyArgs& a, const OrderedStream& st) {
   return a.x_f32 ? launch_nj<NJG, NJD, true, true>(a, st) : launch_nj<NJG, NJD, false, true>(a, st);
 }
 
-hipError_t launch_verify_q4(const VerifyArgs& a, hipStream_t st) {
+hipError_t launch_verify_q4(const VerifyArgs& a, const OrderedStream& st) {
   const int njg = a.H / 128, njd = a.I / 128;
 #define SS_CASE(G_, D_) \
   if (njg == G_ && njd == D_) return launch_x_q4<G_, D_>(a, st);
