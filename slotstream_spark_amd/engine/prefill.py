@@ -86,6 +86,11 @@ class MoEPrefillLayer:
         if x.shape[0] > self.max_tokens:
             raise ValueError(f"at most {self.max_tokens} tokens per call, got {x.shape[0]}")
         t, H, Is, dev = x.shape[0], self.hidden, self.shared_inter, x.device
+        # the C call takes the weights' shapes from H, Is and the number of experts (the shared rows are padded to H columns)
+        if (self.router_w.shape != (self.experts, H) or self.sh_cat.shape[0] < 2 * Is + 1
+                or self.sh_down.shape[0] < H or self.sh_down.shape[1] != Is):
+            raise ValueError(f"need router_w [{self.experts}, {H}], sh_gate and sh_up [Is, {H}], sh_g [1, {H}] and "
+                             f"sh_down [{H}, {Is}]")
         L, p = _lib.lib(), self.pool
         ids, w, routed = self.ids[:t], self.weights[:t], self.routed[:t]
         y = torch.empty((t, H), dtype=torch.bfloat16, device=dev)

@@ -1,5 +1,7 @@
 """Host-side logic on the CPU: the uniform stream, the acceptance bookkeeping, the slot-pool tables and record
 packing, and the synthetic generators' shapes."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -7,6 +9,7 @@ import torch
 from oracle import oracle as orc
 from slotstream_spark_amd import _lib
 from slotstream_spark_amd.engine.accept import AcceptResult, RoundStats, UniformStream
+from slotstream_spark_amd.engine.prefill import MoEPrefillLayer
 from slotstream_spark_amd.memory import synth
 from slotstream_spark_amd.memory.slot_pool import SlotPool, pack_record
 
@@ -96,3 +99,18 @@ def test_verify_logits_correlation():
     assert t.shape == (4, 20000) and d.shape == (3, 20000)
     c = np.corrcoef(t[:3].flatten().numpy(), d.flatten().numpy())[0, 1]
     assert abs(c - 0.8) < 0.02 and abs(float(t.std()) - 3.0) < 0.1
+
+
+@needs_lib
+@pytest.mark.parametrize("name,shape", [("router_w", (8, 256)), ("sh_down", (512, 512)), ("sh_down", (256, 256)),
+                                        ("sh_up", (100, 512))])
+def test_prefill_layer_refuses_weights_of_another_shape(name, shape):
+    """One C call takes every weight's shape from H, the shared width and the number of experts: a weight of another shape
+    would be read out of range, so the layer raises before it."""
+    H, I, Is, E = 512, 128, 256, 8
+    pool = SimpleNamespace(hidden=H, inter=I, experts=E, device="cpu")
+    w = dict(router_w=(E, H), sh_gate=(Is, H), sh_up=(Is, H), sh_down=(H, Is), sh_g=(1, H))
+    w[name] = shape
+    layer = MoEPrefillLayer(pool, 0, **{n: torch.zeros(s, dtype=torch.bfloat16) for n, s in w.items()}, top_k=2, max_tokens=4)
+    with pytest.raises(ValueError, match="need router_w"):
+        layer(torch.zeros((4, H), dtype=torch.bfloat16))
