@@ -269,7 +269,9 @@ int ssmoe_moe_align(const int32_t* local_expert, int64_t R, int num_local, int b
  * Replaces fused_moe_affine's two launches (kernels/fused_moe_affine.py:136-161, kernels :39-108).
  * x bf16 [T, H]; row_token int32 [R] (a token outside [0, T) reads as a zero row); row_weight fp32 [R];
  * group_ptr int64 [num_local] record bases; h_buf bf16
- * [R, I]; out_rows fp32 [R, H] (rows outside the plan are not written). H % 256 == 0, I % 128 == 0, H, I <= 4096. */
+ * [R, I]; out_rows fp32 [R, H] (rows outside the plan are not written). H % 256 == 0, I % 128 == 0, H, I <= 4096.
+ * A plan may hold up to ssmoe_padded_rows(R, num_local, 128) / 128 blocks, blocks without rows and several partial blocks
+ * of one expert included; the valid rows of a block come first. */
 int ssmoe_fused_moe_affine(const uint16_t* x, const int32_t* row_token, const float* row_weight,
                            const int32_t* sorted_rows, const int32_t* block_expert, const int32_t* num_padded,
                            const int64_t* group_ptr, int num_local, uint16_t* h_buf, float* out_rows, int64_t R,

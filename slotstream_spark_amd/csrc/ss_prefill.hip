@@ -832,10 +832,10 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
   g.w2_off = rec.uw;
   g.s2_off = rec.us;
   g.b2_off = rec.ub;
-  // Grids cover the bound of M blocks (rounded up to a multiple of 8) times the N tiles; blocks past the device-side
-  // count exit at once.
-  const int64_t P = padded_rows(p.R, p.num_local, kBM), bound = mblock_bound(p.R, p.num_local);
-  const int64_t mb = bound < P / kBM ? bound : P / kBM;
+  // Grids cover the M blocks a plan can have (rounded up to a multiple of 8) times the N tiles; blocks past the
+  // device-side count exit at once. The library's own plan has no block without rows and at most one partial block per
+  // expert; a caller's may have any number of blocks that padded_rows holds.
+  const int64_t mb = p.order ? mblock_bound(p.R, p.num_local) : padded_rows(p.R, p.num_local, kBM) / kBM;
   // Tiles: with few rows per expert most M blocks are light and the chip is short of blocks, so a wave takes two
   // weight fragments instead of four (twice the blocks); with more rows the wider wave reads its activations from LDS
   // half as often. Measured with 512 experts (us, two / four fragments): gate/up R = 190 24 / 27, 3330 (H 2560 /

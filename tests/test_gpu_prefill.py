@@ -188,6 +188,43 @@ def test_fused_moe_affine_group_semantics():
     assert np.array_equal(s.cpu().numpy(), rs) and int(n.item()) == rn
 
 
+@pytest.mark.parametrize("counts,blocks", [
+    ([0, 0, 1, 0, 0, 0, 0, 1, 0, 1, 1, 1], None),          # one block per expert, empty ones included
+    # blocks without rows, then an expert's rows one to a block
+    ([12] + [0] * 19, [(e, 0, 0) for e in range(8)] + [(0, r, 1) for r in range(12)]),
+    ([0, 130, 2], [(0, 0, 0), (1, 0, 128), (1, 128, 2), (2, 130, 2)]),
+])
+def test_fused_moe_affine_takes_plans_with_more_blocks(counts, blocks):
+    """A caller's plan may have as many blocks as padded_rows holds, more than the rows need: all of them are computed,
+    with the bits of the aligned plan."""
+    E, R, H, I = len(counts), sum(counts), 256, 128
+    print(f"[plan] counts={counts}", flush=True)
+    if blocks is None:
+        starts = np.concatenate([[0], np.cumsum(counts)])
+        blocks = [(e, int(starts[e]), counts[e]) for e in range(E)]
+    P = int(_lib.lib().ssmoe_padded_rows(R, E, BLOCK_M))
+    assert len(blocks) * BLOCK_M <= P
+    sorted_rows, block_expert = np.full(P, R, np.int32), np.full(P // BLOCK_M, -1, np.int32)
+    for b, (e, r0, n) in enumerate(blocks):
+        block_expert[b] = e
+        sorted_rows[b * BLOCK_M: b * BLOCK_M + n] = np.arange(r0, r0 + n)
+    plan = tuple(torch.from_numpy(t).cuda() for t in (sorted_rows, block_expert,
+                                                      np.array([len(blocks) * BLOCK_M], np.int32)))
+    pool = make_pool(E, H, I, seed=E)
+    x = normal_bf16((R, H), 1.0, E + 1)
+    row_expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32).cuda()
+    emap, gptr = torch.arange(E, dtype=torch.int32, device="cuda"), pool.slot_ptr[pool.map[:E].long()].contiguous()
+    got = []
+    for aligned in (None, plan):
+        h = torch.full((R, I), 7.0, dtype=torch.bfloat16, device="cuda")
+        out_rows = torch.full((R, H), 7.0, device="cuda")
+        fused_moe_affine(x, torch.arange(R, dtype=torch.int32, device="cuda"), torch.ones(R, device="cuda"), emap, gptr,
+                         out_rows, row_expert=row_expert, h_buf=h, aligned=aligned)
+        got.append((h, out_rows))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 def test_combine_rank_order_bitwise():
     T, K, H = 33, 10, 2048
     g = torch.Generator(device="cuda").manual_seed(1)
