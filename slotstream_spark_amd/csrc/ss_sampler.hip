@@ -23,6 +23,8 @@
 // order (a non-finite row ends the round without a draw, :210-212; the round goes on while the token equals the
 // draft). The launch sequence depends only on the parameters, so it can be captured in a graph: three launches for
 // rows with a top-k of at most 512 (below), one launch per step otherwise.
+#include <type_traits>
+
 #include "ss_common.hpp"
 #include "ss_launch.hpp"
 
@@ -36,7 +38,9 @@ constexpr int kPerLane = 16;  // chunk arrays of up to 1024 chunks (V <= 2^20)
 constexpr int kRhoBits = 52;  // 32 key bits above 20 index bits
 constexpr int kRounds = kRhoBits / 4;
 constexpr int kFlagNonfinite = 1, kFlagBadDraft = 2, kFlagFallback = 8;
-constexpr int kSlot = 512;  // candidates a chunk of a top-k row lists
+constexpr int kKeys = 2048;  // group keys of a top-k row, at most
+// Candidates a chunk of a top-k row lists: all of it in rows of up to 64 chunks, 512 beyond.
+__host__ __device__ constexpr int slots_of(int nch) { return nch <= 64 ? 1024 : 512; }
 constexpr int kHistShards = 8;  // copies of each top-k histogram; chunk c adds to copy c % 8 (fewer atomics per bin)
 
 SS_DEV bool is_nan(float v) { return v != v; }
@@ -80,8 +84,8 @@ __host__ __device__ inline Layout layout_of(int V, int nch) {
   l.rr = take((size_t)(kRounds + 1) * 8);   // top-p prefix at the start of each round
   l.res = take(16);                         // token, fallback flag, non-finite row
   l.cnz = take((size_t)nch * 4);            // candidates per chunk (top-k rows)
-  l.cand = take((size_t)nch * kSlot * 8);   // a chunk's candidates (index << 32 | logit bits), up to kSlot
-  l.gkey = take((size_t)nch * 16 * 4);      // largest key of each group of the row (top-k rows)
+  l.cand = take((size_t)nch * slots_of(nch) * 8);  // a chunk's candidates (index << 32 | logit bits)
+  l.gkey = take((size_t)kKeys * 4);         // largest key of each group of the row (top-k rows)
   l.done = take(4);                         // accept mode: rows drawn (row 0's word)
   l.bytes = o;
   return l;
@@ -675,7 +679,7 @@ __global__ __launch_bounds__(64) void samp_draw_kernel(SampArgs a) {
 // A row with 0 < top_k <= kTopkMax (and top_k < V) carries weight on its top-k survivors only, so after the k-th largest
 // logit is known everything else is work on a few dozen values, done by one workgroup per row in LDS:
 //   1. samp_scan_kernel, one wave per 1024-entry chunk: raw argmax, non-finite flag, chunk maximum, and the largest key
-//      of each of G groups of the chunk (1, 4 or 16: the smallest that gives 2 k groups in the row);
+//      of each of G groups of the chunk (a power of two, up to one entry a group: the smallest that gives 2 k groups);
 //   2. samp_cand_kernel, one wave per chunk: tau, the largest threshold with zero low 16 bits that at least k group
 //      maxima reach, bounds the k-th largest entry from below; the chunk's entries >= tau whose exp is not 0 are listed
 //      in index order (an entry with exp 0 carries no weight, and when fewer than k entries carry weight all of them
@@ -683,12 +687,18 @@ __global__ __launch_bounds__(64) void samp_draw_kernel(SampArgs a) {
 //   3. samp_topk_draw_kernel, one workgroup per row: the exact k-th by ranks, exp, z, top-p, min-p and the draw.
 // The operations and sums are those of the launches below (or_sample's): sums over zeros change no bit of a
 // non-negative sum, so a chunk total is the butterfly over its nonzero leaves and chunks without survivors drop out.
-// More than kCand candidates or kSurv survivors (ties at the threshold) take the whole sequence inside the workgroup.
-// Latency bound. Three rows over 248,320 tokens at the default parameters (top-k 40, top-p 0.95): 33 us per round (5 +
-// 7 + 21 in the kernels); eleven launches (four radix passes over the row, exp, the compact top-p search, keep, totals,
-// draw, accept walk) took 106.
+// More than kCand candidates, a chunk's slots or kSurv survivors (ties at the threshold) take the whole sequence inside the
+// workgroup. Latency bound. Three rows over 248,320 tokens at the default parameters (top-k 40, top-p 0.95): 32 us per
+// round (6 + 7 + 21 in the kernels); eleven launches (four radix passes over the row, exp, a top-p search in one
+// workgroup, keep, totals, draw, accept walk) took 106.
+// k from 40 to 512 (one row of normal logits, us, the eleven launches / these three): V 1000 64-132 / 38-85, 5000 67-120 /
+// 29-51, 32,000 73-126 / 29-50, 60,000 73-139 / 29-55, 248,320 91-3094 / 28-81. Of that, against groups of 16 entries or
+// more and sums by one wave: at most 16 groups a chunk left small rows without a bound (every entry listed, the lists
+// overflowed, the whole sequence in one workgroup: k 512 at V 32,000 339), and one wave walked the chunks with several
+// survivors one by one (k 400 at V 60,000 241, now 53). A flat row of 248,320: 3.2 ms (4.5).
 constexpr int kTopkMax = 512;
 constexpr int kCand = 2048, kSurv = 1024;
+constexpr int kRankMax = 256;  // longest list whose k-th key is found by ranks
 
 SS_DEV float logit_of(const SampArgs& a, const float* x, int row, int j) {
   const float xx = x[j];
@@ -722,36 +732,56 @@ __global__ __launch_bounds__(64) void samp_scan_kernel(SampArgs a, int groups, i
   load_chunk(a.x + (size_t)row * a.V, j0, a.V, vec != 0, xv);
   // the first maximum of the raw logits, and the largest key after the penalty (the temperature is applied to the
   // maxima: division by it is monotone, so the maximum of the quotients is the quotient of the maximum)
-  uint32_t br = 0, bp = 0, bad = 0;
+  uint32_t br = 0, bp = 0, bad = 0, ek[kSub];  // ek: each entry's key after the penalty (0: none)
   int ir = 0;
 #pragma unroll
   for (int i = 0; i < kSub; ++i) {
     const int j = j0 + i;
+    ek[i] = 0u;
     if (j < a.V) {
       const uint32_t k = nkey(xv[i]);
       bad |= !is_finite(xv[i]);
       ir = k > br ? j : ir;
       br = k > br ? k : br;
-      if (a.pp != 0.f) {
-        const uint32_t k2 = penalized(a, row, j) ? nkey(xv[i] - a.pp) : k;
-        bp = k2 > bp ? k2 : bp;
-      }
+      ek[i] = a.pp != 0.f && penalized(a, row, j) ? nkey(xv[i] - a.pp) : k;
+      bp = ek[i] > bp ? ek[i] : bp;
     }
   }
-  if (a.pp == 0.f) bp = br;
   const uint64_t kr = ss_wave_max_u64(br ? ((uint64_t)br << 32) | (0xFFFFFFFFu - (uint32_t)ir) : 0ull);
   bad = ss_wave_or(bad);
   auto mx = [](uint32_t p, uint32_t q) { return p > q ? p : q; };
   auto scaled = [&](uint32_t k) { return k ? nkey(unkey_nan(k) / a.temperature) : 0u; };
+  auto put = [&](int g) {  // the group of 64 / g lanes
+    if (groups == g && (lane & (64 / g - 1)) == 0) w.gkey[c * g + lane / (64 / g)] = scaled(bp);
+  };
+  auto put_parts = [&](auto h_c) {  // H groups a lane
+    constexpr int H = decltype(h_c)::value;
+    if (groups != 64 * H) return;
+#pragma unroll
+    for (int g = 0; g < H; ++g) {
+      uint32_t k = 0;
+#pragma unroll
+      for (int i = 0; i < kSub / H; ++i) k = mx(k, ek[g * (kSub / H) + i]);
+      w.gkey[c * groups + lane * H + g] = scaled(k);
+    }
+  };
+  put_parts(std::integral_constant<int, 16>{});
+  put_parts(std::integral_constant<int, 8>{});
+  put_parts(std::integral_constant<int, 4>{});
+  put_parts(std::integral_constant<int, 2>{});
+  put(64);
   bp = mx(bp, ss_xor_lane<1>(bp));
+  put(32);
   bp = mx(bp, ss_xor_lane<2>(bp));
-  if (groups == 16 && (lane & 3) == 0) w.gkey[c * 16 + lane / 4] = scaled(bp);
+  put(16);
   bp = mx(bp, ss_xor_lane<4>(bp));
+  put(8);
   bp = mx(bp, ss_xor_lane<8>(bp));
-  if (groups == 4 && (lane & 15) == 0) w.gkey[c * 4 + lane / 16] = scaled(bp);
+  put(4);
   uint32_t lo, hi;
   ss_pair<16>(bp, lo, hi);
   bp = mx(lo, hi);
+  put(2);
   ss_pair<32>(bp, lo, hi);
   bp = mx(lo, hi);
   if (lane == 0) {
@@ -768,7 +798,7 @@ __global__ __launch_bounds__(64) void samp_scan_kernel(SampArgs a, int groups, i
 // NV: group keys per lane.
 template <int NV>
 __global__ __launch_bounds__(64) void samp_cand_kernel(SampArgs a, int groups, int vec) {
-  const int c = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+  const int c = blockIdx.x, row = blockIdx.y, lane = threadIdx.x, slots = slots_of(a.nch);
   SW w = sw_of(a.work, a.V, a.nch, row);
   const float* x = a.x + (size_t)row * a.V;
   const int ng = groups * a.nch, j0 = c * kChunk + lane * kSub;
@@ -819,7 +849,7 @@ __global__ __launch_bounds__(64) void samp_cand_kernel(SampArgs a, int groups, i
 #pragma unroll
   for (int i = 0; i < kSub; ++i)
     if ((take >> i) & 1u) {
-      if (pos < kSlot) w.cand[(size_t)c * kSlot + pos] = ((uint64_t)(uint32_t)(j0 + i) << 32) | __float_as_uint(lv[i]);
+      if (pos < slots) w.cand[(size_t)c * slots + pos] = ((uint64_t)(uint32_t)(j0 + i) << 32) | __float_as_uint(lv[i]);
       ++pos;
     }
   if (lane == 63) w.cnz[c] = incl;
@@ -867,6 +897,7 @@ struct DrawSmem {
   float by_rank[kSurv];        // probabilities by rank
   int start[kSurv + 1];        // first survivor of each active chunk
   int multi[kSurv];            // the active chunk has survivors in more than one sub-chunk
+  int mlist[kSurv];            // the chunks that have
   __attribute__((aligned(16))) float ct[kDrawThreads];  // chunk totals (the draw; the in-workgroup sequence)
   int wsum[kDrawWaves];
   uint32_t wmax[kDrawWaves];
@@ -898,18 +929,17 @@ SS_DEV int block_scan(int v, int* wsum, int& total) {
   return incl;
 }
 
-// Hierarchical sum of the survivors of rank < m (whole wave): lane t holds active chunk t's total; a chunk whose
-// survivors share one sub-chunk is their sum in index order (the butterfly adds zeros), another takes the butterfly
-// over its leaves. Chunk totals are added in order. `ct` (if not null) receives them.
-SS_DEV float masked_sum(const DrawSmem& s, int na, int m, float* ct) {
-  const int lane = threadIdx.x & 63;
-  float S = 0.f;
-  for (int t0 = 0; t0 < na; t0 += 64) {
-    const int t = t0 + lane;
+// Hierarchical sum of the survivors of rank < m (whole workgroup): the active chunks' totals into s.ct (zero-padded to a
+// multiple of 16), then their sum in order, by every wave. A chunk whose survivors share one sub-chunk is their sum in
+// index order (the butterfly adds zeros), by one thread; another (nm of them) takes the butterfly over its leaves, by one
+// wave, its survivors handed round by lane reads.
+SS_DEV float masked_sum(DrawSmem& s, int na, int nm, int m) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  __syncthreads();  // the sums of the call before have been read
+  if (tid < ((na + 15) & ~15)) {
     float v = 0.f;
-    const bool multi = t < na && s.multi[t];
-    if (t < na && !multi) {
-      const int q0 = s.start[t], q1 = s.start[t + 1];
+    if (tid < na && !s.multi[tid]) {
+      const int q0 = s.start[tid], q1 = s.start[tid + 1];
       const float p0 = s.p[q0];
       v = s.rank[q0] < m ? p0 : 0.f;
       for (int q = q0 + 1; q < q1; ++q) {
@@ -917,41 +947,50 @@ SS_DEV float masked_sum(const DrawSmem& s, int na, int m, float* ct) {
         v = s.rank[q] < m ? nx : v;
       }
     }
-    for (uint64_t todo = __ballot(multi); todo; todo &= todo - 1) {
-      const int src = (int)__builtin_ctzll(todo);
-      float leaf = 0.f;
-      for (int q = s.start[t0 + src]; q < s.start[t0 + src + 1]; ++q) {
-        const float nx = leaf + s.p[q];
-        leaf = s.rank[q] < m && ((s.j2[q] & (kChunk - 1)) >> 4) == lane ? nx : leaf;
-      }
-      leaf = ss_wave_sum(leaf);
-      v = lane == src ? leaf : v;
-    }
-    if (ct && t < na) ct[t] = v;
-    // lanes past the last chunk hold 0, and adding it changes nothing
-    const int nt = na - t0 < 64 ? na - t0 : 64;
-    for (int q = 0; q < nt; q += 16)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) S = S + ss_readlane_f(v, q + i);
+    if (tid >= na || !s.multi[tid]) s.ct[tid] = v;
   }
-  return S;
+  for (int i = wv; i < nm; i += kDrawWaves) {
+    const int t = s.mlist[i], q0 = s.start[t], q1 = s.start[t + 1];
+    float leaf = 0.f;
+    if (q1 - q0 > 64) {  // lane b finds its run of survivors (sub-chunk b) by bisection
+      int lo = q0, hi = q1;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (((s.j2[mid] & (kChunk - 1)) >> 4) < lane) lo = mid + 1;
+        else hi = mid;
+      }
+      for (int q = lo; q < q1 && ((s.j2[q] & (kChunk - 1)) >> 4) == lane; ++q) {
+        const float nx = leaf + s.p[q];
+        leaf = s.rank[q] < m ? nx : leaf;
+      }
+    } else {
+      const int n = q1 - q0, q = lane < n ? q0 + lane : q0;
+      const float p = s.p[q];
+      const int at = s.rank[q] < m ? (s.j2[q] & (kChunk - 1)) >> 4 : -1;
+      for (int k = 0; k < n; ++k) {
+        const float nx = leaf + ss_readlane_f(p, k);
+        leaf = __builtin_amdgcn_readlane(at, k) == lane ? nx : leaf;
+      }
+    }
+    leaf = ss_wave_sum(leaf);
+    if (lane == 0) s.ct[t] = leaf;
+  }
+  __syncthreads();
+  return lds_seq_sum(s.ct, na, 0.f);
 }
 
-// The whole sequence of a top-k row inside the workgroup (the launches below, chunk by chunk): more candidates or
-// survivors than the lists hold. Returns the token, or -1 when the total is not finite and > 0.
-SS_DEV int draw_in_workgroup(const SampArgs& a, const SW& w, DrawSmem& s, int row, float m, float* masses) {
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nch = a.nch;
-  const float* x = a.x + (size_t)row * a.V;
-  for (int j = tid; j < a.V; j += kDrawThreads) w.L[j] = logit_of(a, x, row, j);
-  uint32_t prefix = 0;
-  int need = a.top_k;
+// The key of rank `need` (largest first, counting multiplicity) among key(0) .. key(n - 1), whole workgroup.
+template <class F>
+SS_DEV void radix_select(DrawSmem& s, int n, F key, int need, uint32_t& prefix) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  prefix = 0;
   for (int pass = 0; pass < 4; ++pass) {
     const int shift = 24 - 8 * pass;
     __syncthreads();
     if (tid < 256) s.hist[tid] = 0;
     __syncthreads();
-    for (int j = tid; j < a.V; j += kDrawThreads) {
-      const uint32_t k = nkey(w.L[j]);
+    for (int j = tid; j < n; j += kDrawThreads) {
+      const uint32_t k = key(j);
       if (pass == 0 || (k >> (shift + 8)) == (prefix >> (shift + 8))) atomicAdd(&s.hist[(k >> shift) & 255], 1);
     }
     __syncthreads();
@@ -966,6 +1005,16 @@ SS_DEV int draw_in_workgroup(const SampArgs& a, const SW& w, DrawSmem& s, int ro
     prefix = (uint32_t)s.prefix;
     need = s.need;
   }
+}
+
+// The whole sequence of a top-k row inside the workgroup (the launches below, chunk by chunk): more candidates or
+// survivors than the lists hold. Returns the token, or -1 when the total is not finite and > 0.
+SS_DEV int draw_in_workgroup(const SampArgs& a, const SW& w, DrawSmem& s, int row, float m, float* masses) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nch = a.nch;
+  const float* x = a.x + (size_t)row * a.V;
+  for (int j = tid; j < a.V; j += kDrawThreads) w.L[j] = logit_of(a, x, row, j);
+  uint32_t prefix = 0;
+  radix_select(s, a.V, [&](int j) { return nkey(w.L[j]); }, a.top_k, prefix);
   const float kth = unkey_nan(prefix);
   for (int c = wv; c < nch; c += kDrawWaves) {
     float v[kSub], sub;
@@ -1088,7 +1137,7 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
     if (__hip_atomic_fetch_add(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.R - 1) accept_walk(a);
   };
   const int cnt = tid < nch ? w.cnz[tid] : 0;
-  const bool bad = tid < nch && w.cbad[tid] != 0, over = cnt > kSlot;
+  const bool bad = tid < nch && w.cbad[tid] != 0, over = cnt > slots_of(nch);
   const uint32_t cm = tid < nch ? nkey(w.cmax[tid]) : 0u;
   const uint32_t wm = ss_wave_max_u32(cm);
   if (lane == 0) s.wmax[wv] = wm;
@@ -1104,7 +1153,8 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
   }
   int n;
   s.off[tid] = block_scan(cnt, s.wsum, n);
-  int ns = 0, na = 0;
+  int ns = 0, na = 0, nm = 0;
+  float z = 0.f;
   bool slow = __syncthreads_or(over) || n > kCand;
   if (!slow) {
     // gather the candidates in index order
@@ -1115,7 +1165,7 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
         if (s.off[mid] > q) hi = mid;
         else lo = mid + 1;
       }
-      const uint64_t e = w.cand[(size_t)lo * kSlot + (q - (lo ? s.off[lo - 1] : 0))];
+      const uint64_t e = w.cand[(size_t)lo * slots_of(nch) + (q - (lo ? s.off[lo - 1] : 0))];
       s.j[q] = (int)(e >> 32);
       s.l[q] = __uint_as_float((uint32_t)e);
       s.key[q] = nkey(s.l[q]);
@@ -1123,8 +1173,8 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
     if (tid < 8 && n + tid < kCand) s.key[n + tid] = 0u;
     if (tid == 0) s.kth = 0u;
     __syncthreads();
-    // the k-th largest key, counting multiplicity
-    if (n > a.top_k) {
+    // the k-th largest key, counting multiplicity: by ranks of a short list, by four 8-bit radix passes of a long one
+    if (n > a.top_k && n <= kRankMax) {
       for (int q = tid; q < n; q += kDrawThreads) {
         const uint32_t k = s.key[q];  // above 0, the padding's key
         int gt = 0, ge = 0;
@@ -1136,6 +1186,11 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
         }
         if (gt < a.top_k && a.top_k <= ge) s.kth = k;  // the same value from every thread that holds it
       }
+      __syncthreads();
+    } else if (n > a.top_k) {
+      uint32_t prefix = 0;
+      radix_select(s, n, [&](int q) { return s.key[q]; }, a.top_k, prefix);
+      if (tid == 0) s.kth = prefix;
       __syncthreads();
     }
     const uint32_t kth = s.kth;
@@ -1165,11 +1220,10 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
       if (tid < ns && !head && (s.j2[tid] >> 4) != (s.j2[tid - 1] >> 4)) s.multi[t] = 1;
       if (tid < ns) s.rank[tid] = 0;
       __syncthreads();
-      if (wv == 0) {
-        const float z = masked_sum(s, na, 1, nullptr);
-        if (lane == 0) s.z = z;
-      }
-      __syncthreads();
+      const int mine = tid < na ? s.multi[tid] : 0;
+      const int at = block_scan(mine, s.wsum, nm) - mine;
+      if (mine) s.mlist[at] = tid;
+      z = masked_sum(s, na, nm, 1);
     }
   }
   if (slow) {
@@ -1179,7 +1233,6 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
     return finish((int)(0xFFFFFFFFu - (uint32_t)k), 1, 0);
   }
   // probabilities and their ranks by rho (descending; distinct, they end in the index)
-  const float z = s.z;
   if (tid < ns) {
     s.p[tid] = s.p[tid] / z;
     s.rho[tid] = rho_of(s.p[tid], s.j2[tid]);
@@ -1199,7 +1252,6 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
     s.by_rank[rk] = s.p[tid];
   }
   __syncthreads();
-  if (wv != 0) return;  // one wave from here (its LDS accesses are in order)
   // top-p: cum(r) is a step function of the survivors, so the smallest r with cum(r) < top_p is the rho of the m'-th
   // survivor, m' the smallest m with S(m) >= top_p (S grows with m: every partial sum is a monotone function of
   // non-negative terms): the survivors of rank < m' stay. None: all stay.
@@ -1229,7 +1281,7 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
     while (hi - lo > 1) {
       int mid = g;
       if (mid <= lo || mid >= hi) mid = (lo + hi) >> 1;
-      const bool up = masked_sum(s, na, mid, nullptr) >= a.top_p;
+      const bool up = masked_sum(s, na, nm, mid) >= a.top_p;  // the same in every wave
       if (up) hi = mid;
       else lo = mid;
       g = up ? mid - step : mid + step;
@@ -1238,19 +1290,10 @@ __global__ __launch_bounds__(kDrawThreads) void samp_topk_draw_kernel(SampArgs a
     keep = hi < ns ? hi : ns;
   }
   // min-p on what stays: its largest probability is rank 0's
-  float pm = 0.f;
-  for (int q = lane; q < ns; q += 64) pm = s.rank[q] == 0 ? s.p[q] : pm;
-  pm = ss_wave_max(pm);
-  const float cutoff = pm * a.min_p;
-  for (int q = lane; q < ns; q += 64)
-    if (s.rank[q] >= keep || (a.min_p > 0.f && s.p[q] < cutoff)) s.p[q] = 0.f;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const float total = masked_sum(s, na, ns, s.ct);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float cutoff = s.by_rank[0] * a.min_p;
+  if (tid < ns && (s.rank[tid] >= keep || (a.min_p > 0.f && s.p[tid] < cutoff))) s.p[tid] = 0.f;
+  const float total = masked_sum(s, na, nm, ns);
+  if (wv != 0) return;  // one wave from here
   if (!is_finite(total) || !(total > 0.f)) {
     const uint64_t k = max_u64_of(w.craw, nch);
     return finish((int)(0xFFFFFFFFu - (uint32_t)k), 1, 0);
@@ -1350,6 +1393,16 @@ SampArgs args_of(int V, int R, const int32_t* gen, int n_gen, float temperature,
 
 size_t topp_lds_bytes(int nch) { return (size_t)16 * ((nch + 15) & ~15) * sizeof(float); }
 
+// Groups per chunk of a top-k row: the smallest power of two that gives 2 k groups in the row, kKeys keys at most. Every
+// k <= 512 gets its 2 k: a row of n chunks may have up to kKeys / n groups a chunk (rounded down to a power of two, one
+// entry each at most), which is more than 1024 groups with entries in every row of more than one chunk; one chunk has a
+// group per entry, and then the bound is the k-th largest entry itself but for its low bits.
+int groups_of(const SampArgs& a) {
+  int groups = 1;
+  while (groups < kChunk && (int64_t)groups * a.V < (int64_t)2 * a.top_k * kChunk && 2 * groups * a.nch <= kKeys) groups *= 2;
+  return groups;
+}
+
 // A top-k row's three launches (they draw, and in accept mode walk the round).
 bool topk_rows(const SampArgs& a) {
   return a.temperature > 0.f && a.top_k > 0 && a.top_k < a.V && a.top_k <= kTopkMax && a.nch <= kDrawThreads;
@@ -1357,10 +1410,7 @@ bool topk_rows(const SampArgs& a) {
 
 hipError_t launch_topk_rows(const SampArgs& a, hipStream_t st) {
   const dim3 g(a.nch, a.R), b(64);
-  // the smallest number of groups per chunk that gives 2 k groups, at most 32 group keys per lane
-  int groups = 1;
-  while (groups < 16 && groups * a.nch < 2 * a.top_k && 4 * groups * a.nch <= 2048) groups *= 4;
-  const int ng = groups * a.nch, vec = a.V % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0;
+  const int groups = groups_of(a), ng = groups * a.nch, vec = a.V % 4 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0;
   KernelCfg cfg;
   const hipError_t e = kernel_cfg(reinterpret_cast<const void*>(samp_topk_draw_kernel), kDrawThreads, 64 * 1024, &cfg);
   if (e != hipSuccess) return e;

@@ -246,3 +246,22 @@ def test_topk_round_unaligned_rows_and_two_rounds_on_one_workspace():
         got = acc.sampled_async(torch.from_numpy(t).cuda(), torch.from_numpy(drafts).cuda(), sp, {5, 6},
                                 torch.from_numpy(u).cuda()).cpu().numpy()
         assert got.tolist() == want.tolist()
+
+
+@pytest.mark.parametrize("v", [700, 1025, 2048, 2049, 5000, 10300, 11300, 33793, 60000, 1 << 20])
+def test_topk_rows_over_the_range_of_k(v):
+    """Every k up to 513 by either form (three launches where the row has enough groups for k, a launch per step beyond), 1
+    to 64 groups a chunk, survivors that share chunks and sub-chunks, and logits of a bf16 head (many ties)."""
+    print(f"[sampler] top-k range v={v}", flush=True)
+    rng = np.random.default_rng(v)
+    dev = Dev(v)
+    x = (rng.standard_normal(v) * 3).astype(np.float32)
+    xb = torch.from_numpy(x).to(torch.bfloat16).float().numpy()
+    for name, row in (("n", x), ("bf16", xb)):
+        xd = torch.from_numpy(row).cuda()
+        for tk in (2, 63, 100, 200, 256, 300, 400, 512, 513):
+            if tk >= v:
+                continue
+            for tp, mp in ((0.95, 0.0), (1.0, 0.01), (0.5, 0.0)):
+                u = np.float32(rng.random())
+                assert dev.draw(xd, set(), 0.9, tp, tk, mp, 0.0, u) == O.sample(row, set(), 0.9, tp, tk, mp, 0.0, u), (name, tk, tp)
