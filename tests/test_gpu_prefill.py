@@ -303,10 +303,11 @@ def test_prefill_layer_end_to_end():
 
 
 @pytest.mark.parametrize("T,E,H,Is", [(1, 8, 256, 256), (33, 64, 512, 256), (70, 520, 2048, 512), (300, 64, 256, 768),
-                                      (1100, 512, 512, 512)])
+                                      (1100, 512, 512, 512), (2049, 512, 256, 512), (1800, 520, 512, 512)])
 def test_prefill_layer_equals_its_parts(T, E, H, Is):
-    """The layer in one C call (the three dense tile shapes, ragged T and router columns) against the separate calls,
-    bit for bit."""
+    """The layer in one C call against the separate calls, bit for bit. Its input projections take the 32 x 64 tile in the
+    first three cases, 64 x 64 in the next two and 128 x 128 in the last two (17 x 13 and 15 x 13 tiles); T and the
+    router's columns are ragged."""
     K, I = 4, 128
     pool = make_pool(E, H, I, seed=T)
     lw = LayerWeights(H, E, Is, seed=T + 1)
