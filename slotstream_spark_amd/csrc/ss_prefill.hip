@@ -369,9 +369,11 @@ hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
 // holds elements 16 q + 8 s .. + 7 of the group (packed word 2q + s), of the weight row and of the activation rows alike.
 // That is the dense GEMM's order, the same for every tile shape and every number of live rows, so a row's bits depend on
 // that row and its record only. A quad loads 16 bytes (four words of one group: quads 0, 1, 2, 3 words 0-3 of the first,
-// 0-3 of the second, 4-7 of the first, 4-7 of the second) and neighbouring quads exchange two words by v_permlane16_swap.
-// (Whole 16-byte pieces in K order, without the exchange, save 1-2 % of a layer but sum in another order; two 8-byte loads
-// instead of the exchange cost 5-9 % of a layer more: 2048 tokens 302 -> 324 us, 19 tokens 69 -> 75.)
+// 0-3 of the second, 4-7 of the first, 4-7 of the second) and neighbouring quads exchange two words by v_permlane16_swap
+// (their nibbles: the words sit in a loaded quadruple, which the exchange would copy first; layer at 333 tokens 175.5 us
+// against 176.9, 8192 962 against 965). Whole 16-byte pieces in K order, without the exchange, save 1 % of a layer but sum in
+// another order; two 8-byte loads instead of the exchange cost 5-9 % of a layer (2048 tokens 302 -> 324 us, 19 tokens
+// 69 -> 75).
 // Memory paths:
 //  * A (activations for gate/up, h for down): direct global -> LDS loads of 16 bytes per lane (four whole 256-byte row
 //    pieces per instruction), double-buffered; only the live 16-row fragments are loaded. The two stages are separate
@@ -418,8 +420,21 @@ SS_DEV uint32_t and_opaque(uint32_t x, uint32_t m) {
   asm("v_and_b32 %0, %1, %2" : "=v"(r) : "s"(m), "v"(x));
   return r;
 }
-SS_DEV ss_u32x4 dequant8(uint32_t w, float s9, float bi) {
-  const int lo = (int)and_opaque(w, 0x0F0F0F0Fu), hi = (int)and_opaque(w >> 4, 0x0F0F0F0Fu);  // n0 n2 n4 n6 / n1 n3 n5 n7
+struct ss_nibbles {
+  uint32_t lo, hi;  // n0 n2 n4 n6 / n1 n3 n5 n7, one to a byte
+};
+SS_DEV ss_nibbles nibbles_of(uint32_t w) { return {and_opaque(w, 0x0F0F0F0Fu), and_opaque(w >> 4, 0x0F0F0F0Fu)}; }
+// Lanes of odd quads of a with lanes of even quads of b.
+SS_DEV void quad_exchange(ss_nibbles& a, ss_nibbles& b) {
+  const auto l = __builtin_amdgcn_permlane16_swap(a.lo, b.lo, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(a.hi, b.hi, false, false);
+  a.lo = l[0];
+  b.lo = l[1];
+  a.hi = h[0];
+  b.hi = h[1];
+}
+SS_DEV ss_u32x4 dequant8(const ss_nibbles& w, float s9, float bi) {
+  const int lo = (int)w.lo, hi = (int)w.hi;
   const auto e02 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, false), e46 = __builtin_amdgcn_cvt_pk_f32_fp8(lo, true);
   const auto e13 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, false), e57 = __builtin_amdgcn_cvt_pk_f32_fp8(hi, true);
   ss_u32x4 r;
@@ -605,16 +620,16 @@ SS_DEV void gemm_tiles(const GemmArgs& g, const GemmSmem& sm, uint8_t* a0, uint8
     for (int u = 0; u < KS; ++u) {
       if (u > 0 && st * KS + u >= nsteps) break;
       // Neighbouring quads exchange two words: each then holds words 2 q, 2 q + 1 of the first group, then of the second.
-      uint32_t wd[4][NB];
+      ss_nibbles wd[4][NB];
 #pragma unroll
       for (int j = 0; j < NB; ++j) {
         const uint4 v = bw[P][u][j];
-        const auto e0 = __builtin_amdgcn_permlane16_swap(v.x, v.z, false, false);
-        const auto e1 = __builtin_amdgcn_permlane16_swap(v.y, v.w, false, false);
-        wd[0][j] = e0[0];
-        wd[1][j] = e1[0];
-        wd[2][j] = e0[1];
-        wd[3][j] = e1[1];
+        wd[0][j] = nibbles_of(v.x);
+        wd[2][j] = nibbles_of(v.z);
+        quad_exchange(wd[0][j], wd[2][j]);
+        wd[1][j] = nibbles_of(v.y);
+        wd[3][j] = nibbles_of(v.w);
+        quad_exchange(wd[1][j], wd[3][j]);
       }
       float sc[NB], bi[NB];
 #pragma unroll
