@@ -58,6 +58,7 @@ struct PlanArgs {
   int32_t* block_expert;
   int32_t* num_padded;
   MBlock* order;      // null, or the M blocks in launch order
+  bool heavy_first;   // that order: see align_scan
 };
 
 // Key of row i: its local expert, nl for a row that is skipped, nl + 1 past R.
@@ -117,8 +118,12 @@ SS_DEV int64_t record_of(const PlanArgs& a, int e) {
 // One workgroup of 1024: the padded start of every key (ps, nl + 1 entries; hv: the heavy blocks before it), the
 // expert of every M block and, with `order`, the blocks in launch order. Thread t holds the totals of keys
 // kpt t .. kpt t + kpt - 1 in loc.
-// Launch order: blocks with more than half their rows first, the others behind them, so the light blocks fill the
-// chip's tail instead of leaving it to a few heavy ones (gate/up at 2048 tokens 136 -> 124 us, at 333 105 -> 92).
+// Launch order: with heavy_first the blocks with more than half their rows come first and the others behind them, so the
+// light blocks fill the chip's tail instead of leaving it to a few heavy ones; otherwise plan order, which mixes full
+// blocks with partial ones on a CU. Heavy first pays with few rows per expert, where the tail is most of a launch (layer,
+// us, heavy first / plan order, top-10 of 512: 200 tokens 101 / 107, 333 118 / 128, 333 at H 2560 175 / 193, 850 189 / 199,
+// 1400 254 / 272), is level from 1700 on (294 / 291, at H 2560 440 / 443; 2048 316 / 313, at H 2560 471 / 474) and loses
+// in long prompts (3300 471 / 461, 5500 695 / 678, 8192 973 / 931): up to 32 rows per expert.
 SS_DEV void align_scan(const PlanArgs& a, const int (&loc)[4], int kpt, int* ps, int* hv) {
   __shared__ int wsum[2][16];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -183,7 +188,7 @@ SS_DEV void align_scan(const PlanArgs& a, const int (&loc)[4], int kpt, int* ps,
     a.block_expert[q] = lo;
     if (a.order) {
       const int b0 = ps[lo] / bm, j = (int)q - b0, h = hv[lo + 1] - hv[lo];
-      const int at = j < h ? hv[lo] + j : nheavy + (b0 - hv[lo]) + (j - h);
+      const int at = !a.heavy_first ? (int)q : j < h ? hv[lo] + j : nheavy + (b0 - hv[lo]) + (j - h);
       a.order[at] = MBlock{record_of(a, lo), lo, (int32_t)q};
     }
   }
@@ -355,6 +360,7 @@ hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
   a.block_expert = q.block_expert;
   a.num_padded = q.num_padded;
   a.order = q.order;
+  a.heavy_first = q.R <= 32 * (int64_t)q.E;
   return launch_plan(a, q.scratch, st);
 }
 
@@ -480,11 +486,11 @@ SS_DEV void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Block index -> (M block, group of N tiles). The plan's M blocks are dealt round-robin to the XCDs (workgroup b runs on
-// XCD b % 8), in plan order, so every XCD gets an even share of the heavy and the light experts' blocks; each XCD takes
-// all N tiles of one M block in a row (they share its activation rows in the XCD's L2). Measured on MI355X, contiguous
-// per-XCD ranges of the plan end 140-180 us apart at 2048 tokens, and groups of 2, 4 or 8 M blocks per XCD (for the
-// weights they share) change nothing.
+// Block index -> (M block, group of N tiles). The M blocks are dealt round-robin to the XCDs (workgroup b runs on XCD
+// b % 8), in launch order (plan order for a caller's plan), so every XCD gets an even share of the heavy and the light
+// experts' blocks; each XCD takes all N tiles of one M block in a row (they share its activation rows in the XCD's L2).
+// Measured on MI355X with the former kernel, contiguous per-XCD ranges of the plan end 140-180 us apart at 2048 tokens,
+// and groups of 2, 4 or 8 M blocks per XCD (for the weights they share) change nothing.
 SS_DEV bool xcd_tile(int mb, int nt, int& pid_m, int& pid_n) {
   const int b = blockIdx.x, x = b & 7, s = b >> 3;
   const int sm = s / nt;
