@@ -47,11 +47,21 @@ __global__ __launch_bounds__(256) void mfma_loop_kernel(const uint32_t* __restri
   ss_f32x4 acc[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) acc[k] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-  for (int it = 0; it < iters; ++it) {
+  // 16 rounds per pass: the compiler moves the accumulators once per pass of the loop. With one round per pass that was 6.5
+  // moves to an MFMA, and the loop a measure of them: 1,310 TFLOP/s, the matrix units busy 52 %; now 2,380 and 94 %
+  // (512 workgroups, 20,000 rounds; random operands 1,870, the clock falls).
+  auto round = [&]() {
 #pragma unroll
     for (int k = 0; k < 8; ++k) acc[k] = ss_mfma(a, b, acc[k]);
+  };
+  int it = 0;
+#pragma unroll 1
+  for (; it + 16 <= iters; it += 16) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) round();
   }
+#pragma unroll 1
+  for (; it < iters; ++it) round();
   float s = 0.f;
 #pragma unroll
   for (int k = 0; k < 8; ++k) s += acc[k].x + acc[k].y + acc[k].z + acc[k].w;
