@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void dense_gemm_kernel(DenseGemmArgs g) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   gemm_barrier();
   // acc[i][j][r]: row 16 i + 4 q + r, column 16 j + n of the wave's fragment grid. The block's C tile goes through
-  // LDS (two stages, dead by now) so that it leaves in 16-byte row pieces.
+  // LDS (one stage, dead by now) so that it leaves in 16-byte row pieces.
   static_assert(BM * BN * 2 <= (BM + BN) * 128, "the C tile fits one stage");
   uint16_t* ct = reinterpret_cast<uint16_t*>(l0);
   const int cw = pairs ? BN / 2 : BN;  // columns of the output tile

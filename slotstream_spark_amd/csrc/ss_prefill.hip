@@ -4,8 +4,8 @@
 // Semantics follow kernels/moe_align.py:11-48, kernels/fused_moe_affine.py:39-172 (the reference's prefill path):
 //  * moe_align: a stable counting sort of the rows by local expert (rows outside [0, num_local) are skipped); each
 //    expert's rows padded to block_m with the sentinel R; every block of block_m positions belongs to one expert.
-//    Computed without atomics in any order-dependent place: ranks inside a 256-row chunk by comparison, chunk
-//    offsets by a sequential scan per expert.
+//    Computed without atomics in any order-dependent place: ranks inside a 1024-row chunk by ballots and per-wave
+//    counts, chunk offsets by a sequential scan per expert.
 //  * gate/up: h[r, n] = bf16(silu(g) * u), g = sum_k x[tok(r), k] * bf16(q*s + b)[n, k] with bf16 products and
 //    fp32 accumulation (the dequantized weight is rounded to bf16 as the reference's _wtile does; q*s is exact
 //    in fp32, so one rounding of q*s + b, fused or not, gives the same value).
@@ -385,19 +385,21 @@ hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
 //    pieces per instruction), double-buffered; only the live 16-row fragments are loaded. The two stages are separate
 //    LDS objects, so the compiler knows that a pending load into one does not touch reads of the other. 16-byte chunk
 //    c of row m sits at chunk position c ^ a_swz(m), the lane that loads a position reads the chunk that belongs
-//    there, and the 16 lanes one ds_read_b128 phase serves fall on distinct banks (1.6 M conflict cycles per gate/up
-//    launch at 8192 tokens; with c ^ (m & 15) 23 M).
+//    there, and the 16 lanes one ds_read_b128 phase serves fall on distinct banks (3.2 M conflict cycles per gate/up
+//    launch at 8192 tokens, 1.5 % of the CU cycles).
 //  * Packed weights: 16 bytes per lane per step straight into registers, one stage ahead.
 //  * Scales and biases: 8 groups (4 steps) of the wave's own rows at a time, direct to LDS, loaded once the last
 //    step of the previous 8 groups has read its values.
 // A stage holds KS steps: KS rises as the live rows fall (the loads of one stage are in flight while the previous one
 // is computed, and a light stage has little to compute), at the same LDS bytes.
-// What bounds it (MI355X, 8192 tokens x top-10, H 2048 / I 512, gate/up): 372 us, 924 TFLOP/s; without the loads 330,
-// without the dequantisation 315, without either 256, MFMA alone 161: the dequantisation (19 VALU per 8 nibbles) and
-// the MFMAs of the two waves of a SIMD overlap only in part (ordering one slice's dequantisation between the MFMAs of
-// the slice before, with or without wave priorities, changes nothing). The down product writes 671 MB of out_rows: 280
-// us, 195 without the stores. The former kernel (64-wide K steps, activations through registers, a barrier per 64 K,
-// four fragments always) took 424 and 325 us, and the pair 245 us at 2048 tokens and 45 at 19 (now 232 and 39).
+// What bounds it (MI355X, inside a layer, 512 experts top-10, counters over the SIMD cycles): at 8192 tokens (H 2048 / I 512)
+// gate/up takes 450 us, 764 TFLOP/s, the matrix units busy 40 % and other VALU (19 instructions per 8 nibbles, most of it)
+// 41 %, LDS 15 %; two waves a SIMD overlap the two only in part (ordering one slice's dequantisation between the MFMAs of
+// the slice before, with or without wave priorities, changes nothing). 2048 tokens 28 and 36 % with 1.45 waves a SIMD, 333
+// tokens (H 2560 / I 640) 14 and 37 %: the dequantisation of records that few rows share, and the launch's tail. The down
+// product at 8192 tokens writes 671 MB of out_rows: 296 us. The former kernel (64-wide K steps, activations through
+// registers, a barrier per 64 K, four fragments always): gate/up and down 473 + 347 us at 8192 tokens, 165 + 110 at 2048 (now
+// 145-159 + 93-99), 28 + 17 at 19 (now 22 + 14).
 constexpr int kBM = 128;
 constexpr int kStepK = 128;          // K per step: two quantisation groups
 constexpr int kRowB = kStepK * 2;    // bytes of one activation row per step
@@ -453,9 +455,9 @@ SS_DEV ss_u32x4 dequant8(const ss_nibbles& w, float s9, float bi) {
 
 // out_rows larger than the memory-side cache (256 MB) leave by non-temporal stores: the combine finds them in memory
 // either way, and they no longer push the packed weights and h out of the caches. Smaller ones stay plain, so that the
-// combine reads them from that cache. Measured (layer, us, plain / non-temporal, H 2048): 3300 tokens (270 MB) 474 / 468,
-// 4096 555 / 547, 5500 710 / 691, 8192 974 / 960; 2600 at H 2560 (266 MB) 574 / 572; below the line 2048 (168 MB)
-// 310 / 316, 333 at H 2560 189 / 191.
+// combine reads them from that cache. Measured (layer, us, plain / non-temporal, two runs of each in turn within 0.2 %,
+// H 2048): 3300 tokens (270 MB) 479 / 471, 4096 557 / 548, 5500 708 / 695, 8192 986 / 973; 2600 at H 2560 (266 MB) level,
+// 566 / 566; below the line, in an earlier measurement, 2048 (168 MB) 310 / 316.
 constexpr int64_t kStreamBytes = 256ll << 20;
 
 struct GemmArgs {
@@ -877,8 +879,9 @@ hipError_t launch_prefill_gemm(const PrefillArgs& p, hipStream_t st) {
 
 // ---------------------------------------------------------------- combine_rank_order (fused_moe_affine.py:164-172)
 // With LAYER also y = bf16(bf16(out) + bf16(bf16(sigmoid(sgl)) * sh)), the roundings of combine_shared_kernel, so the
-// sums are not read back (at 8192 tokens the two launches took 162 + 21 us). Bound by HBM: T K H 4 bytes in, read
-// once and non-temporally (layer, us, plain / non-temporal loads: 333 tokens at H 2560 189 / 187, 2048 315 / 313).
+// sums are not read back (at 8192 tokens the two launches took 160 + 22 us, this one 132). Bound by HBM: T K H 4 bytes
+// in, read once and non-temporally (layer, us, plain / non-temporal loads, two runs each: 333 tokens at H 2560 level, 2600
+// at H 2560 575 / 566, 2048 326 / 316, 3300 479 / 471, 8192 993 / 973).
 template <bool LAYER>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ rows,
                                                       const int32_t* __restrict__ row_local,

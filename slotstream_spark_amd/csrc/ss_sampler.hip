@@ -19,7 +19,7 @@
 //
 // Every launch covers R rows at once (blockIdx.y). Accept mode is the sampled verify round of _mtp_decode
 // (engine/generate.py:208-229) over D+1 rows: row i is reached only if rows 0..i-1 drew their drafts, so its
-// penalty set is seen + drafts[0..i) and all rows are drawn together; a last one-wave kernel walks the rows in
+// penalty set is seen + drafts[0..i) and all rows are drawn together; their last row, or a last kernel, walks them in
 // order (a non-finite row ends the round without a draw, :210-212; the round goes on while the token equals the
 // draft). The launch sequence depends only on the parameters, so it can be captured in a graph: three launches for
 // rows with a top-k of at most 512 (below), one launch per step otherwise.
@@ -175,8 +175,8 @@ SS_DEV float chunk_sum(const float (&v)[kSub], float& sub) {
   return ss_wave_sum(s);
 }
 
-// Stages a chunk array [n <= 1024] in LDS for the sequential scans below (one wave, every lane).
-// A chunk array into LDS, zero-padded to a multiple of 16 entries (16-byte aligned).
+// Stages a chunk array [n <= 1024] in LDS for the sequential scans below (one wave, every lane), zero-padded to a
+// multiple of 16 entries (16-byte aligned).
 SS_DEV const float* stage(const float* a, int n) {
   __shared__ __attribute__((aligned(16))) float buf[kPerLane * 64];
   const int lane = threadIdx.x & 63;
