@@ -20,9 +20,9 @@
 namespace ss {
 
 // ---------------------------------------------------------------- moe_align
-// Three launches (count, scan, place), or one workgroup for up to kAlignChunk rows and keys: the plan is a chain of
-// small dependent steps, so what it costs is launches and the latency inside each (19 tokens x top-10, 512 experts:
-// seven launches of 1.2-4.2 us each and their gaps before, table look-ups included, one of 10 us now).
+// Three launches (count, scan, place; four with many keys or chunks), or one workgroup for up to kAlignChunk rows and
+// keys: the plan is a chain of small dependent steps, so what it costs is launches and the latency inside each (190 rows,
+// 512 keys, block_m 128: seven launches 17.4 us, one 9.0; 1024 rows 17.8 and 13.4).
 constexpr int kAlignChunk = 1024;         // rows per workgroup of the counting kernel
 constexpr int kAlignWaves = kAlignChunk / 64;
 
@@ -211,9 +211,31 @@ __global__ __launch_bounds__(kAlignChunk) void align_count_kernel(PlanArgs a) {
     a.chunk[(int64_t)blockIdx.x * a.nl + e] = align_count_of(sm_cnt, nk, e);
 }
 
-// One workgroup: exclusive offsets of every key over the chunks (in place) and its total, then the padded starts, the
-// blocks' experts and the launch order. A thread's loads over the chunks are independent, 32 in flight at once.
-__global__ __launch_bounds__(1024) void align_scan_kernel(PlanArgs a) {
+// Exclusive offsets of key e over the chunks (in place); returns its total. The loads are independent, 32 in flight.
+SS_DEV int align_keyscan(const PlanArgs& a, int e) {
+  int run = 0;
+  for (int c0 = 0; c0 < a.nch; c0 += 32) {
+    int v[32];
+#pragma unroll
+    for (int c = 0; c < 32; ++c) v[c] = c0 + c < a.nch ? a.chunk[(int64_t)(c0 + c) * a.nl + e] : 0;
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+      if (c0 + c < a.nch) a.chunk[(int64_t)(c0 + c) * a.nl + e] = run;
+      run += v[c];
+    }
+  }
+  return run;
+}
+
+// The key offsets as a launch of their own, for more counts than one workgroup should pass over.
+__global__ __launch_bounds__(64) void align_keyscan_kernel(PlanArgs a) {
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  if (e < a.nl) a.tot[e] = align_keyscan(a, e);
+}
+
+// One workgroup: the keys' offsets over the chunks and totals (with `scan`; they are there otherwise), then the padded
+// starts, the blocks' experts and the launch order.
+__global__ __launch_bounds__(1024) void align_scan_kernel(PlanArgs a, int scan) {
   extern __shared__ int sm_scan[];  // [2][nl + 1]
   int* ps = sm_scan;
   int* hv = sm_scan + a.nl + 1;
@@ -223,19 +245,8 @@ __global__ __launch_bounds__(1024) void align_scan_kernel(PlanArgs a) {
   for (int q = 0; q < 4; ++q) {
     const int e = kpt * tid + q;
     if (q >= kpt || e >= nl) continue;
-    int run = 0;
-    for (int c0 = 0; c0 < a.nch; c0 += 32) {
-      int v[32];
-#pragma unroll
-      for (int c = 0; c < 32; ++c) v[c] = c0 + c < a.nch ? a.chunk[(int64_t)(c0 + c) * nl + e] : 0;
-#pragma unroll
-      for (int c = 0; c < 32; ++c) {
-        if (c0 + c < a.nch) a.chunk[(int64_t)(c0 + c) * nl + e] = run;
-        run += v[c];
-      }
-    }
-    loc[q] = run;
-    a.tot[e] = run;
+    loc[q] = scan ? align_keyscan(a, e) : a.tot[e];
+    if (scan) a.tot[e] = loc[q];
   }
   align_scan(a, loc, kpt, ps, hv);
   for (int e = tid; e <= nl; e += 1024) a.pad[e] = ps[e];
@@ -270,23 +281,23 @@ __global__ __launch_bounds__(kAlignChunk) void align_small_kernel(PlanArgs a) {
   int loc[4] = {0, 0, 0, 0};
   if (tid < nl) tot[tid] = loc[0] = align_count_of(cnt, nk, tid);
   align_scan(a, loc, 1, ps, hv);
-  const int total = ps[nl];
-  const int64_t fill = a.order ? total : a.P;
-  for (int64_t p = tid; p < fill; p += kAlignChunk) {
-    bool none = p >= total;
-    if (!none) {
-      int lo = 0, hi = nl;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ps[mid] <= p) lo = mid;
-        else hi = mid - 1;
-      }
-      none = p - ps[lo] >= tot[lo];
-    }
-    if (none) a.sorted_rows[p] = (int32_t)a.R;
+  // the sentinel behind every key's rows (a wave for its 64 keys, one key after the other), and past the last one
+  const int p0 = tid < nl ? ps[tid] + tot[tid] : 0, p1 = tid < nl ? ps[tid + 1] : 0, lane = tid & 63;
+  for (uint64_t todo = __ballot(p0 < p1); todo; todo &= todo - 1) {
+    const int src = (int)__builtin_ctzll(todo);
+    const int q1 = __builtin_amdgcn_readlane(p1, src);
+    for (int p = __builtin_amdgcn_readlane(p0, src) + lane; p < q1; p += 64) a.sorted_rows[p] = (int32_t)a.R;
   }
+  if (!a.order)
+    for (int64_t p = ps[nl] + tid; p < a.P; p += kAlignChunk) a.sorted_rows[p] = (int32_t)a.R;
   if (key < nl) a.sorted_rows[ps[key] + r] = tid;
 }
+
+// The keys' offsets are taken inside the scanning workgroup up to 1024 keys (one a thread) and this many counts, by a launch
+// of their own past that. Measured (us, whole plan, inside / own launch): 512 keys x 49 chunks 13.3 / 17.0, 1024 x 49 17.0 /
+// 18.4, 1024 x 81 20.7 / 19.4, 1024 x 196 32.9 / 25.2; 2000 x 2 16.5 / 16.5, 2000 x 20 23.2 / 17.4, 4096 x 1 21.6 / 18.7,
+// 4096 x 81 158 / 27 (seven launches before: 43).
+constexpr int64_t kScanCounts = 1 << 16;
 
 static hipError_t launch_plan(PlanArgs a, int32_t* scratch, hipStream_t st) {
   a.nch = (int)((a.R + kAlignChunk - 1) / kAlignChunk);
@@ -312,7 +323,9 @@ static hipError_t launch_plan(PlanArgs a, int32_t* scratch, hipStream_t st) {
     if (ids) hipLaunchKernelGGL(align_count_kernel<true>, dim3(a.nch), dim3(kAlignChunk), cnt, st, a);
     else hipLaunchKernelGGL(align_count_kernel<false>, dim3(a.nch), dim3(kAlignChunk), cnt, st, a);
   }
-  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(1024), (size_t)(2 * a.nl + 2) * 4, st, a);
+  const bool scan = a.nl <= 1024 && (int64_t)a.nch * a.nl <= kScanCounts;
+  if (!scan) hipLaunchKernelGGL(align_keyscan_kernel, dim3((a.nl + 63) / 64), dim3(64), 0, st, a);
+  hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(1024), (size_t)(2 * a.nl + 2) * 4, st, a, scan ? 1 : 0);
   if (ids) a.le = a.local;
   const int64_t n = a.P > a.R ? a.P : a.R;
   if (n > 0) hipLaunchKernelGGL(align_place_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a);

@@ -33,9 +33,11 @@ def test_moe_align_matches_oracle(R, nl, bm, seed):
     assert np.array_equal(b.cpu().numpy(), rb)
 
 
-@pytest.mark.parametrize("R,nl,bm", [(1024, 1024, 64), (1025, 1024, 64), (1024, 1025, 8), (5000, 4096, 16), (2049, 3, 128)])
+@pytest.mark.parametrize("R,nl,bm", [(1024, 1024, 64), (1025, 1024, 64), (1024, 1025, 8), (5000, 4096, 16), (2049, 3, 128),
+                                     (700, 1, 1), (1, 1024, 1024), (1000, 512, 128), (65536, 1024, 8), (66000, 1024, 8)])
 def test_moe_align_one_and_three_launches(R, nl, bm):
-    """Up to 1024 rows and experts the plan is one workgroup, past that three launches over 1024-row chunks."""
+    """Up to 1024 rows and experts the plan is one workgroup, past that three launches over 1024-row chunks; past 1024
+    experts or 65,536 counts the offsets over the chunks are a launch of their own."""
     print(f"[align] R={R} nl={nl} bm={bm}", flush=True)
     rng = np.random.default_rng(R + nl)
     le = np.minimum(rng.zipf(1.2, size=R) - 2, nl).astype(np.int32)  # -1 and nl: skipped
