@@ -58,7 +58,6 @@ struct PlanArgs {
   int32_t* block_expert;
   int32_t* num_padded;
   MBlock* order;      // null, or the M blocks in launch order
-  bool heavy_first;   // that order: see align_scan
 };
 
 // Key of row i: its local expert, nl for a row that is skipped, nl + 1 past R.
@@ -118,12 +117,12 @@ SS_DEV int64_t record_of(const PlanArgs& a, int e) {
 // One workgroup of 1024: the padded start of every key (ps, nl + 1 entries; hv: the heavy blocks before it), the
 // expert of every M block and, with `order`, the blocks in launch order. Thread t holds the totals of keys
 // kpt t .. kpt t + kpt - 1 in loc.
-// Launch order: with heavy_first the blocks with more than half their rows come first and the others behind them, so the
-// light blocks fill the chip's tail instead of leaving it to a few heavy ones; otherwise plan order, which mixes full
-// blocks with partial ones on a CU. Heavy first pays with few rows per expert, where the tail is most of a launch (layer,
-// us, heavy first / plan order, top-10 of 512: 200 tokens 101 / 107, 333 118 / 128, 333 at H 2560 175 / 193, 850 189 / 199,
-// 1400 254 / 272), is level from 1700 on (294 / 291, at H 2560 440 / 443; 2048 316 / 313, at H 2560 471 / 474) and loses
-// in long prompts (3300 471 / 461, 5500 695 / 678, 8192 973 / 931): up to 32 rows per expert.
+// Launch order: blocks with more than half their rows first, the others behind them, so the light blocks fill the
+// chip's tail instead of leaving it to a few heavy ones. Layer, us, heavy first / plan order: top-10 of 512, Zipf routing,
+// 200 tokens 101 / 107, 333 118 / 128, 1400 254 / 272, 2048 308 / 313, at H 2560 333 175 / 193, 3000 614 / 638; top-8 of 64
+// 1000 tokens 141 / 160, 2048 245 / 268, 4096 402 / 416. It costs some long prompts, where plan order mixes full and
+// partial blocks on a CU: 512 experts 4096 tokens 543 / 531, 8192 937 / 936 and 973 / 931 by the routing's seed, 256 experts
+// 8192 791 / 753; no size tells these from 8192 at H 2560 (1353 / 1358) or 128 experts uniform 6000 (554 / 573).
 SS_DEV void align_scan(const PlanArgs& a, const int (&loc)[4], int kpt, int* ps, int* hv) {
   __shared__ int wsum[2][16];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -188,7 +187,7 @@ SS_DEV void align_scan(const PlanArgs& a, const int (&loc)[4], int kpt, int* ps,
     a.block_expert[q] = lo;
     if (a.order) {
       const int b0 = ps[lo] / bm, j = (int)q - b0, h = hv[lo + 1] - hv[lo];
-      const int at = !a.heavy_first ? (int)q : j < h ? hv[lo] + j : nheavy + (b0 - hv[lo]) + (j - h);
+      const int at = j < h ? hv[lo] + j : nheavy + (b0 - hv[lo]) + (j - h);
       a.order[at] = MBlock{record_of(a, lo), lo, (int32_t)q};
     }
   }
@@ -373,7 +372,6 @@ hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
   a.block_expert = q.block_expert;
   a.num_padded = q.num_padded;
   a.order = q.order;
-  a.heavy_first = q.R <= 32 * (int64_t)q.E;
   return launch_plan(a, q.scratch, st);
 }
 
@@ -406,11 +404,11 @@ hipError_t launch_resident_plan(const ResidentPlan& q, hipStream_t st) {
 // A stage holds KS steps: KS rises as the live rows fall (the loads of one stage are in flight while the previous one
 // is computed, and a light stage has little to compute), at the same LDS bytes.
 // What bounds it (MI355X, inside a layer, 512 experts top-10, counters over the SIMD cycles): at 8192 tokens (H 2048 / I 512)
-// gate/up takes 450 us, 764 TFLOP/s, the matrix units busy 40 % and other VALU (19 instructions per 8 nibbles, most of it)
-// 41 %, LDS 15 %; two waves a SIMD overlap the two only in part (ordering one slice's dequantisation between the MFMAs of
-// the slice before, with or without wave priorities, changes nothing). 2048 tokens 28 and 36 % with 1.45 waves a SIMD, 333
-// tokens (H 2560 / I 640) 14 and 37 %: the dequantisation of records that few rows share, and the launch's tail. The down
-// product at 8192 tokens writes 671 MB of out_rows: 296 us. The former kernel (64-wide K steps, activations through
+// gate/up takes 442-450 us, 764-778 TFLOP/s, the matrix units busy 41 % and other VALU (19 instructions per 8 nibbles, most
+// of it) 42 %, LDS 15 %; two waves a SIMD overlap the two only in part (ordering one slice's dequantisation between the MFMAs of
+// the slice before, with or without wave priorities, changes nothing). 2048 tokens 29 and 37 % with 1.5 waves a SIMD, 333
+// tokens (H 2560 / I 640) 14 and 38 %: the dequantisation of records that few rows share, and the launch's tail. The down
+// product at 8192 tokens writes 671 MB of out_rows: 297 us. The former kernel (64-wide K steps, activations through
 // registers, a barrier per 64 K, four fragments always): gate/up and down 473 + 347 us at 8192 tokens, 165 + 110 at 2048 (now
 // 145-159 + 93-99), 28 + 17 at 19 (now 22 + 14).
 constexpr int kBM = 128;
