@@ -689,7 +689,7 @@ __global__ __launch_bounds__(64) void samp_draw_kernel(SampArgs a) {
 // non-negative sum, so a chunk total is the butterfly over its nonzero leaves and chunks without survivors drop out.
 // More than kCand candidates, a chunk's slots or kSurv survivors (ties at the threshold) take the whole sequence inside the
 // workgroup. Latency bound. Three rows over 248,320 tokens at the default parameters (top-k 40, top-p 0.95): 32 us per
-// round (6 + 7 + 21 in the kernels); eleven launches (four radix passes over the row, exp, a top-p search in one
+// round (5 + 7 + 21 in the kernels); eleven launches (four radix passes over the row, exp, a top-p search in one
 // workgroup, keep, totals, draw, accept walk) took 106.
 // k from 40 to 512 (one row of normal logits, us, the eleven launches / these three): V 1000 64-132 / 38-85, 5000 67-120 /
 // 29-51, 32,000 73-126 / 29-50, 60,000 73-139 / 29-55, 248,320 91-3094 / 28-81. Of that, against groups of 16 entries or
