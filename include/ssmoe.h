@@ -27,7 +27,9 @@ extern "C" {
 #define SSMOE_ERR_NONFINITE 8 /* non-finite logits reached a p/q decision */
 #define SSMOE_ERR_TIMEOUT 16  /* a persistent launch's bounded wait (2^22 polls) for another workgroup ran out: its
                                * workgroups were not all resident at once, e.g. because a graph replayed on another stream
-                               * held CUs. The launch still finishes; its outputs are not valid. */
+                               * held CUs. The launch still finishes; its outputs are not valid. Also raised when a call's
+                               * wait for the launches before it on another stream ran out (about 20 s): it then
+                               * goes ahead. */
 
 /* Text of the last error on this host thread ("" if none). */
 const char* ssmoe_last_error(void);
